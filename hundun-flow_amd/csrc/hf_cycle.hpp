@@ -476,56 +476,6 @@ __device__ __forceinline__ int wrapi(int v, int extent) {
   return v < 0 ? v + extent : (v >= extent ? v - extent : v);
 }
 
-// Prolongation (src/solver_mg.cpp:3893-3993): x_f += sum of ((wx*wy)*wz)*x_c
-// over the (az, ay, ax) corners; fine solids := 0.
-template <class Tc, class Tf>
-__device__ __forceinline__ void prolong_cell(const Lv<Tc>& Cl, const Lv<Tf>& F,
-                                             int mask, int per, int i, int j,
-                                             int k, int c) {
-  using C = typename Compute<Tf>::type;
-  // the fluid flag, x and the corners are loaded together (one memory
-  // round trip); solid cells store zero
-  const bool fluid = F.act[c] != 0;
-  int xl, xr, yl, yr, zl, zr, xw, yw, zw;
-  interp(i, mask & 1, Cl.nx, per & 1, &xl, &xr, &xw);
-  interp(j, (mask >> 1) & 1, Cl.ny, (per >> 1) & 1, &yl, &yr, &yw);
-  interp(k, (mask >> 2) & 1, Cl.nz, (per >> 2) & 1, &zl, &zr, &zw);
-  // all eight corner values are loaded before any is used (a corner that
-  // does not exist on an axis repeats the first one and is skipped below)
-  const int gx[2] = {wrapi(xl, Cl.nx), wrapi(xr, Cl.nx)};
-  const int gy[2] = {wrapi(yl, Cl.ny), wrapi(yr, Cl.ny)};
-  const int gz[2] = {wrapi(zl, Cl.nz), wrapi(zr, Cl.nz)};
-  C corner[2][2][2];
-#pragma unroll
-  for (int az = 0; az < 2; ++az)
-#pragma unroll
-    for (int ay = 0; ay < 2; ++ay)
-#pragma unroll
-      for (int ax = 0; ax < 2; ++ax)
-        corner[az][ay][ax] = C(ld(
-            Cl.x[cell_index(Cl.nx, Cl.ny, gx[ax], gy[ay], gz[az])]));
-  const C xf = C(ld(F.x[c]));
-  const int nz2 = zl == zr ? 1 : 2, ny2 = yl == yr ? 1 : 2,
-            nx2 = xl == xr ? 1 : 2;
-  // the reference order: az, ay, ax; value += ((wx*wy)*wz)*x_c
-  C value = C(0);
-#pragma unroll
-  for (int az = 0; az < 2; ++az) {
-    const C wz = az == 0 ? C(1) - C(zw) * C(0.25) : C(zw) * C(0.25);
-#pragma unroll
-    for (int ay = 0; ay < 2; ++ay) {
-      const C wy = ay == 0 ? C(1) - C(yw) * C(0.25) : C(yw) * C(0.25);
-#pragma unroll
-      for (int ax = 0; ax < 2; ++ax) {
-        const C wx = ax == 0 ? C(1) - C(xw) * C(0.25) : C(xw) * C(0.25);
-        if (az < nz2 && ay < ny2 && ax < nx2)
-          value += wx * wy * wz * corner[az][ay][ax];
-      }
-    }
-  }
-  F.x[c] = fluid ? st<Tf>(xf + value) : st<Tf>(0.0);
-}
-
 // Retained defect fused with the restriction that consumes it
 // (src/solver_mg.cpp:3633-3720).  The z-marching layout of k_stencil_z with
 // full tiles of even width and height and even z-chunks, on a level with
@@ -632,13 +582,13 @@ __global__ void k_defect_restrict(Tiles t, Lv<Tf> L, Bc bc, Lv<Tc> Cl,
   }
 }
 
-// z-marching prolongation: a block owns one 2-D tile of the fine level and
-// t.per consecutive fine planes.  Each thread walks its fine column; the x
-// and y interpolation is set up once, and the four corners of a coarse
-// plane are loaded once and reused while consecutive fine planes need that
-// plane (fine planes 2K+1 and 2K+2 both interpolate between coarse planes K
-// and K+1).  Terms are added in the order of prolong_cell (the tail's
-// per-cell form).
+// z-marching prolongation (src/solver_mg.cpp:3893-3993: x_f += sum of
+// ((wx*wy)*wz)*x_c over the (az, ay, ax) corners; fine solids := 0): a block
+// owns one 2-D tile of the fine level and t.per consecutive fine planes.
+// Each thread walks its fine column; the x and y interpolation is set up
+// once, and the four corners of a coarse plane are loaded once and reused
+// while consecutive fine planes need that plane (fine planes 2K+1 and 2K+2
+// both interpolate between coarse planes K and K+1).
 template <class Tc, class Tf>
 __global__ void k_prolong_z(Tiles t, Lv<Tc> Cl, Lv<Tf> F, int mask, int per) {
   using C = typename Compute<Tf>::type;
@@ -946,336 +896,6 @@ __global__ void k_mg_proj3(Tiles t, const double* rin, const uint8_t* act,
     partials[lb] = p0;
     partials[stride + lb] = p1;
     partials[2 * stride + lb] = p2;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Single-workgroup tail: every level below the tail threshold (FP64) runs as
-// one kernel that interprets the host-built cycle program, removing ~10
-// launches per coarse level.
-// ---------------------------------------------------------------------------
-enum TailKind : uint8_t { T_SMOOTH = 0, T_RESTRICT = 1, T_PROLONG = 2 };
-struct TailOp {
-  uint8_t kind;
-  uint8_t level;
-  uint8_t reverse;
-  uint8_t retain;
-  uint16_t sweeps;
-  uint16_t pad;
-};
-
-struct TailLevel {
-  Lv<double> L;      // coefficients in global memory; x/b/r live in LDS
-  int coarsen_mask;
-  int fused;
-  int cheb;          // Chebyshev-Jacobi smoothing (else red-black)
-  double volume;
-  int lds;           // offset (doubles) of this level's x, b, r in LDS
-};
-
-constexpr int kTailLdsBytes = 64 * 1024;
-
-// Chebyshev-Jacobi stage factors of the tail's Chebyshev levels, stage s:
-// direction d = pf[s] d + rf[s] (b - A x) / D (d = rf[0] (b - A x) / D at
-// s = 0).  The host fills them with the recurrence of the grid levels.
-constexpr int kTailChebStages = 16;
-struct TailCheb {
-  double rf[kTailChebStages];
-  double pf[kTailChebStages];
-};
-
-__device__ __forceinline__ void tail_ijk(const Lv<double>& L, int c, int& i,
-                                         int& j, int& k) {
-  const int plane = L.nx * L.ny;
-  k = c / plane;
-  const int r = c - k * plane;
-  j = r / L.nx;
-  i = r - j * L.nx;
-}
-
-// Level view with the work slots redirected into LDS.
-__device__ __forceinline__ Lv<double> tail_view(const TailLevel& T,
-                                                double* lds) {
-  Lv<double> L = T.L;
-  L.x = lds + T.lds;
-  L.b = L.x + L.cells;
-  L.r = L.b + L.cells;
-  return L;
-}
-
-__device__ __forceinline__ void tail_apply(const Lv<double>& L, const Bc& bc,
-                                           int defect) {
-  for (int c = threadIdx.x; c < L.cells; c += blockDim.x) {
-    int i, j, k;
-    tail_ijk(L, c, i, j, k);
-    const double v = stencil<double>(L, bc, L.x, i, j, k, c, L.x[c]);
-    L.r[c] = defect ? L.b[c] - v : v;
-  }
-  __syncthreads();
-}
-
-// Where a tail cell's six neighbours (x-lo, x-hi, y-lo, y-hi, z-lo, z-hi)
-// sit in its level's x: the neighbour cell, the cell itself on a Neumann
-// face, the wrapped cell on a periodic face, -1 on a Dirichlet face (read
-// as +0).  The values are those neighbour_or_boundary gives; set up once
-// per smoothing call, they spare every pass the boundary-mode branches.
-struct TailNb {
-  int n[6];
-};
-
-__device__ __forceinline__ TailNb tail_neighbours(const Lv<double>& L,
-                                                  const Bc& bc, int i, int j,
-                                                  int k, int c) {
-  const int nx = L.nx, ny = L.ny, nz = L.nz, plane = nx * ny;
-  auto face = [&](bool inside, int next, int mode, int wrapped) {
-    if (inside) return next;
-    return mode == 0 ? -1 : (mode == 1 ? c : wrapped);
-  };
-  TailNb nb;
-  nb.n[0] = face(i > 0, c - 1, bc.m[0], c + (nx - 1));
-  nb.n[1] = face(i + 1 < nx, c + 1, bc.m[1], c - (nx - 1));
-  nb.n[2] = face(j > 0, c - nx, bc.m[2], c + (ny - 1) * nx);
-  nb.n[3] = face(j + 1 < ny, c + nx, bc.m[3], c - (ny - 1) * nx);
-  nb.n[4] = face(k > 0, c - plane, bc.m[4], c + (nz - 1) * plane);
-  nb.n[5] = face(k + 1 < nz, c + plane, bc.m[5], c - (nz - 1) * plane);
-  return nb;
-}
-
-// stencil_with on a tail cell through its neighbour positions: the same
-// operands in the same order.
-__device__ __forceinline__ double tail_stencil(const Lv<double>& L,
-                                               const TailNb& nb, int c,
-                                               double xc,
-                                               const StencilCoef<double>& f) {
-  double v6[6];
-#pragma unroll
-  for (int q = 0; q < 6; ++q) {
-    const int at = nb.n[q];
-    const double v = L.x[at < 0 ? c : at];
-    v6[q] = at < 0 ? 0.0 : v;
-  }
-  double v = f.d * xc;
-  v -= f.xl * v6[0];
-  v -= f.xh * v6[1];
-  v -= f.yl * v6[2];
-  v -= f.yh * v6[3];
-  v -= f.zl * v6[4];
-  v -= f.zh * v6[5];
-  return v;
-}
-
-// tail_smooth on a level of at most one cell per thread: the cell's
-// coefficients are loaded once and kept in registers across the passes (the
-// same values and arithmetic as the general form below).
-__device__ void tail_smooth_small(const Lv<double>& L, int fused, const Bc& bc,
-                                  int sweeps, int reverse, int retain) {
-  const double omega = 0.72;
-  const int c = threadIdx.x;
-  const bool mine = c < L.cells;
-  int i = 0, j = 0, k = 0;
-  StencilCoef<double> f{};
-  TailNb nb{};
-  if (mine) {
-    tail_ijk(L, c, i, j, k);
-    f = stencil_coef<double>(L, j, k, c);
-    nb = tail_neighbours(L, bc, i, j, k, c);
-  }
-  auto apply = [&](int defect) {
-    if (mine) {
-      const double v = tail_stencil(L, nb, c, L.x[c], f);
-      L.r[c] = defect ? L.b[c] - v : v;
-    }
-    __syncthreads();
-  };
-  if (!fused) apply(0);
-  for (int sweep = 0; sweep < sweeps; ++sweep) {
-    const int first = reverse ? 1 : 0;
-    for (int pass = 0; pass < 2; ++pass) {
-      const int color = (first + pass) & 1;
-      if (mine && ((i + j + k) & 1) == color) {
-        const double xc = L.x[c];
-        const double v =
-            fused ? tail_stencil(L, nb, c, xc, f) : L.r[c];
-        L.x[c] = xc + omega * (L.b[c] - v) / f.d;
-      }
-      __syncthreads();
-      const bool final_update = sweep + 1 == sweeps && pass == 1;
-      if (!final_update || retain) {
-        if (!fused || (final_update && retain)) apply(retain && final_update);
-      }
-    }
-  }
-}
-
-__device__ void tail_smooth(const Lv<double>& L, int fused, const Bc& bc,
-                            int sweeps, int reverse, int retain) {
-  if (L.cells <= static_cast<int>(blockDim.x)) {
-    tail_smooth_small(L, fused, bc, sweeps, reverse, retain);
-    return;
-  }
-  const double omega = 0.72;
-  if (!fused) tail_apply(L, bc, 0);
-  for (int sweep = 0; sweep < sweeps; ++sweep) {
-    const int first = reverse ? 1 : 0;
-    for (int pass = 0; pass < 2; ++pass) {
-      const int color = (first + pass) & 1;
-      for (int c = threadIdx.x; c < L.cells; c += blockDim.x) {
-        int i, j, k;
-        tail_ijk(L, c, i, j, k);
-        if (((i + j + k) & 1) != color) continue;
-        const double xc = L.x[c];
-        const double v =
-            fused ? stencil<double>(L, bc, L.x, i, j, k, c, xc) : L.r[c];
-        L.x[c] = xc + omega * (L.b[c] - v) / L.D[c];
-      }
-      __syncthreads();
-      const bool final_update = sweep + 1 == sweeps && pass == 1;
-      if (!final_update || retain) {
-        if (!fused || (final_update && retain))
-          tail_apply(L, bc, retain && final_update);
-      }
-    }
-  }
-}
-
-// Chebyshev-Jacobi smoothing of a tail level (src/solver_mg.cpp:2916-3090):
-// the stages of k_cheb_stage with x updated in place.  A stage stores its
-// direction in r, and x += r follows a barrier, so every neighbour the
-// stencil reads is the stage's input x (Jacobi), the operands and order of
-// operations being those of the grid kernel.  retain: then r = b - A x.
-__device__ void tail_cheb(const Lv<double>& L, const Bc& bc, int stages,
-                          int retain, const TailCheb& ch) {
-  if (L.cells <= static_cast<int>(blockDim.x)) {
-    // at most one cell per thread: its coefficients stay in registers
-    const int c = threadIdx.x;
-    const bool mine = c < L.cells;
-    int i = 0, j = 0, k = 0;
-    StencilCoef<double> f{};
-    TailNb nb{};
-    if (mine) {
-      tail_ijk(L, c, i, j, k);
-      f = stencil_coef<double>(L, j, k, c);
-      nb = tail_neighbours(L, bc, i, j, k, c);
-    }
-    for (int s = 0; s < stages; ++s) {
-      double xn = 0.0;
-      if (mine) {
-        const double xc = L.x[c];
-        const double v = tail_stencil(L, nb, c, xc, f);
-        const double defect = L.b[c] - v;
-        const double scaled = ch.rf[s] * defect / f.d;
-        const double dir = s == 0 ? scaled : ch.pf[s] * L.r[c] + scaled;
-        L.r[c] = dir;
-        xn = xc + dir;
-      }
-      __syncthreads();
-      if (mine) L.x[c] = xn;
-      __syncthreads();
-    }
-    if (retain) {
-      if (mine)
-        L.r[c] = L.b[c] - tail_stencil(L, nb, c, L.x[c], f);
-      __syncthreads();
-    }
-    return;
-  }
-  for (int s = 0; s < stages; ++s) {
-    for (int c = threadIdx.x; c < L.cells; c += blockDim.x) {
-      int i, j, k;
-      tail_ijk(L, c, i, j, k);
-      const double xc = L.x[c];
-      const double v = stencil<double>(L, bc, L.x, i, j, k, c, xc);
-      const double defect = L.b[c] - v;
-      const double scaled = ch.rf[s] * defect / L.D[c];
-      L.r[c] = s == 0 ? scaled : ch.pf[s] * L.r[c] + scaled;
-    }
-    __syncthreads();
-    for (int c = threadIdx.x; c < L.cells; c += blockDim.x)
-      L.x[c] = L.x[c] + L.r[c];
-    __syncthreads();
-  }
-  if (retain) tail_apply(L, bc, 1);
-}
-
-__device__ void tail_project(const Lv<double>& L, double volume, double* field,
-                             double* scratch, double* mean) {
-  double v = 0.0;
-  for (int c = threadIdx.x; c < L.cells; c += blockDim.x)
-    v += L.vol[c] * field[c];
-  v = block_sum(v, scratch);
-  if (threadIdx.x == 0) *mean = v / volume;
-  __syncthreads();
-  const double m = *mean;
-  for (int c = threadIdx.x; c < L.cells; c += blockDim.x)
-    field[c] = L.vol[c] > 0.0 ? field[c] - m : 0.0;
-  __syncthreads();
-}
-
-// The tail's first level receives b (already projected) and x = 0 from the
-// grid-level restriction; its x is stored back for the grid prolongation.
-__global__ void __launch_bounds__(1024)
-k_tail(const TailLevel* levels, int first_level, const TailOp* ops, int nops,
-       Bc bc, int periodic_mask, int null_space, TailCheb cheb) {
-  extern __shared__ double lds[];
-  __shared__ double scratch[16];
-  __shared__ double mean;
-  {
-    const TailLevel& T0 = levels[0];
-    const Lv<double> L0 = tail_view(T0, lds);
-    for (int c = threadIdx.x; c < L0.cells; c += blockDim.x) {
-      L0.x[c] = T0.L.x[c];
-      L0.b[c] = T0.L.b[c];
-    }
-    __syncthreads();
-  }
-  for (int o = 0; o < nops; ++o) {
-    const TailOp op = ops[o];
-    const TailLevel& T = levels[op.level - first_level];
-    const Lv<double> L = tail_view(T, lds);
-    if (op.kind == T_SMOOTH) {
-      if (T.cheb)
-        tail_cheb(L, bc, op.sweeps, op.retain, cheb);
-      else
-        tail_smooth(L, T.fused, bc, op.sweeps, op.reverse, op.retain);
-    } else if (op.kind == T_RESTRICT) {
-      const TailLevel& Cn = levels[op.level + 1 - first_level];
-      const Lv<double> Cl = tail_view(Cn, lds);
-      const int mask = T.coarsen_mask;
-      const int mx = mask & 1, my = (mask >> 1) & 1, mz = (mask >> 2) & 1;
-      for (int t = threadIdx.x; t < Cl.cells; t += blockDim.x) {
-        int ci, cj, ck;
-        tail_ijk(Cl, t, ci, cj, ck);
-        const int xb = mx ? 2 * ci : ci, yb = my ? 2 * cj : cj,
-                  zb = mz ? 2 * ck : ck;
-        double sum = 0.0;
-        for (int dz = 0; dz < (mz ? 2 : 1); ++dz)
-          for (int dy = 0; dy < (my ? 2 : 1); ++dy)
-            for (int dx = 0; dx < (mx ? 2 : 1); ++dx) {
-              const int fx = xb + dx, fy = yb + dy, fz = zb + dz;
-              if (fx >= L.nx || fy >= L.ny || fz >= L.nz) continue;
-              sum += L.r[cell_index(L.nx, L.ny, fx, fy, fz)];
-            }
-        Cl.b[t] = sum;
-        Cl.x[t] = 0.0;
-      }
-      __syncthreads();
-      if (null_space) tail_project(Cl, Cn.volume, Cl.b, scratch, &mean);
-    } else {
-      const TailLevel& Cn = levels[op.level + 1 - first_level];
-      const Lv<double> Cl = tail_view(Cn, lds);
-      for (int c = threadIdx.x; c < L.cells; c += blockDim.x) {
-        int i, j, k;
-        tail_ijk(L, c, i, j, k);
-        prolong_cell(Cl, L, T.coarsen_mask, periodic_mask, i, j, k, c);
-      }
-      __syncthreads();
-    }
-  }
-  {
-    const TailLevel& T0 = levels[0];
-    const Lv<double> L0 = tail_view(T0, lds);
-    for (int c = threadIdx.x; c < L0.cells; c += blockDim.x)
-      T0.L.x[c] = L0.x[c];
   }
 }
 

@@ -19,6 +19,7 @@
 #include "hf_kernels.hpp"
 #include "hf_krylov.hpp"
 #include "hf_line.hpp"
+#include "hf_tail.hpp"
 #include "hundun_flow.h"
 
 namespace hf {
@@ -179,6 +180,7 @@ struct ExecItem {
   CycleOp op{};
   int tail_begin = 0;  // index into tail_ops
   int tail_count = 0;
+  int tail_from_zero = 0;  // x of the tail's first level starts from zero
   // a retaining smoothing whose defect and the following restriction run
   // as one kernel (k_defect_restrict); that restriction item is skipped
   bool defect_restrict = false;
@@ -272,9 +274,15 @@ struct hf_plan {
   std::vector<CycleOp> program;
   std::vector<ExecItem> exec;
   std::vector<TailOp> tail_ops_host;
-  TailOp* d_tail_ops = nullptr;
+  const TailOp* d_tail_ops = nullptr;
   TailCheb tail_cheb{};  // stage factors of the tail's Chebyshev levels
-  TailLevel* d_tail_levels = nullptr;
+  // tail geometry, coefficients and tables (hf_tail.hpp)
+  std::vector<TailGeo> tail_geo;
+  std::vector<double> tail_blob;  // upload image, until the plan is created
+  double* d_tail_blob = nullptr;  // ends with the ops (d_tail_ops)
+  int tail_work = 0;      // LDS doubles of x, b, r
+  int tail_head = 0;      // blob doubles copied to LDS
+  int tail_resident = 0;  // first tail level whose image is copied
   size_t tail_lds_bytes = 0;
   bool coefficients_ready = false;
   bool has_activity = false;
@@ -635,11 +643,12 @@ void build_exec(hf_plan* p) {
     ExecItem e;
     e.tail = true;
     e.tail_begin = static_cast<int>(p->tail_ops_host.size());
+    e.tail_from_zero = p->program[i].from_zero;
     while (i < p->program.size() && op_on_tail(p, p->program[i])) {
       const CycleOp& op = p->program[i];
       TailOp t{};
       t.kind = static_cast<uint8_t>(op.kind);
-      t.level = static_cast<uint8_t>(op.level);
+      t.level = static_cast<uint8_t>(op.level - p->tail_first);
       t.reverse = static_cast<uint8_t>(op.reverse);
       t.retain = static_cast<uint8_t>(op.retain);
       t.sweeps = static_cast<uint16_t>(op.sweeps);
@@ -1018,6 +1027,21 @@ void point_smooth(hf_plan* p, int l, int sweeps, int reverse, int retain,
   }
 }
 
+// A level that needs the projected b and x = 0 in memory before a cycle
+// visits it (a point-smoothed grid level starts from zero and applies the
+// projection in its first pass, the tail when it loads b).
+bool wants_stored_start(const Level& L) {
+  return !L.tail && (L.line_mask != 0 || L.cheb);
+}
+
+// Whether level 0's b is projected in memory before the cycle: also where
+// the residual-minimising scaling reads it after a cycle that projects b as
+// it loads it.
+bool entry_projects(const hf_plan* p) {
+  const Level& L0 = p->levels[0];
+  return wants_stored_start(L0) || (L0.tail && !p->policy.unit_linear);
+}
+
 void exec_grid_op(hf_plan* p, const CycleOp& op,
                   double* mean_partials = nullptr,
                   bool defect_restrict = false) {
@@ -1045,7 +1069,7 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
     // the retained defect and the restriction of the next op, in one pass
     Level& Cd = p->levels[op.level + 1];
     const bool proj = p->policy.null_space_constant != 0;
-    const bool into_tail = Cd.tail || Cd.line_mask != 0 || Cd.cheb;
+    const bool stored = wants_stored_start(Cd);
     dispatch(L.prec, [&](auto tf) {
       using Tf = decltype(tf);
       dispatch(Cd.prec, [&](auto tc) {
@@ -1057,7 +1081,7 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
           HF_PROF(p, P_DEFECT);
           HF_LAUNCH((k_defect_restrict<Tf, Tc, true>), L.tz.blocks, kBlock, 0,
                     p->stream, L.tz, view<Tf>(L), p->bc, view<Tc>(Cd),
-                    into_tail ? 1 : 0,
+                    stored ? 1 : 0,
                     proj ? p->partials : static_cast<double*>(nullptr),
                     static_cast<C>(rf0), static_cast<Tf*>(L.x2));
           std::swap(L.x, L.x2);
@@ -1065,13 +1089,13 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
           HF_PROF(p, P_DEFECT);
           HF_LAUNCH((k_defect_restrict<Tf, Tc>), L.tz.blocks, kBlock, 0,
                     p->stream, L.tz, view<Tf>(L), p->bc, view<Tc>(Cd),
-                    into_tail ? 1 : 0,
+                    stored ? 1 : 0,
                     proj ? p->partials : static_cast<double*>(nullptr));
         }
         if (proj) {
           finalize(p, L.tz.blocks, 1, F_MEAN, S_MEAN0 + op.level + 1,
                    Cd.volume);
-          if (into_tail)
+          if (stored)
             project_apply<Tc>(p, op.level + 1, static_cast<Tc*>(Cd.b));
         }
       });
@@ -1081,10 +1105,7 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
   Level& Cn = p->levels[op.level + 1];
   if (op.kind == T_RESTRICT) {
     const bool proj = p->policy.null_space_constant != 0;
-    // a point-smoothed grid level starts from zero and applies the
-    // projection in its first pass; the tail and line levels need x = 0 and
-    // a projected b up front
-    const bool into_tail = Cn.tail || Cn.line_mask != 0 || Cn.cheb;
+    const bool stored = wants_stored_start(Cn);
     dispatch(L.prec, [&](auto tf) {
       using Tf = decltype(tf);
       dispatch(Cn.prec, [&](auto tc) {
@@ -1093,13 +1114,13 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
           HF_PROF(p, P_RESTRICT);
           HF_LAUNCH((k_restrict<Tf, Tc>), Cn.tr.blocks, kBlock, 0, p->stream,
                     Cn.tr, view<Tf>(L), view<Tc>(Cn), L.coarsen_mask,
-                    into_tail ? 1 : 0,
+                    stored ? 1 : 0,
                     proj ? p->partials : static_cast<double*>(nullptr));
         }
         if (proj) {
           finalize(p, Cn.tr.blocks, 1, F_MEAN, S_MEAN0 + op.level + 1,
                    Cn.volume);
-          if (into_tail) project_apply<Tc>(p, op.level + 1, static_cast<Tc*>(Cn.b));
+          if (stored) project_apply<Tc>(p, op.level + 1, static_cast<Tc*>(Cn.b));
         }
       });
     });
@@ -1144,11 +1165,27 @@ void run_cycle(hf_plan* p, double* mean_partials = nullptr) {
       continue;
     }
     HF_PROF(p, P_TAIL);
-    HF_LAUNCH(k_tail, 1, 1024, p->tail_lds_bytes, p->stream, p->d_tail_levels,
-              p->tail_first,
-              p->d_tail_ops + e.tail_begin, e.tail_count, p->bc,
-              p->periodic_mask, static_cast<int>(p->policy.null_space_constant),
-              p->tail_cheb);
+    const Level& T = p->levels[p->tail_first];
+    TailRun t{};
+    t.blob = p->d_tail_blob;
+    t.x0 = static_cast<double*>(T.x);
+    t.b0 = static_cast<const double*>(T.b);
+    t.act0 = T.act;
+    t.cells0 = static_cast<int>(T.cells);
+    t.mean = p->policy.null_space_constant != 0 &&
+                     !(p->tail_first == 0 && entry_projects(p))
+                 ? p->scalars + S_MEAN0 + p->tail_first
+                 : nullptr;
+    t.levels = static_cast<int>(p->tail_geo.size());
+    t.work = p->tail_work;
+    t.head = p->tail_head;
+    t.resident = p->tail_resident;
+    t.ops = p->d_tail_ops + e.tail_begin;
+    t.nops = e.tail_count;
+    t.zero_x = e.tail_from_zero;
+    t.null_space = p->policy.null_space_constant;
+    t.cheb = p->tail_cheb;
+    HF_LAUNCH(k_tail, 1, kTailThreads, p->tail_lds_bytes, p->stream, t);
   }
 }
 
@@ -1171,13 +1208,11 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
                    ExitOperands* exit = nullptr, int64_t entry_blocks = 0) {
   Level& L0 = p->levels[0];
   const bool proj = p->policy.null_space_constant != 0;
-  // whole cycle inside the tail kernel, or a line level 0: x = 0 and the
-  // projected b are stored before the cycle
-  const bool tail0 = L0.tail || L0.line_mask != 0 || L0.cheb;
+  const bool tail0 = entry_projects(p);
   // (a grid Chebyshev level 0 starts with a from-zero stage, which reads
-  // b and D only: its x needs no zero)
-  const bool zero_x =
-      L0.tail || L0.line_mask != 0 || (L0.cheb && !p->cheb_first);
+  // b and D only, and the tail starts from zero by itself: no x = 0 there)
+  const bool zero_x = !L0.tail && (L0.line_mask != 0 ||
+                                   (L0.cheb && !p->cheb_first));
   dispatch(L0.prec, [&](auto t) {
     using T = decltype(t);
     T* b = static_cast<T*>(L0.b);
@@ -1259,32 +1294,140 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
   return ok();
 }
 
-hf_status upload_tail(hf_plan* p) {
-  const int L = static_cast<int>(p->levels.size());
-  const int count = L - p->tail_first;
+// Tail layout (hf_tail.hpp) of a plan whose levels and program stand: LDS
+// offsets, the blob with its geometry and tables, and the ops.  The
+// coefficients follow at each refresh (pack_tail).
+hf_status build_tail(hf_plan* p) {
+  const int count = static_cast<int>(p->levels.size()) - p->tail_first;
   if (count <= 0) return ok();
-  std::vector<TailLevel> host(count);
-  int64_t lds = 0;
-  for (int l = p->tail_first; l < L; ++l) {
-    TailLevel& t = host[l - p->tail_first];
-    t.L = view<double>(p->levels[l]);
-    t.coarsen_mask = p->levels[l].coarsen_mask;
-    t.fused = p->levels[l].fused;
-    t.cheb = p->levels[l].cheb ? 1 : 0;
-    t.volume = p->levels[l].volume;
-    t.lds = static_cast<int>(lds);
-    lds += 3 * p->levels[l].cells;
+  if (count > kTailMaxLevels) return fail(HF_INVALID_PLAN, kDetailPlan);
+  p->tail_geo.assign(count, TailGeo{});
+  int64_t work = kTailSlots;
+  for (int t = 0; t < count; ++t) {
+    const Level& L = p->levels[p->tail_first + t];
+    TailGeo& g = p->tail_geo[t];
+    g.nx = L.n[0];
+    g.ny = L.n[1];
+    g.nz = L.n[2];
+    g.cells = static_cast<int>(L.cells);
+    g.colour0 = (g.cells + 1) / 2;
+    g.coarsen_mask = L.coarsen_mask;
+    g.fused = L.fused;
+    g.cheb = L.cheb ? 1 : 0;
+    g.work = static_cast<int>(work);
+    work += 3 * L.cells;
   }
-  if (hipMemcpyAsync(p->d_tail_levels, host.data(),
-                     count * sizeof(TailLevel), hipMemcpyHostToDevice,
-                     p->stream) != hipSuccess)
-    return fail(HF_INVALID_PLAN, kDetailHip);
-  if (!p->tail_ops_host.empty() &&
-      hipMemcpyAsync(p->d_tail_ops, p->tail_ops_host.data(),
-                     p->tail_ops_host.size() * sizeof(TailOp),
-                     hipMemcpyHostToDevice, p->stream) != hipSuccess)
-    return fail(HF_INVALID_PLAN, kDetailHip);
-  return hip_check(hipStreamSynchronize(p->stream));
+  work += work & 1;  // 16-byte copies of the blob
+  p->tail_work = static_cast<int>(work);
+  // images, coarsest first; as many as fit are copied to LDS at each launch
+  size_t most_ops = 0;
+  for (const ExecItem& e : p->exec)
+    if (e.tail) most_ops = std::max<size_t>(most_ops, e.tail_count);
+  if (most_ops > kTailMaxOps) return fail(HF_INVALID_PLAN, kDetailPlan);
+  const int64_t room = kTailLdsBytes / static_cast<int64_t>(sizeof(double)) -
+                       work - static_cast<int64_t>(most_ops);
+  int64_t at = static_cast<int64_t>(count) * kTailGeoDoubles;
+  p->tail_head = static_cast<int>(at);
+  p->tail_resident = count;
+  for (int t = count - 1; t >= 0; --t) {
+    p->tail_geo[t].image = static_cast<int>(at);
+    at += tail_image_doubles(p->tail_geo[t].cells);
+    if (at <= room && p->tail_resident == t + 1) {
+      p->tail_resident = t;
+      p->tail_head = static_cast<int>(at);
+    }
+  }
+  p->tail_lds_bytes =
+      static_cast<size_t>(work + p->tail_head + most_ops) * sizeof(double);
+  std::vector<double>& blob = p->tail_blob;
+  blob.assign(static_cast<size_t>(at) + p->tail_ops_host.size(), 0.0);
+  std::memcpy(blob.data(), p->tail_geo.data(), count * sizeof(TailGeo));
+  for (int t = 0; t < count; ++t) {
+    const TailGeo& g = p->tail_geo[t];
+    uint16_t* table =
+        reinterpret_cast<uint16_t*>(blob.data() + g.image + kTailCoefs * g.cells);
+    int next[2] = {0, g.colour0};
+    const int n[3] = {g.nx, g.ny, g.nz};
+    const int step[3] = {1, g.nx, g.nx * g.ny};
+    for (int c = 0; c < g.cells; ++c) {
+      const int ijk[3] = {c % g.nx, (c / g.nx) % g.ny, c / (g.nx * g.ny)};
+      const int s = next[(ijk[0] + ijk[1] + ijk[2]) & 1]++;
+      table[kTailCell * g.cells + s] = static_cast<uint16_t>(c);
+      for (int a = 0; a < 3; ++a) {
+        table[(kTailIjk + a) * g.cells + s] = static_cast<uint16_t>(ijk[a]);
+        if (t + 1 < count) {
+          // the coarse planes between which the cell lies, wrapped or, past
+          // a wall, the one plane (the coarse level has g's axes coarsened)
+          const TailGeo& cg = p->tail_geo[t + 1];
+          const int cn[3] = {cg.nx, cg.ny, cg.nz};
+          const int cstep[3] = {1, cg.nx, cg.nx * cg.ny};
+          int low = ijk[a], high = -1;
+          if ((g.coarsen_mask >> a) & 1) {
+            low = ijk[a] / 2 - (ijk[a] % 2 == 0 ? 1 : 0);
+            high = low + 1;
+            if ((p->periodic_mask >> a) & 1) {
+              low = (low + cn[a]) % cn[a];
+              high %= cn[a];
+            } else if (low < 0) {
+              low = 0;
+              high = -1;
+            } else if (high >= cn[a]) {
+              high = -1;
+            }
+          }
+          table[(kTailLow + a) * g.cells + s] =
+              static_cast<uint16_t>(low * cstep[a]);
+          table[(kTailHigh + a) * g.cells + s] =
+              high < 0 ? kTailNone : static_cast<uint16_t>(high * cstep[a]);
+        }
+        for (int side = 0; side < 2; ++side) {
+          // the neighbour, the cell itself on a Neumann face, the wrapped
+          // cell on a periodic one, none on a Dirichlet one
+          const bool inside = side == 0 ? ijk[a] > 0 : ijk[a] + 1 < n[a];
+          const int mode = p->bc.m[2 * a + side];
+          const int to = side == 0 ? -1 : 1;
+          int nb;
+          if (inside)
+            nb = c + to * step[a];
+          else if (mode == 0)
+            nb = kTailNone;
+          else
+            nb = mode == 1 ? c : c - to * (n[a] - 1) * step[a];
+          table[(kTailNb + 2 * a + side) * g.cells + s] =
+              static_cast<uint16_t>(nb);
+        }
+      }
+    }
+  }
+  std::memcpy(blob.data() + at, p->tail_ops_host.data(),
+              p->tail_ops_host.size() * sizeof(TailOp));
+  HF_TRY(dalloc(p, &p->d_tail_blob, blob.size()));
+  p->d_tail_ops = reinterpret_cast<const TailOp*>(p->d_tail_blob + at);
+  HF_TRY(hip_check(hipMemcpyAsync(p->d_tail_blob, blob.data(),
+                                  blob.size() * sizeof(double),
+                                  hipMemcpyHostToDevice, p->stream)));
+  if (p->tail_lds_bytes <= 64 * 1024) return ok();
+  return hip_check(hipFuncSetAttribute(
+      reinterpret_cast<const void*>(&k_tail),
+      hipFuncAttributeMaxDynamicSharedMemorySize,
+      static_cast<int>(kTailLdsBytes)));
+}
+
+// The published hierarchy's tail coefficients into the blob.
+void pack_tail(hf_plan* p) {
+  if (p->tail_geo.empty()) return;
+  TailPack a{};
+  int most = 0;
+  for (size_t t = 0; t < p->tail_geo.size(); ++t) {
+    const Level& L = p->levels[p->tail_first + t];
+    a.L[t] = op_view(L);
+    a.volume[t] = L.volume;
+    most = std::max(most, p->tail_geo[t].cells);
+  }
+  hipLaunchKernelGGL(k_tail_pack,
+                     dim3(static_cast<uint32_t>(blocks_for(most)),
+                          static_cast<uint32_t>(p->tail_geo.size())),
+                     dim3(kBlock), 0, p->stream, a, p->d_tail_blob);
 }
 
 AxisGeom axis_geom(const hf_plan* p) {
@@ -1958,7 +2101,7 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
     return fail(HF_INVALID_PLAN, kDetailLineOff);
   }
   // the tail is the longest run of coarsest levels whose x, b, r fit the
-  // tail kernel's LDS and each stay under the cell threshold
+  // tail kernel's share of LDS and each stay under the cell threshold
   const int64_t threshold = tail_threshold();
   p->row_pairs = row_pairs_enabled();
   p->cheb_first = cheb_first_enabled();
@@ -1974,8 +2117,8 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
   for (int l = static_cast<int>(p->levels.size()) - 1;
        l >= 0 && !line_plan && (!cheb_plan || cheb_fits); --l) {
     const int64_t need = lds_doubles + 3 * p->levels[l].cells;
-    if (p->levels[l].cells <= threshold &&
-        need * static_cast<int64_t>(sizeof(double)) <= kTailLdsBytes) {
+    if (p->levels[l].cells <= std::min<int64_t>(threshold, kTailMaxCells) &&
+        need * static_cast<int64_t>(sizeof(double)) <= kTailWorkBytes) {
       p->tail_first = l;
       lds_doubles = need;
     } else {
@@ -1991,11 +2134,9 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
   // tail kernel
   if (!line_plan && p->tail_first > static_cast<int>(p->levels.size()) - 1)
     p->tail_first = static_cast<int>(p->levels.size()) - 1;
-  int64_t tail_doubles = 0;
   for (size_t l = 0; l < p->levels.size(); ++l) {
     Level& L = p->levels[l];
     L.tail = static_cast<int>(l) >= p->tail_first;
-    if (L.tail) tail_doubles += 3 * L.cells;
     const bool coarsest = l + 1 == p->levels.size();
     L.prec = (L.tail || coarsest) ? HF_PRECISION_FP64 : policy->precision;
     // Chebyshev-Jacobi on every point level but the coarsest
@@ -2050,9 +2191,10 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
     }
   }
   p->chunk0 = make_chunk(static_cast<int>(p->cells));
-  p->tail_lds_bytes = static_cast<size_t>(tail_doubles) * sizeof(double);
-  if (p->tail_lds_bytes > static_cast<size_t>(kTailLdsBytes)) {
-    // the coarsest level alone exceeds the tail kernel's LDS
+  if (!line_plan && 3 * p->levels.back().cells *
+                            static_cast<int64_t>(sizeof(double)) >
+                        kTailWorkBytes) {
+    // the coarsest level alone exceeds the tail
     delete p;
     return fail(HF_INVALID_PLAN, kDetailPlan);
   }
@@ -2105,9 +2247,7 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
   guard(dalloc(p, &p->kr, p->cells));
   guard(dalloc(p, &p->kp, p->cells));
   guard(dalloc(p, &p->kq, p->cells));
-  const int tail_levels = static_cast<int>(p->levels.size()) - p->tail_first;
-  guard(dalloc(p, &p->d_tail_levels, std::max(tail_levels, 1)));
-  guard(dalloc(p, &p->d_tail_ops, std::max<size_t>(p->tail_ops_host.size(), 1)));
+  if (s.code == HF_OK) guard(build_tail(p));
   if (s.code == HF_OK &&
       hipHostMalloc(reinterpret_cast<void**>(&p->host_scalars),
                     S_COUNT * sizeof(double), hipHostMallocDefault) != hipSuccess) {
@@ -2134,6 +2274,7 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
     hf_plan_destroy(p);
     return s;
   }
+  std::vector<double>().swap(p->tail_blob);
   *out = p;
   return ok();
 }
@@ -2435,11 +2576,9 @@ hf_status hf_plan_set_coefficients(hf_plan* p, const double* diag,
   p->shortcut = shortcut;
   if (into_spare)
     for (Level& L : p->levels) std::swap(static_cast<Coeffs&>(L), L.spare);
-  // the tail kernel reads its level descriptors from device memory; a plan
-  // whose descriptors could not follow the swap accepts no further solves
-  const hf_status uploaded = upload_tail(p);
-  p->coefficients_ready = uploaded.code == HF_OK;
-  HF_TRY(uploaded);
+  // a shortcut plan has no coarse hierarchy and never runs the tail
+  if (!shortcut) pack_tail(p);
+  p->coefficients_ready = true;
   return hip_check(hipGetLastError());
 }
 

@@ -236,6 +236,35 @@ def test_mg_apply_chebyshev_bitwise(torch_cuda, monkeypatch, name, stages,
     plan.close()
 
 
+@pytest.mark.parametrize("smoother", ["rb", "cheb"])
+@pytest.mark.parametrize("n", [
+    (4, 4, 4),      # one wavefront
+    (5, 13, 1),     # 65 cells: the first size beyond it
+    (16, 8, 8),     # one cell for each of the 1024 threads
+    (25, 41, 1),    # 1025
+    (13, 13, 13),   # 2197: the first level's image stays in memory
+    (9, 10, 11),    # odd periodic extent: passes from the values before
+])
+def test_tail_level_sizes_bitwise(torch_cuda, n, smoother):
+    """Grids that lie wholly in the single-workgroup tail, at the edges of
+    its cell-per-thread and residency splits: the V-cycle equals the oracle
+    bit for bit."""
+    torch = torch_cuda
+    _say(f"[tail sizes] n={n} smoother={smoother}")
+    case = mixed_case(n=n, seed=31, radius=0.12)
+    pol = dict(null_space_constant=0, anisotropy_threshold=64.0,
+               **(dict(_CHEB, f_cycle=1) if smoother == "cheb" else {}))
+    plan = _gpu_plan(torch, case, **pol)
+    assert all(plan.level_info(l)["on_tail"]
+               for l in range(plan.level_count()))
+    _, mg = O.from_case(case, O.policy(**pol))
+    r = np.random.default_rng(9).standard_normal(plan.cells)
+    z = plan.mg_apply(_t(torch, r)).cpu().numpy()
+    zo = mg.apply(r)
+    assert np.array_equal(z, zo), np.max(np.abs(z - zo))
+    plan.close()
+
+
 @pytest.mark.parametrize("name", ["sphere32", "step"])
 @pytest.mark.parametrize("tail", ["default", "0"])
 def test_mg_apply_chebyshev_projected(torch_cuda, monkeypatch, name, tail):
