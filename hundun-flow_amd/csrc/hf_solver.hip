@@ -19,6 +19,7 @@
 #include "hf_kernels.hpp"
 #include "hf_krylov.hpp"
 #include "hf_line.hpp"
+#include "hf_march.hpp"
 #include "hf_tail.hpp"
 #include "hundun_flow.h"
 
@@ -113,6 +114,9 @@ struct Level : Coeffs {
   void* lghost = nullptr;
   bool cheb = false;   // Chebyshev-Jacobi smoothing (x2 holds x_next)
   bool sweep = false;  // fused two-colour sweep kernel
+  bool march = false;  // two sweeps per launch (k_rb_march)
+  int march_zc = 0;    // planes per block of it
+  int march_blocks = 0;
   int sweep_zc = 0;    // planes per block of the sweep kernel
   int sweep_gx = 0, sweep_gy = 0, sweep_blocks = 0;
   // launch geometry: one tile per block (cells / colour cells) and chunked
@@ -523,6 +527,29 @@ int64_t sweep_min_cells() {
   return int64_t{1} << 21;
 }
 
+// HF_SWEEP_MARCH=0: two sweeps of a smoothing as two launches everywhere
+// (k_rb_march is bit for bit the same; the switch lets the parity tests
+// compare the two).
+bool march_enabled() {
+  const char* env = std::getenv("HF_SWEEP_MARCH");
+  return env == nullptr || std::atoi(env) != 0;
+}
+
+// Coarse levels run two sweeps as one march from this many cells: a march
+// takes at least seven plane steps, 13 to 16 us however small the level.
+// Measured against two colour passes per sweep: 64^3 FP64 37 us for the four
+// sweeps of a cycle either way, and the defect and restriction then fuse (4.9
+// against 9.8 us); 150x90x70 FP32 47 against 72 us; 32^3 FP64 29 against 28.
+// HF_SWEEP_MIN_CELLS overrides it.
+int64_t march_min_cells() {
+  const char* env = std::getenv("HF_SWEEP_MIN_CELLS");
+  if (env != nullptr) {
+    const long long v = std::atoll(env);
+    if (v >= 0) return v;
+  }
+  return int64_t{1} << 18;
+}
+
 // Planes per block of the fused sweep on every level that takes it (0: the
 // planner's choice); HF_SWEEP_ZC sets it.
 int sweep_zc_override() {
@@ -532,6 +559,30 @@ int sweep_zc_override() {
     if (v > 0) return v;
   }
   return 0;
+}
+
+// Launch shape of k_rb_march on level L: the z-chunks that take the fewest
+// plane steps over the rounds in which 256 CUs, one block each, work them off
+// (a chunk pays six steps to fill).
+void plan_march(Level& L) {
+  dispatch(L.prec, [&](auto t) {
+    using T = decltype(t);
+    const int64_t tiles =
+        static_cast<int64_t>((L.n[0] + kMaOutX - 1) / kMaOutX) *
+        ((L.n[1] + kMaOutY<T> - 1) / kMaOutY<T>);
+    int64_t best = 0;
+    for (int chunks = 1; chunks <= L.n[2]; ++chunks) {
+      const int zc = (L.n[2] + chunks - 1) / chunks;
+      const int64_t steps = (tiles * chunks + 255) / 256 * (zc + 6);
+      if (best != 0 && steps >= best) continue;
+      best = steps;
+      L.march_zc = zc;
+    }
+    if (sweep_zc_override() > 0)
+      L.march_zc = std::min(L.n[2], sweep_zc_override());
+    L.march_blocks = static_cast<int>(
+        tiles * ((L.n[2] + L.march_zc - 1) / L.march_zc));
+  });
 }
 
 // The retained defect of a fused-sweep level and its restriction run as one
@@ -608,7 +659,7 @@ bool op_on_tail(const hf_plan* p, const CycleOp& op) {
   return lo >= p->tail_first;
 }
 
-// k_defect_restrict applies on level l: a fused-sweep or Chebyshev level
+// k_defect_restrict applies on level l: a fused-sweep, march or Chebyshev level
 // (its retained defect comes from one stencil pass after the smoothing),
 // coarsened along every axis with even extents, full z-marching tiles of
 // even width and height, even z-chunks.
@@ -619,8 +670,8 @@ bool defect_restrict_ok(const hf_plan* p, int l) {
   const Level& Cn = p->levels[l + 1];
   const Tiles& t = L.tz;
   const int tw = 1 << t.txl, th = kBlock >> t.txl;
-  return (L.sweep || L.cheb) && L.coarsen_mask == 7 && L.n[0] % 2 == 0 &&
-         L.n[1] % 2 == 0 && L.n[2] % 2 == 0 && Cn.n[0] * 2 == L.n[0] &&
+  return (L.sweep || L.march || L.cheb) && L.coarsen_mask == 7 &&
+         L.n[0] % 2 == 0 && L.n[1] % 2 == 0 && L.n[2] % 2 == 0 && Cn.n[0] * 2 == L.n[0] &&
          Cn.n[1] * 2 == L.n[1] && Cn.n[2] * 2 == L.n[2] && tw % 2 == 0 &&
          th % 2 == 0 && L.n[0] % tw == 0 && L.n[1] % th == 0 &&
          t.per % 2 == 0;
@@ -778,6 +829,42 @@ void project_apply(hf_plan* p, int l, T* field) {
   HF_LAUNCH(k_project_apply<T>, L.tc.blocks, kBlock, 0, p->stream, L.tc,
             field, static_cast<const uint8_t*>(L.act),
             static_cast<const double*>(p->scalars + S_MEAN0 + l));
+}
+
+// Two sweeps in one launch (k_rb_march).
+template <class T>
+void march_smooth(hf_plan* p, int l, int reverse, int from_zero,
+                  double* mean_partials) {
+  Level& L = p->levels[l];
+  MarchArgs<T> a;
+  a.L = view<T>(L);
+  a.bc = p->bc;
+  a.xout = static_cast<T*>(L.x2);
+  a.mean = from_zero && p->policy.null_space_constant
+               ? p->scalars + S_MEAN0 + l
+               : nullptr;
+  a.bout = a.mean != nullptr ? static_cast<T*>(L.b2) : nullptr;
+  a.first = reverse ? 1 : 0;
+  a.zc = L.march_zc;
+  a.gx = (L.n[0] + kMaOutX - 1) / kMaOutX;
+  a.gy = (L.n[1] + kMaOutY<T> - 1) / kMaOutY<T>;
+  a.partials = mean_partials;
+  a.wx = p->d_widths[0];
+  a.wy = p->d_widths[1];
+  a.wz = p->d_widths[2];
+  const int blocks = L.march_blocks;
+  HF_PROF(p, l == 0 ? P_SWEEP_FINEST : P_SWEEP_COARSE);
+  if (from_zero)
+    HF_LAUNCH((k_rb_march<T, true, false>), blocks, kMaThreads<T>, 0,
+              p->stream, a);
+  else if (mean_partials != nullptr)
+    HF_LAUNCH((k_rb_march<T, false, true>), blocks, kMaThreads<T>, 0,
+              p->stream, a);
+  else
+    HF_LAUNCH((k_rb_march<T, false, false>), blocks, kMaThreads<T>, 0,
+              p->stream, a);
+  std::swap(L.x, L.x2);
+  if (a.bout != nullptr) std::swap(L.b, L.b2);
 }
 
 // mean_partials: the last sweep also writes the per-block partial sums of the
@@ -985,6 +1072,14 @@ template <class T>
 void point_smooth(hf_plan* p, int l, int sweeps, int reverse, int retain,
                   int from_zero, double* mean_partials) {
   Level& L = p->levels[l];
+  if (L.march && sweeps == 2) {
+    march_smooth<T>(p, l, reverse, from_zero, mean_partials);
+    if (retain) {
+      HF_PROF(p, P_DEFECT);
+      level_apply<T>(p, L, view<T>(L), 1);
+    }
+    return;
+  }
   if (L.sweep) {
     sweep_smooth<T>(p, l, sweeps, reverse, retain, from_zero, mean_partials);
     return;
@@ -1143,18 +1238,19 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
   });
 }
 
-// Whether the cycle ends with a fused level-0 sweep that can sum the mean of
-// its output: the last op smooths level 0 and its last sweep is not the
-// from-zero one.
-bool mean_in_sweep(const hf_plan* p) {
-  if (p->exec.empty() || p->exec.back().tail) return false;
+// Blocks of the level-0 launch that ends the cycle and sums the mean of its
+// output (0: none does): the last op smooths level 0, by a march or by fused
+// sweeps the last of which is not the from-zero one.
+int64_t mean_blocks(const hf_plan* p) {
+  if (p->exec.empty() || p->exec.back().tail) return 0;
   const CycleOp& op = p->exec.back().op;
   const Level& L0 = p->levels[0];
-  return op.kind == T_SMOOTH && op.level == 0 && L0.sweep && op.sweeps >= 1 &&
-         !(op.sweeps == 1 && op.from_zero);
+  if (op.kind != T_SMOOTH || op.level != 0 || op.sweeps < 1) return 0;
+  if (L0.march && op.sweeps == 2) return op.from_zero ? 0 : L0.march_blocks;
+  return L0.sweep && !(op.sweeps == 1 && op.from_zero) ? L0.sweep_blocks : 0;
 }
 
-// mean_partials: passed to the cycle's final op (see mean_in_sweep).
+// mean_partials: passed to the cycle's final op (see mean_blocks).
 void run_cycle(hf_plan* p, double* mean_partials = nullptr) {
   for (size_t n = 0; n < p->exec.size(); ++n) {
     const ExecItem& e = p->exec[n];
@@ -1233,7 +1329,7 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
     }
   });
   // the cycle's last fused sweep also sums the level-0 mean of its output
-  const bool sweep_mean = proj && !p->shortcut && mean_in_sweep(p);
+  const int64_t sweep_mean = proj && !p->shortcut ? mean_blocks(p) : 0;
   if (p->shortcut) {
     // z = D^-1 r (src/solver_mg.cpp:4926-4936); the shortcut is only
     // selected without a null space
@@ -1245,7 +1341,7 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
                 view<T>(L0));
     });
   } else {
-    run_cycle(p, sweep_mean ? p->partials : nullptr);
+    run_cycle(p, sweep_mean > 0 ? p->partials : nullptr);
   }
   const double* alpha = nullptr;
   const double* mean = nullptr;
@@ -1253,8 +1349,8 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
     using T = decltype(t);
     T* x = static_cast<T*>(L0.x);
     if (proj) {
-      if (sweep_mean)
-        finalize(p, L0.sweep_blocks, 1, F_MEAN, S_MEAN0, L0.volume);
+      if (sweep_mean > 0)
+        finalize(p, sweep_mean, 1, F_MEAN, S_MEAN0, L0.volume);
       else
         level_mean<T>(p, 0, x);
       mean = p->scalars + S_MEAN0;
@@ -2172,12 +2268,11 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
                   static_cast<int64_t>(L.n[0]) * (L.n[1] + 1) * L.n[2],
                   static_cast<int64_t>(L.n[0]) * L.n[1] * (L.n[2] + 1)});
     // (each lane owns a pair of cells of a row: nx even)
-    L.sweep = (l == 0 || L.cells >= sweep_min_cells()) && !L.tail &&
-              L.line_mask == 0 && L.fused && !L.cheb &&
-              L.n[0] >= 32 && L.n[0] % 2 == 0 && L.n[1] >= 8 &&
-              sweep_enabled() &&
-              widest * static_cast<int64_t>(elem_size(L.prec)) <
-                  (int64_t{1} << 32);
+    const bool sweep_shape =
+        !L.tail && L.line_mask == 0 && L.fused && !L.cheb && L.n[0] >= 32 &&
+        L.n[0] % 2 == 0 && L.n[1] >= 8 && sweep_enabled() &&
+        widest * static_cast<int64_t>(elem_size(L.prec)) < (int64_t{1} << 32);
+    L.sweep = sweep_shape && (l == 0 || L.cells >= sweep_min_cells());
     if (L.sweep) {
       L.sweep_gx = (L.n[0] + kSwTX - 1) / kSwTX;
       L.sweep_gy = (L.n[1] + kSwTY - 1) / kSwTY;
@@ -2189,6 +2284,9 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
         L.sweep_zc = std::min(L.n[2], sweep_zc_override());
       L.sweep_blocks = per_plane * ((L.n[2] + L.sweep_zc - 1) / L.sweep_zc);
     }
+    L.march = l == 0 ? sweep_shape : sweep_shape && L.cells >= march_min_cells();
+    L.march = L.march && L.n[2] >= 8 && march_enabled();
+    if (L.march) plan_march(L);
   }
   p->chunk0 = make_chunk(static_cast<int>(p->cells));
   if (!line_plan && 3 * p->levels.back().cells *
@@ -2214,7 +2312,7 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
     guard(dalloc_raw(p, &L.x, es * L.cells));
     guard(dalloc_raw(p, &L.b, es * L.cells));
     guard(dalloc_raw(p, &L.r, es * L.cells));
-    if (L.sweep) {
+    if (L.sweep || L.march) {
       guard(dalloc_raw(p, &L.x2, es * L.cells));
       guard(dalloc_raw(p, &L.b2, es * L.cells));
     }

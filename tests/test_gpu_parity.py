@@ -647,6 +647,56 @@ DEFECT_RESTRICT = {
 }
 
 
+def march_case(n, bc, seed=23):
+    """A sphere case on an n grid with six boundary kinds."""
+    case = hf_cases.lognormal_sphere(n=n, seed=seed, radius=0.2)
+    act = case["cell_active"].reshape(n[2], n[1], n[0])
+    fx, fy, fz = hf_cases.face_activity(act, bc)
+    case.update(bc=list(bc), x_active=fx, y_active=fy, z_active=fz)
+    return case
+
+
+@pytest.mark.parametrize("zc", ["", "1", "5"])
+@pytest.mark.parametrize("n,bc", [
+    ((32, 8, 8), (0, 0, 1, 1, 2, 2)),      # the smallest grid it takes
+    ((56, 24, 9), (1, 1, 0, 1, 1, 0)),     # one FP32 tile, three FP64 ones
+    ((58, 25, 10), (2, 2, 1, 0, 2, 2)),    # a partial tile of two columns
+    ((114, 18, 12), (0, 1, 2, 2, 1, 1)),   # wrapped rows, walls in z
+])
+def test_two_sweep_march(torch_cuda, monkeypatch, n, bc, zc):
+    """Two sweeps in one pass over a level (k_rb_march) on tile and chunk
+    edges and every boundary kind: FP64 equal to the oracle, FP32 and BF16 to
+    two launches, bit for bit; the projected cycle to 1e-12."""
+    torch = torch_cuda
+    _say(f"[march] n={n} bc={bc} zc={zc or 'planned'}")
+    monkeypatch.setenv("HF_SWEEP_MIN_CELLS", "0")
+    if zc:
+        monkeypatch.setenv("HF_SWEEP_ZC", zc)
+    case = march_case(n, bc)
+    pol = dict(null_space_constant=0, anisotropy_threshold=64.0)
+    _, mg = O.from_case(case, O.policy(**pol))
+    r = np.random.default_rng(17).standard_normal(n[0] * n[1] * n[2])
+    zo = mg.apply(r)
+    for precision in ("fp64", "fp32", "bf16"):
+        z = {}
+        for on in ("1", "0"):
+            monkeypatch.setenv("HF_SWEEP_MARCH", on)
+            plan = _gpu_plan(torch, case, precision=precision, **pol)
+            z[on] = plan.mg_apply(_t(torch, r)).cpu().numpy()
+            plan.close()
+        assert np.array_equal(z["1"], z["0"]), precision
+        if precision == "fp64":
+            assert np.array_equal(z["1"], zo)
+    monkeypatch.setenv("HF_SWEEP_MARCH", "1")
+    pol["null_space_constant"] = 1
+    _, mg = O.from_case(case, O.policy(**pol))
+    plan = _gpu_plan(torch, case, **pol)
+    r = case["rhs"]
+    z, zo = plan.mg_apply(_t(torch, r)).cpu().numpy(), mg.apply(r)
+    plan.close()
+    assert np.linalg.norm(z - zo) <= 1e-12 * np.linalg.norm(zo)
+
+
 @pytest.mark.parametrize("name", list(DEFECT_RESTRICT))
 @pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16"])
 @pytest.mark.parametrize("null", [0, 1])
