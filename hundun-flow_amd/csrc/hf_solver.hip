@@ -13,11 +13,13 @@
 #include <limits>
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "hf_assembly.hpp"
 #include "hf_kernels.hpp"
 #include "hf_krylov.hpp"
+#include "hf_leg.hpp"
 #include "hf_line.hpp"
 #include "hf_march.hpp"
 #include "hf_tail.hpp"
@@ -114,6 +116,7 @@ struct Level : Coeffs {
   void* lghost = nullptr;
   bool cheb = false;   // Chebyshev-Jacobi smoothing (x2 holds x_next)
   bool sweep = false;  // fused two-colour sweep kernel
+  bool leg = false;    // one launch per way down and way up (k_leg)
   bool march = false;  // two sweeps per launch (k_rb_march)
   int march_zc = 0;    // planes per block of it
   int march_blocks = 0;
@@ -188,6 +191,9 @@ struct ExecItem {
   // a retaining smoothing whose defect and the following restriction run
   // as one kernel (k_defect_restrict); that restriction item is skipped
   bool defect_restrict = false;
+  // the smoothing and restriction, or prolongation and smoothing, that start
+  // here run as one launch (k_leg); the second item is skipped
+  bool leg = false;
   bool skip = false;
 };
 
@@ -626,6 +632,22 @@ bool line_relaxation_enabled() {
 }
 
 
+// Largest level whose way down and way up each run as one launch (k_leg).
+// Measured, both legs of a V(2,2) cycle against the separate launches: 16^3
+// FP64 15 us against 41, 32^3 30 against 42, 64x32x32 FP32 about 57 against
+// 43; Chebyshev (1,2) legs 16^3 15 against 19, 64^3 29 against 23.
+// HF_LEG_CELLS overrides it (0: none).
+constexpr int64_t kLegMaxBlocks = 512;
+
+int64_t leg_max_cells() {
+  const char* env = std::getenv("HF_LEG_CELLS");
+  if (env != nullptr) {
+    const long long v = std::atoll(env);
+    if (v >= 0) return v;
+  }
+  return int64_t{1} << 15;
+}
+
 int64_t tail_threshold() {
   const char* env = std::getenv("HF_TAIL_CELLS");
   if (env != nullptr) {
@@ -677,6 +699,49 @@ bool defect_restrict_ok(const hf_plan* p, int l) {
          t.per % 2 == 0;
 }
 
+// Passes over a level of one smoothing: colour passes or Chebyshev stages.
+int smoothing_passes(const Level& L, int sweeps) {
+  return L.cheb ? sweeps : 2 * sweeps;
+}
+
+// Halo of a leg: every pass that reads neighbours takes one cell, and so
+// does the defect on the way down; the first pass from x = 0 reads none.
+int leg_halo(const Level& L, int sweeps, bool down, bool from_zero) {
+  return smoothing_passes(L, sweeps) + (down && !from_zero ? 1 : 0);
+}
+
+// Boxes of a leg with halo h on level L.
+struct LegBoxes {
+  int o, g[3];
+  int64_t blocks;
+};
+
+LegBoxes leg_boxes(const Level& L, int h) {
+  LegBoxes b{};
+  b.o = kLegE - 2 * h;
+  b.blocks = 1;
+  for (int a = 0; a < 3; ++a) {
+    b.g[a] = (L.n[a] + b.o - 1) / b.o;
+    b.blocks *= b.g[a];
+  }
+  return b;
+}
+
+// k_leg runs level l: a point-smoothed grid level coarsened along every
+// axis, small enough, whose legs take at most two blocks per CU.
+bool leg_ok(const hf_plan* p, int l) {
+  if (l + 1 >= static_cast<int>(p->levels.size())) return false;
+  const Level& L = p->levels[l];
+  // a V-cycle visits every level from zero, an F-cycle the coarse ones twice
+  const bool zero_only = !p->policy.f_cycle || l == 0;
+  const int h =
+      std::max(leg_halo(L, p->policy.pre_sweeps, true, zero_only),
+               leg_halo(L, p->policy.post_sweeps, false, false));
+  return !L.tail && L.line_mask == 0 && L.coarsen_mask == 7 &&
+         L.cells <= leg_max_cells() && h <= kLegHalo &&
+         leg_boxes(L, h).blocks <= kLegMaxBlocks;
+}
+
 void build_exec(hf_plan* p) {
   p->program.clear();
   p->exec.clear();
@@ -712,6 +777,14 @@ void build_exec(hf_plan* p) {
   for (size_t n = 0; n + 1 < p->exec.size(); ++n) {
     ExecItem& a = p->exec[n];
     ExecItem& b = p->exec[n + 1];
+    if (!a.tail && !b.tail && a.op.level == b.op.level &&
+        p->levels[a.op.level].leg &&
+        ((a.op.kind == T_SMOOTH && b.op.kind == T_RESTRICT) ||
+         (a.op.kind == T_PROLONG && b.op.kind == T_SMOOTH))) {
+      a.leg = true;
+      b.skip = true;
+      continue;
+    }
     if (a.tail || b.tail || a.op.kind != T_SMOOTH || !a.op.retain ||
         b.op.kind != T_RESTRICT || b.op.level != a.op.level ||
         !defect_restrict_ok(p, a.op.level))
@@ -1124,9 +1197,9 @@ void point_smooth(hf_plan* p, int l, int sweeps, int reverse, int retain,
 
 // A level that needs the projected b and x = 0 in memory before a cycle
 // visits it (a point-smoothed grid level starts from zero and applies the
-// projection in its first pass, the tail when it loads b).
+// projection in its first pass, the tail and a leg whenever they load b).
 bool wants_stored_start(const Level& L) {
-  return !L.tail && (L.line_mask != 0 || L.cheb);
+  return !L.tail && !L.leg && (L.line_mask != 0 || L.cheb);
 }
 
 // Whether level 0's b is projected in memory before the cycle: also where
@@ -1134,7 +1207,78 @@ bool wants_stored_start(const Level& L) {
 // it loads it.
 bool entry_projects(const hf_plan* p) {
   const Level& L0 = p->levels[0];
-  return wants_stored_start(L0) || (L0.tail && !p->policy.unit_linear);
+  return wants_stored_start(L0) ||
+         ((L0.tail || L0.leg) && !p->policy.unit_linear);
+}
+
+// One leg of level op.level (k_leg): the smoothing `op` with the defect and
+// the restriction that follow it (down), or with the prolongation before it.
+void exec_leg(hf_plan* p, const CycleOp& op, bool down,
+              double* mean_partials) {
+  Level& L = p->levels[op.level];
+  Level& Cd = p->levels[op.level + 1];
+  const bool proj = p->policy.null_space_constant != 0;
+  const int h = leg_halo(L, op.sweeps, down, op.from_zero != 0);
+  const LegBoxes box = leg_boxes(L, h);
+  dispatch(L.prec, [&](auto tf) {
+    using Tf = decltype(tf);
+    using C = typename Compute<Tf>::type;
+    dispatch(Cd.prec, [&](auto tc) {
+      using Tc = decltype(tc);
+      // (a coarse level has the fine one's storage type or is FP64)
+      if constexpr (std::is_same<Tc, Tf>::value ||
+                    std::is_same<Tc, double>::value) {
+        LegArgs<Tf, Tc> a{};
+        a.F = view<Tf>(L);
+        a.Cl = view<Tc>(Cd);
+        a.bc = p->bc;
+        a.xout = static_cast<Tf*>(L.x2);
+        a.mean = proj && !(op.level == 0 && entry_projects(p))
+                     ? p->scalars + S_MEAN0 + op.level
+                     : nullptr;
+        a.passes = smoothing_passes(L, op.sweeps);
+        a.first = op.reverse ? 1 : 0;
+        a.from_zero = op.from_zero;
+        a.h = h;
+        a.zero_x = wants_stored_start(Cd) ? 1 : 0;
+        a.o = box.o;
+        a.gx = box.g[0];
+        a.gy = box.g[1];
+        a.partials = down ? (proj ? p->partials : nullptr) : mean_partials;
+        ChebStage factors(p->policy.chebyshev_lower_fraction);
+        for (int s = 0; L.cheb && s < a.passes; ++s) {
+          double rf = 0.0, pf = 0.0;
+          factors.next(&rf, &pf);
+          a.rf[s] = static_cast<C>(rf);
+          a.pf[s] = static_cast<C>(pf);
+        }
+        HF_PROF(p, op.level == 0 ? P_RB_FINEST : P_RB_COARSE);
+        auto launch = [&](auto mode) {
+          constexpr int kMode = decltype(mode)::value;
+          if (down)
+            HF_LAUNCH((k_leg<Tf, Tc, true, kMode>), box.blocks, kLegThreads,
+                      0, p->stream, a);
+          else
+            HF_LAUNCH((k_leg<Tf, Tc, false, kMode>), box.blocks, kLegThreads,
+                      0, p->stream, a);
+        };
+        if (L.cheb && L.fused)
+          launch(std::integral_constant<int, kLegCheb>{});
+        else if (L.cheb)
+          launch(std::integral_constant<int, kLegChebOdd>{});
+        else if (L.fused)
+          launch(std::integral_constant<int, kLegRb>{});
+        else
+          launch(std::integral_constant<int, kLegSeparated>{});
+      }
+      if (down && proj) {
+        finalize(p, box.blocks, 1, F_MEAN, S_MEAN0 + op.level + 1, Cd.volume);
+        if (wants_stored_start(Cd))
+          project_apply<Tc>(p, op.level + 1, static_cast<Tc*>(Cd.b));
+      }
+    });
+  });
+  std::swap(L.x, L.x2);
 }
 
 void exec_grid_op(hf_plan* p, const CycleOp& op,
@@ -1246,6 +1390,7 @@ int64_t mean_blocks(const hf_plan* p) {
   const CycleOp& op = p->exec.back().op;
   const Level& L0 = p->levels[0];
   if (op.kind != T_SMOOTH || op.level != 0 || op.sweeps < 1) return 0;
+  if (L0.leg) return leg_boxes(L0, leg_halo(L0, op.sweeps, false, false)).blocks;
   if (L0.march && op.sweeps == 2) return op.from_zero ? 0 : L0.march_blocks;
   return L0.sweep && !(op.sweeps == 1 && op.from_zero) ? L0.sweep_blocks : 0;
 }
@@ -1255,6 +1400,12 @@ void run_cycle(hf_plan* p, double* mean_partials = nullptr) {
   for (size_t n = 0; n < p->exec.size(); ++n) {
     const ExecItem& e = p->exec[n];
     if (e.skip) continue;
+    if (e.leg) {
+      const bool down = e.op.kind == T_SMOOTH;
+      exec_leg(p, down ? e.op : p->exec[n + 1].op, down,
+               n + 2 == p->exec.size() ? mean_partials : nullptr);
+      continue;
+    }
     if (!e.tail) {
       exec_grid_op(p, e.op, n + 1 == p->exec.size() ? mean_partials : nullptr,
                    e.defect_restrict);
@@ -1306,9 +1457,11 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
   const bool proj = p->policy.null_space_constant != 0;
   const bool tail0 = entry_projects(p);
   // (a grid Chebyshev level 0 starts with a from-zero stage, which reads
-  // b and D only, and the tail starts from zero by itself: no x = 0 there)
-  const bool zero_x = !L0.tail && (L0.line_mask != 0 ||
-                                   (L0.cheb && !p->cheb_first));
+  // b and D only, and the tail and a leg start from zero by themselves: no
+  // x = 0 there)
+  const bool zero_x =
+      !L0.tail && !L0.leg &&
+      (L0.line_mask != 0 || (L0.cheb && !p->cheb_first));
   dispatch(L0.prec, [&](auto t) {
     using T = decltype(t);
     T* b = static_cast<T*>(L0.b);
@@ -1826,7 +1979,7 @@ hf_status fgmres_impl(hf_plan* p, const double* rhs, double* solution,
   // projection, no volume-scaled rows.
   const bool entry_in_combine =
       !vrows && p->policy.null_space_constant == 0 && !L0.tail &&
-      L0.line_mask == 0 && (!L0.cheb || p->cheb_first);
+      L0.line_mask == 0 && (!L0.cheb || L0.leg || p->cheb_first);
   bool entered_next = false;
   auto combine = [&](double* dst, const double* src, const double* basis,
                      const double* s, size_t count, double post, int scale) {
@@ -2268,8 +2421,9 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
                   static_cast<int64_t>(L.n[0]) * (L.n[1] + 1) * L.n[2],
                   static_cast<int64_t>(L.n[0]) * L.n[1] * (L.n[2] + 1)});
     // (each lane owns a pair of cells of a row: nx even)
+    L.leg = leg_ok(p, static_cast<int>(l));
     const bool sweep_shape =
-        !L.tail && L.line_mask == 0 && L.fused && !L.cheb && L.n[0] >= 32 &&
+        !L.tail && !L.leg && L.line_mask == 0 && L.fused && !L.cheb && L.n[0] >= 32 &&
         L.n[0] % 2 == 0 && L.n[1] >= 8 && sweep_enabled() &&
         widest * static_cast<int64_t>(elem_size(L.prec)) < (int64_t{1} << 32);
     L.sweep = sweep_shape && (l == 0 || L.cells >= sweep_min_cells());
@@ -2315,8 +2469,9 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
     if (L.sweep || L.march) {
       guard(dalloc_raw(p, &L.x2, es * L.cells));
       guard(dalloc_raw(p, &L.b2, es * L.cells));
+    } else if (L.cheb || L.leg) {
+      guard(dalloc_raw(p, &L.x2, es * L.cells));
     }
-    if (L.cheb) guard(dalloc_raw(p, &L.x2, es * L.cells));
     if (L.line_mask != 0) {
       const size_t cs = L.prec == HF_PRECISION_FP64 ? 8 : 4;
       guard(dalloc_raw(p, &L.lcw, cs * L.cells));
@@ -2333,8 +2488,10 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
   }
   // one partial per tile (level 0 has the most) or per 256-element block
   int64_t max_blocks = blocks_for(p->cells);
-  for (const Level& L : p->levels)
+  for (const Level& L : p->levels) {
     max_blocks = std::max<int64_t>(max_blocks, L.tc.count);
+    if (L.leg) max_blocks = std::max(max_blocks, leg_boxes(L, kLegHalo).blocks);
+  }
   p->partial_stride = max_blocks + 8;
   guard(dalloc(p, &p->partials, 3 * p->partial_stride));
   guard(dalloc(p, &p->folded, 3 * kFoldStride));
@@ -2712,7 +2869,8 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
   // reads no x in its first stage, and mg_apply projects its b)
   const bool fuse_entry = !p->levels[0].tail &&
                           p->levels[0].line_mask == 0 &&
-                          (!p->levels[0].cheb || p->cheb_first);
+                          (!p->levels[0].cheb || p->levels[0].leg ||
+                           p->cheb_first);
   const Chunk ch = p->chunk0;
   const int nbv = chunk_blocks(ch);
   double* x = p->kx;

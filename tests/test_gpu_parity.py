@@ -647,6 +647,51 @@ DEFECT_RESTRICT = {
 }
 
 
+@pytest.mark.parametrize("smoother", ["rb", "rb_f", "cheb"])
+@pytest.mark.parametrize("n,bc", [
+    ((18, 17, 13), (0, 1, 1, 0, 1, 1)),    # partial boxes at every far side
+    ((20, 16, 12), (2, 2, 0, 1, 2, 2)),    # whole boxes, wrapped regions
+    ((21, 14, 19), (1, 0, 2, 2, 2, 2)),    # odd periodic z: values before
+    ((32, 4, 32), (1, 1, 2, 2, 0, 0)),     # a region of three periods in y
+])
+def test_leg_bitwise(torch_cuda, monkeypatch, n, bc, smoother):
+    """A small level's way down and way up as one launch each (k_leg), on box
+    edges, wrapped regions and every boundary kind: FP64 equal to the oracle,
+    FP32 and BF16 to the separate launches, bit for bit; the projected cycle
+    to 1e-12."""
+    torch = torch_cuda
+    _say(f"[leg] n={n} bc={bc} smoother={smoother}")
+    monkeypatch.setenv("HF_TAIL_CELLS", "0")
+    case = march_case(n, bc, seed=29)
+    pol = dict(null_space_constant=0, anisotropy_threshold=64.0)
+    if smoother == "cheb":
+        pol.update(_CHEB, f_cycle=1, pre_sweeps=1, post_sweeps=2)
+    elif smoother == "rb_f":
+        pol.update(f_cycle=1)
+    _, mg = O.from_case(case, O.policy(**pol))
+    r = np.random.default_rng(19).standard_normal(n[0] * n[1] * n[2])
+    zo = mg.apply(r)
+    for precision in ("fp64", "fp32", "bf16"):
+        z = {}
+        for cells in ("32768", "0"):
+            monkeypatch.setenv("HF_LEG_CELLS", cells)
+            plan = _gpu_plan(torch, case, precision=precision, **pol)
+            z[cells] = plan.mg_apply(_t(torch, r)).cpu().numpy()
+            plan.close()
+        assert np.array_equal(z["32768"], z["0"]), precision
+        if precision == "fp64":
+            assert np.array_equal(z["0"], zo)
+    monkeypatch.setenv("HF_LEG_CELLS", "32768")
+    for unit in (1, 0):
+        pol.update(null_space_constant=1, unit_linear=unit)
+        _, mg = O.from_case(case, O.policy(**pol))
+        plan = _gpu_plan(torch, case, **pol)
+        r = case["rhs"]
+        z, zo = plan.mg_apply(_t(torch, r)).cpu().numpy(), mg.apply(r)
+        plan.close()
+        assert np.linalg.norm(z - zo) <= 1e-12 * np.linalg.norm(zo)
+
+
 def march_case(n, bc, seed=23):
     """A sphere case on an n grid with six boundary kinds."""
     case = hf_cases.lognormal_sphere(n=n, seed=seed, radius=0.2)
