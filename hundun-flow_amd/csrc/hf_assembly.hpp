@@ -32,46 +32,49 @@ struct PressureSystem {
   double* rhs;
 };
 
-// Face inputs must be finite, the coefficients also non-negative
-// (finite_nonnegative_faces / finite_faces); a violation sets bit 0 of *bad.
-__global__ void k_check_faces(const double* beta, const double* phi,
-                              int64_t count, int* bad) {
-  const int64_t f = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (f >= count) return;
-  const double b = beta[f];
-  if (!isfinite(b) || b < 0.0 || !isfinite(phi[f])) atomicOr(bad, 1);
-}
-
 // One cell per thread.  write == 0: the preflight, which only checks every
-// value the reference checks (a failure sets bit 1 of *bad); write == 1:
-// stores D and b.
+// value the reference checks: the cell's (a failure sets bit 1 of *bad), and
+// its six faces' coefficients (finite, not negative) and fluxes (finite;
+// finite_nonnegative_faces / finite_faces, a failure sets bit 0), which it
+// reads anyway.  write == 1: stores D and b.
 __global__ void k_pressure_system(PressureSystem s, int write, int* bad) {
-  const int64_t c = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  const int64_t plane = static_cast<int64_t>(s.nx) * s.ny;
-  if (c >= plane * s.nz) return;
-  const int i = static_cast<int>(c % s.nx);
-  const int j = static_cast<int>((c / s.nx) % s.ny);
-  const int k = static_cast<int>(c / plane);
+  const int plane = s.nx * s.ny;
+  const int c = xcd_block32(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  if (c < 0 || c >= plane * s.nz) return;
+  const int k = c / plane;
+  const int in_plane = c - k * plane;
+  const int j = in_plane / s.nx;
+  const int i = in_plane - j * s.nx;
   const double volume = s.w.x[i] * s.w.y[j] * s.w.z[k];
   const double r = s.rho[c], rn = s.rho_n[c];
   const double rnm1 = s.rho_nm1 != nullptr ? s.rho_nm1[c] : 0.0;
   const double src = s.source != nullptr ? s.source[c] : 0.0;
   const double drho = s.drho_dp[c];
   const double defect = volume * (s.a0 * r + s.a1 * rn + s.a2 * rnm1 - src);
-  const int64_t xf = i + static_cast<int64_t>(s.nx + 1) * (j + static_cast<int64_t>(s.ny) * k);
-  const int64_t yf = i + static_cast<int64_t>(s.nx) * (j + static_cast<int64_t>(s.ny + 1) * k);
-  const int64_t zf = c;
-  const double faces = s.bx[xf] + s.bx[xf + 1] + s.by[yf] + s.by[yf + s.nx] +
-                       s.bz[zf] + s.bz[zf + plane];
+  const int xf = c + j + s.ny * k;
+  const int yf = c + s.nx * k;
+  const int zf = c;
+  const double beta[6] = {s.bx[xf], s.bx[xf + 1],     s.by[yf],
+                          s.by[yf + s.nx], s.bz[zf], s.bz[zf + plane]};
+  const double phi[6] = {s.phix[xf], s.phix[xf + 1],     s.phiy[yf],
+                         s.phiy[yf + s.nx], s.phiz[zf], s.phiz[zf + plane]};
+  const double faces =
+      beta[0] + beta[1] + beta[2] + beta[3] + beta[4] + beta[5];
   const double d = s.a0 * volume * drho + faces;
-  const double flux = s.phix[xf + 1] - s.phix[xf] + s.phiy[yf + s.nx] -
-                      s.phiy[yf] + s.phiz[zf + plane] - s.phiz[zf];
+  const double flux =
+      phi[1] - phi[0] + phi[3] - phi[2] + phi[5] - phi[4];
   const double b = -(defect + flux);
   if (write) {
     s.diag[c] = d;
     s.rhs[c] = b;
     return;
   }
+  bool face_ok = true;
+#pragma unroll
+  for (int f = 0; f < 6; ++f)
+    face_ok = face_ok && isfinite(beta[f]) && !(beta[f] < 0.0) &&
+              isfinite(phi[f]);
+  if (!face_ok) atomicOr(bad, 1);
   const bool inputs = isfinite(r) && isfinite(rn) && isfinite(drho) &&
                       (s.rho_nm1 == nullptr || isfinite(rnm1)) &&
                       (s.source == nullptr || isfinite(src));

@@ -86,30 +86,41 @@ __device__ __forceinline__ void face_rule_grad(const double* f, int count,
   *gr = beta * beta / area * (dr / (mr * mr));
 }
 
-__global__ void k_assemble_faces(AxisGeom g, int axis, const double* m,
-                                 double* out, int64_t count) {
-  const int64_t t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (t >= count) return;
-  int e[3] = {g.n[0], g.n[1], g.n[2]};
-  e[axis] += 1;
-  const int i = static_cast<int>(t % e[0]);
-  const int j = static_cast<int>((t / e[0]) % e[1]);
-  const int k = static_cast<int>(t / ((int64_t)e[0] * e[1]));
-  int c[3] = {i, j, k};
-  const int nrm = c[axis];
-  const int a1 = axis == 0 ? 1 : 0;
-  const int a2 = axis == 2 ? 1 : 2;
-  const double area = (g.faces[a1][c[a1] + 1] - g.faces[a1][c[a1]]) *
-                      (g.faces[a2][c[a2] + 1] - g.faces[a2][c[a2]]);
-  int cl[3] = {i, j, k};
-  int cr[3] = {i, j, k};
-  cl[axis] = nrm == 0 ? g.n[axis] - 1 : nrm - 1;
-  cr[axis] = nrm == g.n[axis] ? 0 : nrm;
-  const int64_t nx = g.n[0], ny = g.n[1];
-  const double ml = m[cl[0] + nx * (cl[1] + ny * cl[2])];
-  const double mr = m[cr[0] + nx * (cr[1] + ny * cr[2])];
-  const int kind = nrm == 0 ? g.kind[2 * axis] : g.kind[2 * axis + 1];
-  out[t] = face_rule(g.faces[axis], g.n[axis], nrm, kind, area, ml, mr);
+// All face coefficients: a thread owns the low face of its cell along each
+// axis, and the high one at the end of the axis.  32 bytes a cell and nine
+// FP64 divisions, which bound it: 220 us at 256^3.  A launch per axis, with
+// 64-bit divisions for the indices, read m three times over: 345 us.
+__global__ void k_assemble_faces(AxisGeom g, const double* m, double* bx,
+                                 double* by, double* bz) {
+  const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
+  const int plane = nx * ny;
+  const int c = xcd_block32(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  if (c < 0 || c >= plane * nz) return;
+  const int k = c / plane;
+  const int r = c - k * plane;
+  const int j = r / nx;
+  const int ijk[3] = {r - j * nx, j, k};
+  const int step[3] = {1, nx, plane};
+  double w[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+    w[a] = g.faces[a][ijk[a] + 1] - g.faces[a][ijk[a]];
+  const double mc = m[c];
+  double* out[3] = {bx, by, bz};
+  const int at[3] = {c + j + ny * k, c + nx * k, c};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const double area = a == 0 ? w[1] * w[2]
+                               : (a == 1 ? w[0] * w[2] : w[0] * w[1]);
+    const int n = g.n[a], i = ijk[a];
+    const double low = m[i > 0 ? c - step[a] : c + (n - 1) * step[a]];
+    out[a][at[a]] =
+        face_rule(g.faces[a], n, i, g.kind[2 * a], area, low, mc);
+    if (i + 1 == n)
+      out[a][at[a] + step[a]] =
+          face_rule(g.faces[a], n, n, g.kind[2 * a + 1], area, mc,
+                    m[c - (n - 1) * step[a]]);
+  }
 }
 
 __global__ void k_face_sum_diag(int nx, int ny, int nz, const double* bx,
@@ -126,66 +137,128 @@ __global__ void k_face_sum_diag(int nx, int ny, int nz, const double* bx,
             bz[c + (int64_t)nx * ny];
 }
 
+// Storage-precision copies of one level's operator (null: the level is FP64).
+template <class T>
+struct StoredCoeffs {
+  T* D;
+  T* fx;
+  T* fy;
+  T* fz;
+};
+
+// What a refresh kernel leaves for k_refresh_finish: the block sums of fluid
+// volume and, on level 0, the block maxima of the row ratio; failed checks
+// set bits of *bad.
+struct RefreshOut {
+  double* volume;
+  double* ratio;  // null: not taken
+  int* bad;
+};
+
+// Certified SDD M-matrix check of one row (src/solver_mg.cpp:1965-2019).
+__device__ __forceinline__ bool row_invalid(double d, double faces,
+                                            double vol) {
+  const bool fail =
+      !isfinite(d) || !(d > 0.0) || !isfinite(faces) || faces < 0.0;
+  return fail || (vol == 0.0 ? d != 1.0 || faces != 0.0 : faces > d);
+}
+
+// Largest value of the block (fixed order); valid in thread 0.
+__device__ __forceinline__ double block_max(double v, double* scratch) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+#pragma unroll
+  for (int offset = kWave / 2; offset > 0; offset >>= 1)
+    v = fmax(v, __shfl_down(v, offset, kWave));
+  if (lane == 0) scratch[wave] = v;
+  __syncthreads();
+  double m = 0.0;
+  if (threadIdx.x == 0) {
+    const int waves = (blockDim.x + kWave - 1) / kWave;
+    for (int w = 0; w < waves; ++w) m = fmax(m, scratch[w]);
+  }
+  __syncthreads();
+  return m;
+}
+
 // Level-0 masking (src/solver_mg.cpp:1469-1570): faces times activity,
 // solid diagonal 1, fluid diagonal D - original faces + active faces, fluid
-// volume w_x*w_y*w_z (0 on solids).
+// volume w_x*w_y*w_z (0 on solids); with it the checks of the masked row, its
+// ratio (sum of the six faces, physical boundaries included) / D for the
+// diagonal shortcut (src/solver_mg.cpp:1573-1611), the storage-precision
+// copies and a copy of the face masks for the adjoint.  A thread owns its
+// cell and the cell's low faces, and the high ones at the end of an axis.
+// One pass, 96 bytes a cell for an FP32 cycle, near the copy rate: 362 us at
+// 256^3.  Masking, the checks, the ratio, the copies and the volume sum as
+// launches of their own took 1020 us.
 struct Finest {
   int nx, ny, nz;
   const double* D;
-  const double* bx;
-  const double* by;
-  const double* bz;
-  const uint8_t* ca;
-  const uint8_t* fxa;
-  const uint8_t* fya;
-  const uint8_t* fza;
-  const double* wx;
-  const double* wy;
-  const double* wz;
+  const double* b[3];
+  const uint8_t* ca;      // null: every cell and face active
+  const uint8_t* fa[3];
+  const double* w[3];
   double* oD;
-  double* ofx;
-  double* ofy;
-  double* ofz;
+  double* of[3];
   double* vol;
   uint8_t* act;
+  uint8_t* ofa[3];
 };
 
-__global__ void k_mask_faces(const double* raw, const uint8_t* active,
-                             double* out, int64_t count) {
-  const int64_t t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (t >= count) return;
-  out[t] = raw[t] * (active == nullptr ? 1.0 : static_cast<double>(active[t]));
-}
-
-__global__ void k_mask_cells(Finest f) {
-  const int64_t nx = f.nx, ny = f.ny;
-  const int64_t cells = nx * ny * f.nz;
-  const int64_t c = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (c >= cells) return;
-  const int i = static_cast<int>(c % nx);
-  const int j = static_cast<int>((c / nx) % ny);
-  const int k = static_cast<int>(c / (nx * ny));
-  double v = f.wx[i] * f.wy[j] * f.wz[k];
-  const bool solid = f.ca != nullptr && f.ca[c] == 0;
-  if (solid) v = 0.0;
-  f.vol[c] = v;
-  f.act[c] = solid ? 0 : 1;
-  double d = f.D[c];
-  if (f.ca != nullptr) {
-    if (solid) {
-      d = 1.0;
-    } else {
-      const int64_t row = j + ny * k;
-      const int64_t fyo = c + nx * k;
-      const int64_t zhi = c + nx * ny;
-      const double original = f.bx[c + row] + f.bx[c + row + 1] + f.by[fyo] +
-                              f.by[fyo + nx] + f.bz[c] + f.bz[zhi];
-      const double active = f.ofx[c + row] + f.ofx[c + row + 1] + f.ofy[fyo] +
-                            f.ofy[fyo + nx] + f.ofz[c] + f.ofz[zhi];
-      d = d - original + active;
+template <class T>
+__global__ void k_mask_level(Finest f, StoredCoeffs<T> s, RefreshOut out) {
+  __shared__ double scratch[16];
+  const int nx = f.nx, ny = f.ny, plane = nx * ny;
+  const int lb = xcd_block32(blockIdx.x, gridDim.x);
+  const int c = lb * kBlock + static_cast<int>(threadIdx.x);
+  double vol = 0.0, ratio = 0.0;
+  if (c >= 0 && c < plane * f.nz) {
+    const int k = c / plane;
+    const int r = c - k * plane;
+    const int j = r / nx;
+    const int ijk[3] = {r - j * nx, j, k};
+    const int n[3] = {nx, ny, f.nz};
+    const int step[3] = {1, nx, plane};
+    const int at[3] = {c + j + ny * k, c + nx * k, c};
+    const bool solid = f.ca != nullptr && f.ca[c] == 0;
+    vol = f.w[0][ijk[0]] * f.w[1][j] * f.w[2][k];
+    if (solid) vol = 0.0;
+    T* copies[3] = {s.fx, s.fy, s.fz};
+    double original = 0.0, active = 0.0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        const int face = at[a] + side * step[a];
+        const double raw = f.b[a][face];
+        const uint8_t open = f.ca == nullptr ? 1 : f.fa[a][face];
+        const double masked =
+            raw * (f.ca == nullptr ? 1.0 : static_cast<double>(open));
+        original = a == 0 && side == 0 ? raw : original + raw;
+        active = a == 0 && side == 0 ? masked : active + masked;
+        if (side == 0 || ijk[a] + 1 == n[a]) {
+          f.of[a][face] = masked;
+          if (copies[a] != nullptr) copies[a][face] = st<T>(masked);
+          if (f.ca != nullptr) f.ofa[a][face] = open;
+        }
+      }
     }
+    double d = f.D[c];
+    if (f.ca != nullptr) d = solid ? 1.0 : d - original + active;
+    f.oD[c] = d;
+    if (s.D != nullptr) s.D[c] = st<T>(d);
+    f.vol[c] = vol;
+    f.act[c] = solid ? 0 : 1;
+    if (row_invalid(d, active, vol)) atomicOr(out.bad, 2);
+    ratio = active / d;
+    if (!(ratio >= 0.0)) ratio = 0.0;  // max(0, NaN) keeps 0 (std::max)
   }
-  f.oD[c] = d;
+  vol = block_sum(vol, scratch);
+  if (threadIdx.x == 0) out.volume[lb] = vol;
+  if (out.ratio != nullptr) {
+    ratio = block_max(ratio, scratch);
+    if (threadIdx.x == 0) out.ratio[lb] = ratio;
+  }
 }
 
 // Coarse aggregation (src/solver_mg.cpp:1706-1962) evaluated per coarse
@@ -257,95 +330,115 @@ struct Coarse64 {
   uint8_t* act;
 };
 
-__global__ void k_coarse_cells(Agg a, Fine64 f, Coarse64 c) {
-  const int64_t cells = (int64_t)a.cn[0] * a.cn[1] * a.cn[2];
-  const int64_t t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (t >= cells) return;
-  const int ci = static_cast<int>(t % a.cn[0]);
-  const int cj = static_cast<int>((t / a.cn[0]) % a.cn[1]);
-  const int ck = static_cast<int>(t / ((int64_t)a.cn[0] * a.cn[1]));
-  const int* fn = a.fn;
-  const int fxe[3] = {fn[0] + 1, fn[1], fn[2]};
-  const int fye[3] = {fn[0], fn[1] + 1, fn[2]};
-  const int fze[3] = {fn[0], fn[1], fn[2] + 1};
-  c.vol[t] = aggregate_entry(a, -1, ci, cj, ck, [&](int i, int j, int k) {
-    return f.vol[fidx(fn, i, j, k)];
-  });
-  c.D[t] = aggregate_entry(a, -1, ci, cj, ck, [&](int i, int j, int k) {
-    const int64_t cc = fidx(fn, i, j, k);
-    if (f.vol[cc] == 0.0) return 0.0;
-    const double faces = f.fx[fidx(fxe, i, j, k)] + f.fx[fidx(fxe, i + 1, j, k)] +
-                         f.fy[fidx(fye, i, j, k)] + f.fy[fidx(fye, i, j + 1, k)] +
-                         f.fz[fidx(fze, i, j, k)] + f.fz[fidx(fze, i, j, k + 1)];
-    const double reaction = f.D[cc] - faces;
-    return reaction > 0.0 ? reaction : 0.0;
-  });
-}
-
-__global__ void k_coarse_faces(Agg a, int axis, const double* fine,
-                               double* coarse, double scale) {
-  int ce[3] = {a.cn[0], a.cn[1], a.cn[2]};
-  ce[axis] += 1;
-  int fe[3] = {a.fn[0], a.fn[1], a.fn[2]};
-  fe[axis] += 1;
-  const int64_t count = (int64_t)ce[0] * ce[1] * ce[2];
-  const int64_t t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (t >= count) return;
-  const int ci = static_cast<int>(t % ce[0]);
-  const int cj = static_cast<int>((t / ce[0]) % ce[1]);
-  const int ck = static_cast<int>(t / ((int64_t)ce[0] * ce[1]));
-  const double v = aggregate_entry(a, axis, ci, cj, ck,
-                                   [&](int i, int j, int k) {
-                                     return fine[fidx(fe, i, j, k)];
-                                   });
-  coarse[t] = scale == 1.0 ? v : v * scale;
-}
-
-__global__ void k_coarse_diag(int nx, int ny, int nz, Coarse64 c,
-                              int* bad) {
-  const int64_t cells = (int64_t)nx * ny * nz;
-  const int64_t t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (t >= cells) return;
-  const int j = static_cast<int>((t / nx) % ny);
-  const int k = static_cast<int>(t / ((int64_t)nx * ny));
-  const int64_t row = j + (int64_t)ny * k;
-  const int64_t fyo = t + (int64_t)nx * k;
-  double d = c.D[t];
-  d += c.fx[t + row] + c.fx[t + row + 1] + c.fy[fyo] + c.fy[fyo + nx] +
-       c.fz[t] + c.fz[t + (int64_t)nx * ny];
-  const double v = c.vol[t];
-  if (v == 0.0) d = 1.0;
-  c.D[t] = d;
-  c.act[t] = v > 0.0 ? 1 : 0;
-  if (v < 0.0 || !isfinite(v) || !(d > 0.0) || !isfinite(d)) atomicOr(bad, 1);
-}
-
-// Certified SDD M-matrix check of one level (src/solver_mg.cpp:1965-2019).
-__global__ void k_validate(int nx, int ny, int nz, const double* D,
-                           const double* fx, const double* fy,
-                           const double* fz, const double* vol, int* bad) {
-  const int64_t cells = (int64_t)nx * ny * nz;
-  const int64_t t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (t >= cells) return;
-  const int j = static_cast<int>((t / nx) % ny);
-  const int k = static_cast<int>(t / ((int64_t)nx * ny));
-  const int64_t row = j + (int64_t)ny * k;
-  const int64_t fyo = t + (int64_t)nx * k;
-  const double faces = fx[t + row] + fx[t + row + 1] + fy[fyo] + fy[fyo + nx] +
-                       fz[t] + fz[t + (int64_t)nx * ny];
-  const double d = D[t];
-  bool fail = !isfinite(d) || !(d > 0.0) || !isfinite(faces) || faces < 0.0;
-  if (vol[t] == 0.0)
-    fail = fail || d != 1.0 || faces != 0.0;
-  else
-    fail = fail || faces > d;
-  if (fail) atomicOr(bad, 2);
-}
-
+// One coarse level: a thread forms its cell's volume and reaction, its six
+// faces (each from the fine faces below it), the diagonal from them, the
+// checks and the storage-precision copies; it stores the low faces, and the
+// high ones at the end of an axis.  scale: the distance correction per axis.
+// ratio: the diagonal shortcut's maximum; at or below `limit` the level is
+// not built.
 template <class T>
-__global__ void k_convert(const double* src, T* dst, int64_t count) {
-  const int64_t t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (t < count) dst[t] = st<T>(src[t]);
+__global__ void k_coarse_level(Agg a, Fine64 f, Coarse64 c, StoredCoeffs<T> s,
+                               RefreshOut out, double scale_x, double scale_y,
+                               double scale_z, const double* ratio,
+                               double limit) {
+  __shared__ double scratch[16];
+  if (ratio != nullptr && *ratio <= limit) return;
+  const int nx = a.cn[0], ny = a.cn[1], nz = a.cn[2], plane = nx * ny;
+  const int lb = xcd_block32(blockIdx.x, gridDim.x);
+  const int t = lb * kBlock + static_cast<int>(threadIdx.x);
+  double vol = 0.0;
+  if (t >= 0 && t < plane * nz) {
+    const int ck = t / plane;
+    const int r = t - ck * plane;
+    const int cj = r / nx;
+    const int ci = r - cj * nx;
+    const int* fn = a.fn;
+    const int fe[3][3] = {{fn[0] + 1, fn[1], fn[2]},
+                          {fn[0], fn[1] + 1, fn[2]},
+                          {fn[0], fn[1], fn[2] + 1}};
+    const double* fine[3] = {f.fx, f.fy, f.fz};
+    vol = aggregate_entry(a, -1, ci, cj, ck, [&](int i, int j, int k) {
+      return f.vol[fidx(fn, i, j, k)];
+    });
+    double d = aggregate_entry(a, -1, ci, cj, ck, [&](int i, int j, int k) {
+      const int64_t cc = fidx(fn, i, j, k);
+      if (f.vol[cc] == 0.0) return 0.0;
+      const double faces =
+          f.fx[fidx(fe[0], i, j, k)] + f.fx[fidx(fe[0], i + 1, j, k)] +
+          f.fy[fidx(fe[1], i, j, k)] + f.fy[fidx(fe[1], i, j + 1, k)] +
+          f.fz[fidx(fe[2], i, j, k)] + f.fz[fidx(fe[2], i, j, k + 1)];
+      const double reaction = f.D[cc] - faces;
+      return reaction > 0.0 ? reaction : 0.0;
+    });
+    const int co[3] = {ci, cj, ck};
+    const int at[3] = {t + cj + ny * ck, t + nx * ck, t};
+    const int step[3] = {1, nx, plane};
+    const double scale[3] = {scale_x, scale_y, scale_z};
+    double* coarse[3] = {c.fx, c.fy, c.fz};
+    T* copies[3] = {s.fx, s.fy, s.fz};
+    double faces = 0.0;
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        int e[3] = {ci, cj, ck};
+        e[ax] += side;
+        double v = aggregate_entry(a, ax, e[0], e[1], e[2],
+                                   [&](int i, int j, int k) {
+                                     return fine[ax][fidx(fe[ax], i, j, k)];
+                                   });
+        v = scale[ax] == 1.0 ? v : v * scale[ax];
+        faces = ax == 0 && side == 0 ? v : faces + v;
+        if (side == 0 || co[ax] + 1 == a.cn[ax]) {
+          const int face = at[ax] + side * step[ax];
+          coarse[ax][face] = v;
+          if (copies[ax] != nullptr) copies[ax][face] = st<T>(v);
+        }
+      }
+    }
+    d += faces;
+    if (vol == 0.0) d = 1.0;
+    c.D[t] = d;
+    if (s.D != nullptr) s.D[t] = st<T>(d);
+    c.vol[t] = vol;
+    c.act[t] = vol > 0.0 ? 1 : 0;
+    if (vol < 0.0 || !isfinite(vol) || !(d > 0.0) || !isfinite(d))
+      atomicOr(out.bad, 1);
+    if (row_invalid(d, faces, vol)) atomicOr(out.bad, 2);
+  }
+  vol = block_sum(vol, scratch);
+  if (threadIdx.x == 0) out.volume[lb] = vol;
+}
+
+// *out = the largest of `count` block maxima (one block).
+__global__ void __launch_bounds__(1024)
+k_refresh_ratio(const double* ratio, int count, double* out) {
+  __shared__ double scratch[16];
+  double m = 0.0;
+  for (int b = threadIdx.x; b < count; b += blockDim.x) m = fmax(m, ratio[b]);
+  m = block_max(m, scratch);
+  if (threadIdx.x == 0) *out = m;
+}
+
+// Block l: the fluid volume of level l from its block sums, which lie one
+// level after the other; block 0 also turns the check flags into a scalar.
+struct RefreshLevels {
+  int first[33];  // first block sum of a level; the last entry ends them
+};
+
+__global__ void __launch_bounds__(1024)
+k_refresh_finish(const double* volume, RefreshLevels levels, const int* bad,
+                 double* volumes, double* flag) {
+  __shared__ double scratch[16];
+  const int l = blockIdx.x;
+  double v = 0.0;
+  for (int b = levels.first[l] + static_cast<int>(threadIdx.x);
+       b < levels.first[l + 1]; b += blockDim.x)
+    v += volume[b];
+  v = block_sum(v, scratch);
+  if (threadIdx.x != 0) return;
+  volumes[l] = v;
+  if (l == 0) *flag = static_cast<double>(*bad);
 }
 
 // ---------------------------------------------------------------------------
@@ -467,23 +560,6 @@ namespace hf {
 // it.  The solvers take it where a plain sum of squares overflowed, so a
 // norm overflows only where the reference's does.  A non-finite element
 // makes its block's maximum +inf.
-__device__ __forceinline__ double block_max(double v, double* scratch) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-#pragma unroll
-  for (int offset = kWave / 2; offset > 0; offset >>= 1)
-    v = fmax(v, __shfl_down(v, offset, kWave));
-  if (lane == 0) scratch[wave] = v;
-  __syncthreads();
-  double m = 0.0;
-  if (threadIdx.x == 0) {
-    const int waves = (blockDim.x + kWave - 1) / kWave;
-    for (int w = 0; w < waves; ++w) m = fmax(m, scratch[w]);
-  }
-  __syncthreads();
-  return m;
-}
-
 __global__ void k_absmax(Chunk ch, const double* v, double* partials) {
   __shared__ double scratch[16];
   const int lb = xcd_block32(blockIdx.x, gridDim.x);

@@ -298,7 +298,6 @@ struct hf_plan {
   bool has_activity = false;
   // the published hierarchy applies z = D^-1 r (diagonal shortcut)
   bool shortcut = false;
-  unsigned long long* d_ratio = nullptr;  // shortcut selection maximum
   // FGMRES basis and reduction buffers (allocated by the first solve)
   int fg_capacity = 0;
   double* fg_v = nullptr;        // restart + 1 basis vectors
@@ -311,6 +310,10 @@ struct hf_plan {
   uint8_t* fxa = nullptr;
   uint8_t* fya = nullptr;
   uint8_t* fza = nullptr;
+  uint8_t* spare_fxa = nullptr;  // a refresh writes these, then swaps
+  uint8_t* spare_fya = nullptr;
+  uint8_t* spare_fza = nullptr;
+  double* refresh_sums = nullptr;  // block sums and maxima of a refresh
   Chunk chunk0{};  // 1-D chunking of level-0 vectors
   // reductions
   double* partials = nullptr;
@@ -2497,7 +2500,11 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
   guard(dalloc(p, &p->folded, 3 * kFoldStride));
   guard(dalloc(p, &p->scalars, S_COUNT));
   guard(dalloc(p, &p->d_flag, 4));
-  guard(dalloc(p, &p->d_ratio, 1));
+  {
+    int64_t sums = blocks_for(p->cells);
+    for (const Level& L : p->levels) sums += blocks_for(L.cells);
+    guard(dalloc(p, &p->refresh_sums, sums));
+  }
   guard(dalloc(p, &p->kx, p->cells));
   guard(dalloc(p, &p->kr, p->cells));
   guard(dalloc(p, &p->kp, p->cells));
@@ -2553,11 +2560,8 @@ hf_status hf_assemble_coefficients(hf_plan* p, const double* mobility,
     return fail(HF_INVALID_PLAN, kDetailPlan);
   const AxisGeom g = axis_geom(p);
   const Level& L = p->levels[0];
-  double* out[3] = {bx, by, bz};
-  const int64_t counts[3] = {L.nfx, L.nfy, L.nfz};
-  for (int a = 0; a < 3; ++a)
-    HF_LAUNCH(k_assemble_faces, blocks_for(counts[a]), kBlock, 0, p->stream, g,
-              a, mobility, out[a], counts[a]);
+  HF_LAUNCH(k_assemble_faces, blocks_for(L.cells), kBlock, 0, p->stream, g,
+            mobility, bx, by, bz);
   HF_LAUNCH(k_face_sum_diag, blocks_for(L.cells), kBlock, 0, p->stream,
             p->n[0], p->n[1], p->n[2], bx, by, bz, diag);
   return hip_check(hipGetLastError());
@@ -2601,12 +2605,6 @@ hf_status hf_assemble_pressure_system(
   s.rhs = rhs;
   // the preflight checks everything before anything is written
   HF_TRY(hip_check(hipMemsetAsync(p->d_flag, 0, sizeof(int), p->stream)));
-  const double* beta[3] = {bx, by, bz};
-  const double* phi[3] = {phi_x, phi_y, phi_z};
-  const int64_t counts[3] = {L.nfx, L.nfy, L.nfz};
-  for (int a = 0; a < 3; ++a)
-    HF_LAUNCH(k_check_faces, blocks_for(counts[a]), kBlock, 0, p->stream,
-              beta[a], phi[a], counts[a], p->d_flag);
   HF_LAUNCH(k_pressure_system, blocks_for(L.cells), kBlock, 0, p->stream, s, 0,
             p->d_flag);
   int flag = 0;
@@ -2698,63 +2696,73 @@ hf_status hf_plan_set_coefficients(hf_plan* p, const double* diag,
   }
   Level& L0 = p->levels[0];
   Coeffs& K0 = *target[0];
-  // level 0: masking
-  HF_LAUNCH(k_mask_faces, blocks_for(L0.nfx), kBlock, 0, p->stream, bx, fxa, K0.fx64, L0.nfx);
-  HF_LAUNCH(k_mask_faces, blocks_for(L0.nfy), kBlock, 0, p->stream, by, fya, K0.fy64, L0.nfy);
-  HF_LAUNCH(k_mask_faces, blocks_for(L0.nfz), kBlock, 0, p->stream, bz, fza, K0.fz64, L0.nfz);
+  uint8_t** masks[3] = {&p->fxa, &p->fya, &p->fza};
+  uint8_t** spare_masks[3] = {&p->spare_fxa, &p->spare_fya, &p->spare_fza};
+  const int64_t face_count[3] = {L0.nfx, L0.nfy, L0.nfz};
+  for (int a = 0; a < 3 && all; ++a)
+    if (*spare_masks[a] == nullptr)
+      HF_TRY(dalloc(p, spare_masks[a], face_count[a]));
+  // block sums of the levels' volumes, one level after the other, then level
+  // 0's block maxima of the row ratio
+  RefreshLevels at{};
+  for (size_t l = 0; l < p->levels.size(); ++l)
+    at.first[l + 1] =
+        at.first[l] + static_cast<int>(blocks_for(p->levels[l].cells));
+  const bool may_shortcut = p->policy.diagonal_shortcut_ratio != 0.0 &&
+                            !p->policy.null_space_constant;
+  double* const sums = p->refresh_sums;
+  double* const maxima = sums + at.first[p->levels.size()];
+  double* const ratio = p->scalars + S_SUM2;
+  {
+    const Chunk one = make_chunk(1);
+    HF_LAUNCH(k_fill, 1, kBlock, 0, p->stream, one,
+              reinterpret_cast<double*>(p->d_flag), 0.0);
+  }
+  const auto copies = [](const Level& L, const Coeffs& K, auto t) {
+    using T = decltype(t);
+    StoredCoeffs<T> s{};
+    if (L.prec != HF_PRECISION_FP64) {
+      s.D = static_cast<T*>(K.DT);
+      s.fx = static_cast<T*>(K.fxT);
+      s.fy = static_cast<T*>(K.fyT);
+      s.fz = static_cast<T*>(K.fzT);
+    }
+    return s;
+  };
+  // level 0
   Finest f{};
   f.nx = p->n[0];
   f.ny = p->n[1];
   f.nz = p->n[2];
   f.D = diag;
-  f.bx = bx;
-  f.by = by;
-  f.bz = bz;
   f.ca = ca;
-  f.fxa = fxa;
-  f.fya = fya;
-  f.fza = fza;
-  f.wx = p->d_widths[0];
-  f.wy = p->d_widths[1];
-  f.wz = p->d_widths[2];
   f.oD = K0.D64;
-  f.ofx = K0.fx64;
-  f.ofy = K0.fy64;
-  f.ofz = K0.fz64;
   f.vol = K0.vol;
   f.act = K0.act;
-  HF_LAUNCH(k_mask_cells, blocks_for(L0.cells), kBlock, 0, p->stream, f);
-  HF_TRY(hip_check(hipMemsetAsync(p->d_flag, 0, sizeof(int), p->stream)));
-  // diagonal shortcut (src/solver_mg.cpp:4545-4575): the finest level is
-  // validated first, then its largest row ratio decides; a shortcut plan
-  // never builds or reads the coarse hierarchy
-  bool shortcut = false;
-  if (p->policy.diagonal_shortcut_ratio != 0.0 &&
-      !p->policy.null_space_constant) {
-    HF_LAUNCH(k_validate, blocks_for(L0.cells), kBlock, 0, p->stream, L0.n[0],
-              L0.n[1], L0.n[2], K0.D64, K0.fx64, K0.fy64, K0.fz64, K0.vol,
-              p->d_flag);
-    HF_TRY(hip_check(hipMemsetAsync(p->d_ratio, 0, sizeof(unsigned long long),
-                                    p->stream)));
-    HF_LAUNCH(k_row_ratio_max,
-              std::min<int64_t>(blocks_for(L0.cells), kRatioBlocks), kBlock, 0,
-              p->stream, L0.n[0], L0.n[1], L0.n[2], K0.D64, K0.fx64, K0.fy64,
-              K0.fz64, p->d_ratio);
-    int flag0 = 0;
-    unsigned long long bits = 0;
-    HF_TRY(hip_check(hipMemcpyAsync(&flag0, p->d_flag, sizeof(int),
-                                    hipMemcpyDeviceToHost, p->stream)));
-    HF_TRY(hip_check(hipMemcpyAsync(&bits, p->d_ratio, sizeof bits,
-                                    hipMemcpyDeviceToHost, p->stream)));
-    HF_TRY(hip_check(hipStreamSynchronize(p->stream)));
-    if (flag0 != 0) return fail(HF_NUMERICAL_FAILURE, kDetailCoefficients);
-    double ratio = 0.0;
-    std::memcpy(&ratio, &bits, sizeof ratio);
-    shortcut = ratio <= p->policy.diagonal_shortcut_ratio;
+  const double* raw[3] = {bx, by, bz};
+  const uint8_t* open[3] = {fxa, fya, fza};
+  double* masked[3] = {K0.fx64, K0.fy64, K0.fz64};
+  for (int a = 0; a < 3; ++a) {
+    f.b[a] = raw[a];
+    f.fa[a] = open[a];
+    f.w[a] = p->d_widths[a];
+    f.of[a] = masked[a];
+    f.ofa[a] = *spare_masks[a];
   }
-  const size_t built = shortcut ? 1 : p->levels.size();
+  RefreshOut out{sums, may_shortcut ? maxima : nullptr, p->d_flag};
+  dispatch(L0.prec, [&](auto t) {
+    HF_LAUNCH((k_mask_level<decltype(t)>), blocks_for(L0.cells), kBlock, 0,
+              p->stream, f, copies(L0, K0, t), out);
+  });
+  // diagonal shortcut (src/solver_mg.cpp:4545-4575): the finest level's
+  // largest row ratio decides; a shortcut plan never builds or reads the
+  // coarse hierarchy
+  if (may_shortcut)
+    HF_LAUNCH(k_refresh_ratio, 1, 1024, 0, p->stream,
+              static_cast<const double*>(maxima), at.first[1], ratio);
   // coarse levels
-  for (size_t l = 1; l < built; ++l) {
+  out.ratio = nullptr;
+  for (size_t l = 1; l < p->levels.size(); ++l) {
     const Level& F = p->levels[l - 1];
     const Level& C = p->levels[l];
     const Coeffs& KF = *target[l - 1];
@@ -2767,66 +2775,40 @@ hf_status hf_plan_set_coefficients(hf_plan* p, const double* diag,
     a.mask = F.coarsen_mask;
     Fine64 fine{KF.D64, KF.fx64, KF.fy64, KF.fz64, KF.vol};
     Coarse64 coarse{KC.D64, KC.fx64, KC.fy64, KC.fz64, KC.vol, KC.act};
-    HF_LAUNCH(k_coarse_cells, blocks_for(C.cells), kBlock, 0, p->stream, a, fine, coarse);
     // distance-corrected aggregation halves faces whose normal was coarsened
     const bool dc = p->policy.coarse_face_scaling != 0;
-    const double sx = dc && (F.coarsen_mask & 1) ? 0.5 : 1.0;
-    const double sy = dc && (F.coarsen_mask & 2) ? 0.5 : 1.0;
-    const double sz = dc && (F.coarsen_mask & 4) ? 0.5 : 1.0;
-    HF_LAUNCH(k_coarse_faces, blocks_for(C.nfx), kBlock, 0, p->stream, a, 0, KF.fx64, KC.fx64, sx);
-    HF_LAUNCH(k_coarse_faces, blocks_for(C.nfy), kBlock, 0, p->stream, a, 1, KF.fy64, KC.fy64, sy);
-    HF_LAUNCH(k_coarse_faces, blocks_for(C.nfz), kBlock, 0, p->stream, a, 2, KF.fz64, KC.fz64, sz);
-    HF_LAUNCH(k_coarse_diag, blocks_for(C.cells), kBlock, 0, p->stream, C.n[0], C.n[1], C.n[2], coarse, p->d_flag);
-  }
-  for (size_t l = 0; l < built; ++l) {
-    const Level& L = p->levels[l];
-    const Coeffs& K = *target[l];
-    HF_LAUNCH(k_validate, blocks_for(L.cells), kBlock, 0, p->stream, L.n[0], L.n[1], L.n[2], K.D64, K.fx64, K.fy64, K.fz64, K.vol, p->d_flag);
-  }
-  // storage-precision copies
-  for (size_t l = 0; l < built; ++l) {
-    const Level& L = p->levels[l];
-    const Coeffs& K = *target[l];
-    if (L.prec == HF_PRECISION_FP64) continue;
-    dispatch(L.prec, [&](auto t) {
-      using T = decltype(t);
-      HF_LAUNCH(k_convert<T>, blocks_for(L.cells), kBlock, 0, p->stream, K.D64, static_cast<T*>(K.DT), L.cells);
-      HF_LAUNCH(k_convert<T>, blocks_for(L.nfx), kBlock, 0, p->stream, K.fx64, static_cast<T*>(K.fxT), L.nfx);
-      HF_LAUNCH(k_convert<T>, blocks_for(L.nfy), kBlock, 0, p->stream, K.fy64, static_cast<T*>(K.fyT), L.nfy);
-      HF_LAUNCH(k_convert<T>, blocks_for(L.nfz), kBlock, 0, p->stream, K.fz64, static_cast<T*>(K.fzT), L.nfz);
+    auto scale = [&](int axis) {
+      return dc && (F.coarsen_mask & axis) ? 0.5 : 1.0;
+    };
+    out.volume = sums + at.first[l];
+    dispatch(C.prec, [&](auto t) {
+      HF_LAUNCH((k_coarse_level<decltype(t)>), blocks_for(C.cells), kBlock, 0,
+                p->stream, a, fine, coarse, copies(C, KC, t), out, scale(1),
+                scale(2), scale(4),
+                may_shortcut ? static_cast<const double*>(ratio) : nullptr,
+                p->policy.diagonal_shortcut_ratio);
     });
   }
-  // projection volumes (sum of fluid volumes per level)
-  for (size_t l = 0; l < built; ++l) {
-    const Level& L = p->levels[l];
-    Coeffs& K = *target[l];
-    const Chunk ch = make_chunk(static_cast<int>(L.cells));
-    const int nb = chunk_blocks(ch);
-    HF_LAUNCH(k_sum, nb, kBlock, 0, p->stream, ch, K.vol,
-              static_cast<const uint8_t*>(nullptr), p->partials);
-    finalize(p, nb, 1, F_STORE, S_SUM);
-    HF_TRY(read_scalars(p));
-    K.volume = p->host_scalars[S_SUM];
-  }
-  int flag = 0;
-  HF_TRY(hip_check(hipMemcpyAsync(&flag, p->d_flag, sizeof(int), hipMemcpyDeviceToHost, p->stream)));
-  HF_TRY(hip_check(hipStreamSynchronize(p->stream)));
+  // volumes (through the idle mean slots), check flags and the ratio come
+  // back in one read
+  HF_LAUNCH(k_refresh_finish, p->levels.size(), 1024, 0, p->stream,
+            static_cast<const double*>(sums), at,
+            static_cast<const int*>(p->d_flag), p->scalars + S_MEAN0,
+            p->scalars + S_SUM);
   HF_TRY(hip_check(hipGetLastError()));
-  if (flag != 0) return fail(HF_NUMERICAL_FAILURE, kDetailCoefficients);
-  if (p->policy.null_space_constant && !(target[0]->volume > 0.0))
+  HF_TRY(read_scalars(p));
+  const bool shortcut =
+      may_shortcut &&
+      p->host_scalars[S_SUM2] <= p->policy.diagonal_shortcut_ratio;
+  if (p->host_scalars[S_SUM] != 0.0)
     return fail(HF_NUMERICAL_FAILURE, kDetailCoefficients);
-  // every check passed: keep the raw activity masks for the adjoint, then
-  // publish
-  if (all) {
-    if (p->fxa == nullptr) {
-      HF_TRY(dalloc(p, &p->fxa, L0.nfx));
-      HF_TRY(dalloc(p, &p->fya, L0.nfy));
-      HF_TRY(dalloc(p, &p->fza, L0.nfz));
-    }
-    HF_TRY(hip_check(hipMemcpyAsync(p->fxa, fxa, L0.nfx, hipMemcpyDeviceToDevice, p->stream)));
-    HF_TRY(hip_check(hipMemcpyAsync(p->fya, fya, L0.nfy, hipMemcpyDeviceToDevice, p->stream)));
-    HF_TRY(hip_check(hipMemcpyAsync(p->fza, fza, L0.nfz, hipMemcpyDeviceToDevice, p->stream)));
-  }
+  if (p->policy.null_space_constant && !(p->host_scalars[S_MEAN0] > 0.0))
+    return fail(HF_NUMERICAL_FAILURE, kDetailCoefficients);
+  const size_t built = shortcut ? 1 : p->levels.size();
+  for (size_t l = 0; l < built; ++l)
+    target[l]->volume = p->host_scalars[S_MEAN0 + l];
+  // every check passed: publish
+  for (int a = 0; a < 3 && all; ++a) std::swap(*masks[a], *spare_masks[a]);
   p->has_activity = all;
   p->shortcut = shortcut;
   if (into_spare)

@@ -161,3 +161,40 @@ def test_pcg_mid_loop_breakdown_matches_oracle(torch_cuda, seed):
     # a failed solve publishes nothing
     assert torch.count_nonzero(x).item() == 0
     plan.close()
+
+
+@pytest.mark.parametrize("n", [(2, 3, 2), (17, 5, 3), (16, 4, 4),
+                               (33, 8, 31)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_refresh_reaches_every_entry(torch_cuda, n, masked):
+    """The refresh checks, masks and stores each face once, the ends of every
+    axis and a last, partly filled block included: an invalid first or last
+    entry of any array is refused, and without masks the finest level is the
+    input itself."""
+    import hundun_flow as H
+    torch = torch_cuda
+    _say(f"[refresh entries] n={n} masked={masked}")
+    case = hf_cases.lognormal_sphere(n=n, seed=5)
+    plan = H.Plan(case["n"], case["faces"], case["bc"],
+                  H.default_policy(minimum_coarse_extent=2,
+                                   anisotropy_threshold=64.0))
+    d, bx, by, bz = O.assemble(case["n"], case["faces"], case["bc"],
+                               case["mobility"])
+    d = d + 1.0  # no row is the sum of its faces alone
+    coeffs = [_t(torch, v) for v in (d, bx, by, bz)]
+    masks = [torch.ones(v.numel(), dtype=torch.uint8, device="cuda")
+             for v in coeffs] if masked else []
+    plan.set_coefficients(*coeffs, *masks)
+    for which in range(1, 4):
+        assert torch.equal(plan.level_array(0, which).flatten(),
+                           coeffs[which])
+    if not masked:
+        assert torch.equal(plan.level_array(0, 0).flatten(), coeffs[0])
+    for array in range(4):
+        for entry in (0, -1):
+            bad = [c.clone() for c in coeffs]
+            bad[array][entry] = float("nan")
+            with pytest.raises(H.HundunFlowError) as err:
+                plan.set_coefficients(*bad, *masks)
+            assert err.value.code == 5  # numerical_failure
+    plan.close()
