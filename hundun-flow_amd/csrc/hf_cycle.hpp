@@ -383,24 +383,6 @@ __global__ void k_rb(Tiles t, Lv<T> L, Bc bc, int color) {
   L.x[c] = st<T>(xc + omega * (C(ld(L.b[c])) - v) / C(ld(L.D[c])));
 }
 
-// Separated route for levels with an odd periodic extent
-// (src/solver_mg.cpp:3262-3307): the colour update uses the A x computed
-// before the pass.
-template <class T>
-__global__ void k_rb_separated(Tiles t, Lv<T> L, int color) {
-  using C = typename Compute<T>::type;
-  int ic, j, k;
-  tile_xyz(t, xcd_block32(blockIdx.x, gridDim.x), ic, j, k);
-  if (ic >= t.nx || j >= t.ny) return;
-  const int i = 2 * ic + ((color + j + k) & 1);
-  if (i >= L.nx) return;
-  const int c = cell_index(L.nx, L.ny, i, j, k);
-  const C omega = C(0.72);
-  L.x[c] = st<T>(C(ld(L.x[c])) +
-                 omega * (C(ld(L.b[c])) - C(ld(L.r[c]))) / C(ld(L.D[c])));
-}
-
-
 // Restriction (src/solver_mg.cpp:3633-3720): coarse b = sum of children in
 // dz, dy, dx order, coarse x := 0 (skipped when the next smoothing starts
 // from zero by itself).  With a constant null space the block partials of
@@ -477,7 +459,7 @@ __device__ __forceinline__ int wrapi(int v, int extent) {
 }
 
 // Retained defect fused with the restriction that consumes it
-// (src/solver_mg.cpp:3633-3720).  The z-marching layout of k_stencil_z with
+// (src/solver_mg.cpp:3633-3720).  The z-marching layout of k_residual_z with
 // full tiles of even width and height and even z-chunks, on a level with
 // even extents coarsened along every axis: each step's defects, stored and
 // reloaded at the fine storage type, go through LDS to the thread owning the
@@ -900,25 +882,20 @@ __global__ void k_mg_proj3(Tiles t, const double* rin, const uint8_t* act,
 }
 
 // ---------------------------------------------------------------------------
-// z-marching stencil kernels.  A block owns one 2-D tile of the plane (the
+// The true residual r = 1 b + (-1) A x and the partial sum of r.r
+// (axpby(r, 1, b, -1, Ax): src/solver_krylov.cpp:1082-1091); bb_at > 0: also
+// the partial sum of b.b, bb_at partials after those of r.r.  A z-marching
+// stencil kernel: a block owns one 2-D tile of the plane (the
 // Tiles layout with k = 0) and t.per consecutive planes of it; each thread
 // walks its cell column upwards, carrying x at k-1 and k and the z-face
 // coefficient between steps, so a step loads x and the coefficients of one
 // new plane and the in-plane neighbours (cache hits from the tile's rows).
-// Operand values and the order of operations are those of stencil():
-//   kZOpDot    q = A p and the partial sum of p.q (Krylov operator)
-//   kZResidual r = 1 b + (-1) A x and the partial sum of r.r (the true
-//              residual, axpby(r, 1, b, -1, Ax): src/solver_krylov.cpp:
-//              1082-1091); aux > 0: also the partial sum of b.b, aux
-//              partials after those of r.r
-//   kZApply    r = b - A x (aux != 0, defect) or r = A x at level storage
+// Operand values and the order of operations are those of stencil().
 // ---------------------------------------------------------------------------
-constexpr int kZOpDot = 0, kZResidual = 1, kZApply = 2;
-
-template <class T, int kMode>
-__global__ void k_stencil_z(Tiles t, Lv<T> L, Bc bc, const T* x, const T* b,
-                            T* out, double* partials, int aux) {
-  using C = typename Compute<T>::type;
+__global__ void k_residual_z(Tiles t, Lv<double> L, Bc bc, const double* x,
+                             const double* b, double* out, double* partials,
+                             int bb_at) {
+  using C = double;
   __shared__ double scratch[16];
   const int lb = xcd_block32(blockIdx.x, gridDim.x);
   const int gxy = t.gx * t.gy;
@@ -966,35 +943,26 @@ __global__ void k_stencil_z(Tiles t, Lv<T> L, Bc bc, const T* x, const T* b,
       v -= C(ld(L.fy[fyo + nx])) * yh;
       v -= fzl * zl;
       v -= fzh * zh;
-      if constexpr (kMode == kZOpDot) {
-        out[c] = v;
-        d += xc * v;
-      } else if constexpr (kMode == kZResidual) {
-        const double bv = b[c];
-        const double rc = 1.0 * bv + -1.0 * v;
-        out[c] = rc;
-        d += rc * rc;
-        bb += bv * bv;
-      } else {
-        out[c] = aux ? st<T>(C(ld(b[c])) - v) : st<T>(v);
-      }
+      const double bv = b[c];
+      const double rc = 1.0 * bv + -1.0 * v;
+      out[c] = rc;
+      d += rc * rc;
+      bb += bv * bv;
       zl = xc;
       xc = zh;
       fzl = fzh;
       c += plane;
     }
   }
-  if (kMode != kZApply && partials != nullptr) {
-    d = block_sum(d, scratch);
-    if (threadIdx.x == 0) partials[lb] = d;
-    if (kMode == kZResidual && aux > 0) {
-      bb = block_sum(bb, scratch);
-      if (threadIdx.x == 0) partials[lb + aux] = bb;
-    }
+  d = block_sum(d, scratch);
+  if (threadIdx.x == 0) partials[lb] = d;
+  if (bb_at > 0) {
+    bb = block_sum(bb, scratch);
+    if (threadIdx.x == 0) partials[lb + bb_at] = bb;
   }
 }
 
-// The true residual of k_stencil_z<double, kZResidual> (same operands and
+// The true residual of k_residual_z (same operands and
 // order) fused with the preconditioner's entry of k_mg_entry, which the
 // restart after an unconverged check runs on that residual: b_mg = fluid ?
 // r : 0 at the level-0 storage precision.  Accumulators `stride` apart:

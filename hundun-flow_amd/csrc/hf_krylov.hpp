@@ -24,7 +24,7 @@ __device__ __forceinline__ double geom_volume(const Widths& w, int i, int j,
 //   d = rf (b - A x) / D            (first stage)
 //   d = pf d + rf (b - A x) / D     (later stages)
 //   x_next = x + d.
-// z-marching as k_stencil_z; x and x_next are distinct buffers.
+// z-marching as k_residual_z; x and x_next are distinct buffers.
 // ---------------------------------------------------------------------------
 template <class T>
 __global__ void k_cheb_stage(Tiles t, Lv<T> L, Bc bc, const T* x, T* xn,
@@ -263,7 +263,7 @@ enum FgMode : int { kFgArnoldi = 0, kFgResidual = 1, kFgOpDot = 2 };
 
 // Level-0 FP64 action y = A' x, A' = A or A divided by the geometric cell
 // volume (the per-volume rows of the cold system), z-marching as
-// k_stencil_z, with the FGMRES epilogues:
+// k_residual_z, with the FGMRES epilogues:
 //  kFgArnoldi:  out = A' x - shift * aux (aux = v_col); accumulator a < kNd
 //               holds basis_a . out, accumulator wacc holds out . out;
 //  kFgResidual: out = 1 b + (-1) A' x (b = aux); accumulator 0 = out . out
@@ -404,8 +404,9 @@ __global__ void k_fg_dots(Tiles t, const double* wv, const double* basis,
 // cell's operator value is formed as in k_fg_stencil; a thread adds its two
 // cells' products to its accumulators in cell order.  t tiles (nx / 2) x ny
 // columns in z-chunks; partials as in k_fg_stencil, one per block of t.
-// kFgOpDot (the PCG operator, k_stencil_z<double, kZOpDot> over pairs):
-// out = A' x and accumulator wacc holds x . out; aux is not read.
+// kFgOpDot (the PCG operator; k_rows makes it on other rows):
+// out = A' x and accumulator wacc holds x . out (partials may be null); aux
+// is not read.
 template <int kMode, int kNd>
 __global__ void k_fg_stencil2(Tiles t, Lv<double> A, Bc bc, const double* x,
                               const double* aux, double* out,
@@ -552,6 +553,7 @@ __global__ void k_fg_stencil2(Tiles t, Lv<double> A, Bc bc, const double* x,
       if (threadIdx.x == 0) partials[a * pstride + lb] = s;
     }
   }
+  if (kMode == kFgOpDot && partials == nullptr) return;
   const double s = block_sum(ww, scratch);
   if (threadIdx.x == 0) partials[wacc * pstride + lb] = s;
 }

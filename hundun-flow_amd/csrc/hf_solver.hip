@@ -22,6 +22,7 @@
 #include "hf_leg.hpp"
 #include "hf_line.hpp"
 #include "hf_march.hpp"
+#include "hf_rows.hpp"
 #include "hf_tail.hpp"
 #include "hundun_flow.h"
 
@@ -873,13 +874,41 @@ Widths widths(const hf_plan* p) {
   return Widths{p->d_widths[0], p->d_widths[1], p->d_widths[2]};
 }
 
-// r = b - A x (defect) or r = A x on level l, z-marching.
+// One k_rows pass over a level; returns its blocks.  Two planes per block
+// share the rows of x between them; with one plane per block a level that
+// stays in the last-level cache is faster (A x in FP64, 1 and 2 planes:
+// 201x149x97 22.3 and 25.3 us, 192x192x128 33.9 and 37.5, 300x180x140 77 and
+// 74, 511x255x255 376 and 347).
+template <class T, int kMode>
+int64_t rows_pass(hf_plan* p, const Lv<T>& v, const T* x, T* out,
+                  double* partials, int colour) {
+  RowsArgs<T> a;
+  a.L = v;
+  a.bc = p->bc;
+  a.x = x;
+  a.out = out;
+  a.partials = partials;
+  a.colour = colour;
+  a.pairs = (v.nx + 1) / 2;
+  a.per_plane = static_cast<int>(
+      blocks_for(static_cast<int64_t>(a.pairs) * v.ny));
+  const bool cached = static_cast<int64_t>(v.cells) * sizeof(T) < (48ll << 20);
+  const int64_t blocks =
+      static_cast<int64_t>(a.per_plane) * (cached || v.nx == 1 ? v.nz : (v.nz + 1) / 2);
+  if (v.nx == 1)
+    HF_LAUNCH((k_rows<T, kMode, 1, true>), blocks, kBlock, 0, p->stream, a);
+  else if (cached)
+    HF_LAUNCH((k_rows<T, kMode, 1, false>), blocks, kBlock, 0, p->stream, a);
+  else
+    HF_LAUNCH((k_rows<T, kMode, 2, false>), blocks, kBlock, 0, p->stream, a);
+  return blocks;
+}
+
+// The retained defect r = b - A x of a level.
 template <class T>
-void level_apply(hf_plan* p, const Level& L, const Lv<T>& v, int defect) {
-  HF_LAUNCH((k_stencil_z<T, kZApply>), L.tz.blocks, kBlock, 0, p->stream,
-            L.tz, v, p->bc, static_cast<const T*>(v.x),
-            static_cast<const T*>(v.b), v.r, static_cast<double*>(nullptr),
-            defect);
+void level_defect(hf_plan* p, const Lv<T>& v) {
+  HF_PROF(p, P_DEFECT);
+  rows_pass<T, kRowsDefect>(p, v, v.x, v.r, nullptr, 0);
 }
 
 // Mean of a level field for the constant projection: scalars[S_MEAN0 + l].
@@ -986,10 +1015,7 @@ void sweep_smooth(hf_plan* p, int l, int sweeps, int reverse, int retain,
     std::swap(L.x, L.x2);
     if (a.bout != nullptr) std::swap(L.b, L.b2);
   }
-  if (retain) {
-    HF_PROF(p, P_DEFECT);
-    level_apply<T>(p, L, view<T>(L), 1);
-  }
+  if (retain) level_defect<T>(p, view<T>(L));
 }
 
 template <class T>
@@ -1117,10 +1143,7 @@ void cheb_smooth(hf_plan* p, int l, int stages, int retain, int from_zero) {
     }
     std::swap(L.x, L.x2);
   }
-  if (retain) {
-    HF_PROF(p, P_DEFECT);
-    level_apply<T>(p, L, view<T>(L), 1);
-  }
+  if (retain) level_defect<T>(p, view<T>(L));
 }
 
 template <class T>
@@ -1135,10 +1158,7 @@ void grid_smooth(hf_plan* p, int l, int sweeps, int reverse, int retain,
     // x starts from an explicit zero on line levels; the retained defect is
     // recomputed after line smoothing (compute_residual, :4256-4262)
     line_smooth<T>(p, l, sweeps, reverse);
-    if (retain) {
-      HF_PROF(p, P_DEFECT);
-      level_apply<T>(p, L, view<T>(L), 1);
-    }
+    if (retain) level_defect<T>(p, view<T>(L));
     return;
   }
   point_smooth<T>(p, l, sweeps, reverse, retain, from_zero, mean_partials);
@@ -1150,52 +1170,40 @@ void point_smooth(hf_plan* p, int l, int sweeps, int reverse, int retain,
   Level& L = p->levels[l];
   if (L.march && sweeps == 2) {
     march_smooth<T>(p, l, reverse, from_zero, mean_partials);
-    if (retain) {
-      HF_PROF(p, P_DEFECT);
-      level_apply<T>(p, L, view<T>(L), 1);
-    }
+    if (retain) level_defect<T>(p, view<T>(L));
     return;
   }
   if (L.sweep) {
     sweep_smooth<T>(p, l, sweeps, reverse, retain, from_zero, mean_partials);
     return;
   }
-  const Lv<T> v = view<T>(L);
   const int rb_class = l == 0 ? P_RB_FINEST : P_RB_COARSE;
   // a pending constant projection of b is folded into the first pass
   const double* mean = (from_zero && p->policy.null_space_constant)
                            ? p->scalars + S_MEAN0 + l
                            : nullptr;
-  if (!L.fused && !from_zero) {
-    HF_PROF(p, P_DEFECT);
-    level_apply<T>(p, L, v, 0);
-  }
   for (int sweep = 0; sweep < sweeps; ++sweep) {
     const int first = reverse ? 1 : 0;
     for (int pass = 0; pass < 2; ++pass) {
       const int color = (first + pass) & 1;
       const bool zero_pass = from_zero && sweep == 0 && pass == 0;
-      {
-        HF_PROF(p, zero_pass ? P_RB_FIRST : rb_class);
-        if (zero_pass)
-          HF_LAUNCH(k_rb_first<T>, L.tc.blocks, kBlock, 0, p->stream, L.tc, v,
-                    mean);
-        else if (L.fused)
-          HF_LAUNCH(k_rb<T>, L.tcol.blocks, kBlock, 0, p->stream, L.tcol, v,
-                    p->bc, color);
-        else
-          HF_LAUNCH(k_rb_separated<T>, L.tcol.blocks, kBlock, 0, p->stream,
-                    L.tcol, v, color);
-      }
-      const bool final_update = sweep + 1 == sweeps && pass == 1;
-      if (!final_update || retain) {
-        if (!L.fused || (final_update && retain)) {
-          HF_PROF(p, P_DEFECT);
-          level_apply<T>(p, L, v, (retain && final_update) ? 1 : 0);
-        }
+      HF_PROF(p, zero_pass ? P_RB_FIRST : rb_class);
+      const Lv<T> v = view<T>(L);
+      if (zero_pass) {
+        HF_LAUNCH(k_rb_first<T>, L.tc.blocks, kBlock, 0, p->stream, L.tc, v,
+                  mean);
+      } else if (L.fused) {
+        HF_LAUNCH(k_rb<T>, L.tcol.blocks, kBlock, 0, p->stream, L.tcol, v,
+                  p->bc, color);
+      } else {
+        // (the pass reads x from before it everywhere)
+        rows_pass<T, kRowsColour>(p, v, v.x, static_cast<T*>(L.x2), nullptr,
+                                  color);
+        std::swap(L.x, L.x2);
       }
     }
   }
+  if (retain) level_defect<T>(p, view<T>(L));
 }
 
 // A level that needs the projected b and x = 0 in memory before a cycle
@@ -1517,10 +1525,7 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
         project_apply<T>(p, 0, x);
         mean = nullptr;
       }
-      {
-        HF_PROF(p, P_DEFECT);
-        level_apply<T>(p, L0, view<T>(L0), 1);
-      }
+      level_defect<T>(p, view<T>(L0));
       {
         HF_PROF(p, P_MG_ENTRY_EXIT);
         HF_LAUNCH(k_mg_proj3<T>, L0.tred.blocks, kBlock, 0, p->stream, L0.tred, r,
@@ -2472,7 +2477,7 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
     if (L.sweep || L.march) {
       guard(dalloc_raw(p, &L.x2, es * L.cells));
       guard(dalloc_raw(p, &L.b2, es * L.cells));
-    } else if (L.cheb || L.leg) {
+    } else if (L.cheb || L.leg || (!L.fused && !L.tail)) {
       guard(dalloc_raw(p, &L.x2, es * L.cells));
     }
     if (L.line_mask != 0) {
@@ -2819,13 +2824,29 @@ hf_status hf_plan_set_coefficients(hf_plan* p, const double* diag,
   return hip_check(hipGetLastError());
 }
 
+// y = A x on level 0 with the block sums of x . y at `partials` (null: not
+// taken); returns their number.  Rows of whole 64-pair tiles on a level that
+// streams from memory run as pairs in tiles (k_fg_stencil2; 166 us against
+// 176 at 256^3, 318 against 338 at 512x256x256), the others as k_rows
+// (256x256x128 81 us against 83, 400x160x240 158 against 168).
+static int64_t operator_pass(hf_plan* p, const double* x, double* y,
+                             double* partials) {
+  const Level& L = p->levels[0];
+  if (!p->krylov_pairs || L.n[0] % 128 != 0 || L.cells < (int64_t{12} << 20))
+    return rows_pass<double, kRowsOperator>(p, krylov_view(p), x, y, partials,
+                                            0);
+  HF_LAUNCH((k_fg_stencil2<kFgOpDot, 0>), L.tzp.blocks, kBlock, 0, p->stream,
+            L.tzp, krylov_view(p), p->bc, x,
+            static_cast<const double*>(nullptr), y,
+            static_cast<const double*>(nullptr), int64_t{0}, 0, 0.0, 0,
+            widths(p), partials, int64_t{0});
+  return L.tzp.blocks;
+}
+
 hf_status hf_operator_apply(hf_plan* p, const double* x, double* y) {
   if (p == nullptr || x == nullptr || y == nullptr || !p->coefficients_ready)
     return fail(HF_INVALID_PLAN, kDetailPlan);
-  const Tiles& t = p->levels[0].tz;
-  HF_LAUNCH((k_stencil_z<double, kZOpDot>), t.blocks, kBlock, 0, p->stream, t,
-            krylov_view(p), p->bc, x, static_cast<const double*>(nullptr), y,
-            static_cast<double*>(nullptr), 0);
+  operator_pass(p, x, y, nullptr);
   return hip_check(hipGetLastError());
 }
 
@@ -2843,9 +2864,6 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
                           const hf_solve_control* ctl, hf_solve_result* res) {
   const Lv<double> A = krylov_view(p);
   const Tiles& tr = p->levels[0].tz;  // z-marching Krylov stencils
-  // the operator over pairs of cells of a row on rows of even length
-  const bool op_pairs = p->krylov_pairs && p->levels[0].n[0] % 2 == 0;
-  const Tiles& L0p = p->levels[0].tzp;
   // the PCG update stores the preconditioner's entry when level 0 is a grid
   // level (the tail and line-relaxed entries also zero x; a Chebyshev level 0
   // reads no x in its first stage, and mg_apply projects its b)
@@ -2874,8 +2892,7 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
   auto true_residual = [&](bool with_bb) -> hf_status {
     HF_PROF(p, P_TRUE_RESIDUAL);
     if (!fuse_entry) {
-      HF_LAUNCH((k_stencil_z<double, kZResidual>), tr.blocks, kBlock, 0,
-                p->stream, tr, A, p->bc, static_cast<const double*>(x), rhs,
+      HF_LAUNCH(k_residual_z, tr.blocks, kBlock, 0, p->stream, tr, A, p->bc, static_cast<const double*>(x), rhs,
                 r, p->partials, with_bb ? 2 * stride : 0);
       return ok();
     }
@@ -2970,22 +2987,13 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
       return finish(fail(HF_NUMERICAL_FAILURE, kDetailBreakdown),
                     HF_TERM_BREAKDOWN);
     };
-    if (op_pairs) {
-      // q = A p over pairs of cells of a row (p.q rounds in another order)
+    int64_t op_blocks = 0;
+    {
       HF_PROF(p, P_OPERATOR);
-      HF_LAUNCH((k_fg_stencil2<kFgOpDot, 0>), L0p.blocks, kBlock, 0,
-                p->stream, L0p, A, p->bc, static_cast<const double*>(pp),
-                static_cast<const double*>(nullptr), q,
-                static_cast<const double*>(nullptr), int64_t{0}, 0, 0.0, 0,
-                widths(p), p->partials, int64_t{0});
-    } else {
-      HF_PROF(p, P_OPERATOR);
-      HF_LAUNCH((k_stencil_z<double, kZOpDot>), tr.blocks, kBlock, 0,
-                p->stream, tr, A, p->bc, static_cast<const double*>(pp),
-                static_cast<const double*>(nullptr), q, p->partials, 0);
+      op_blocks = operator_pass(p, pp, q, p->partials);
     }
     res->operator_applies++;
-    finalize(p, op_pairs ? L0p.blocks : tr.blocks, 1, F_ALPHA, 0);
+    finalize(p, op_blocks, 1, F_ALPHA, 0);
     // an iteration that verifies on schedule replaces r with the true
     // residual, so its update forms x alone and its step checks wait for the
     // true residual's read

@@ -847,3 +847,38 @@ def test_pcg_row_pair_operator(torch_cuda, monkeypatch, name, precision):
     assert out["1"][2] == "converged" and out["0"][2] == "converged"
     assert out["1"][1] == out["0"][1]
     assert rel <= 1e-12, rel
+
+
+@pytest.mark.parametrize("n,bc", [
+    ((1, 40, 33), (1, 1, 0, 1, 2, 2)),       # rows of one cell
+    ((2, 37, 21), (2, 2, 2, 2, 0, 0)),       # one pair, y odd and periodic
+    ((3, 5, 7), (2, 2, 2, 2, 2, 2)),         # every axis odd and periodic
+    ((33, 21, 9), (0, 1, 2, 2, 1, 0)),       # last pairs of one cell
+    ((35, 8, 12), (2, 2, 1, 0, 0, 1)),       # the seam along the row
+    ((181, 191, 193), (1, 1, 0, 1, 2, 2)),   # two planes per block
+])
+def test_row_passes_bitwise(torch_cuda, monkeypatch, n, bc):
+    """The operator, the retained defect and the colour passes of levels with
+    an odd periodic extent over rows of any length (k_rows): FP64 equal to the
+    oracle, FP32 and BF16 to the same passes made in LDS, bit for bit."""
+    torch = torch_cuda
+    _say(f"[rows] n={n} bc={bc}")
+    monkeypatch.setenv("HF_TAIL_CELLS", "0")
+    case = march_case(n, bc, seed=37)
+    pol = dict(null_space_constant=0, anisotropy_threshold=4096.0)
+    _, mg = O.from_case(case, O.policy(**pol))
+    rng = np.random.default_rng(41)
+    r = rng.standard_normal(n[0] * n[1] * n[2])
+    zo = mg.apply(r)
+    for precision in ("fp64", "fp32", "bf16"):
+        z = {}
+        for cells in ("0", "32768"):
+            monkeypatch.setenv("HF_LEG_CELLS", cells)
+            plan = _gpu_plan(torch, case, precision=precision, **pol)
+            z[cells] = plan.mg_apply(_t(torch, r)).cpu().numpy()
+            y = plan.operator_apply(_t(torch, r)).cpu().numpy()
+            plan.close()
+            assert np.array_equal(y, mg.masked_apply(r)), precision
+            if precision == "fp64":
+                assert np.array_equal(z[cells], zo), cells
+        assert np.array_equal(z["32768"], z["0"]), precision
