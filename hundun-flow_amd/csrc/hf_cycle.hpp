@@ -232,16 +232,34 @@ __global__ void k_vol_dot(Tiles t, const T* field, const double* vol,
 // storage type.  Partial sums: r.r in accumulator 0 and, with the constant
 // null space, vol*b in accumulator 1 (stride apart).  Tiles of the reduction
 // layout (kRedPer per block).  x == nullptr: x is left for the direction
-// update (k_update_p_exit), which reads p anyway.
+// update (k_update_p_exit), which reads p anyway.  alpha.count > 0: p.q is
+// still the operator's block sums; every block folds them (F_ALPHA).
+struct AlphaRef {
+  double* scalars;
+  const double* partials;  // p.q
+  int count;
+  int rho;  // slot of r.z
+};
+
 template <class T>
 __global__ void k_update_xr_entry(Tiles t, double* x, const double* pv,
                                   double* r, const double* q,
-                                  const double* alpha, const uint8_t* act,
+                                  AlphaRef alpha, const uint8_t* act,
                                   Widths w, T* b, double* partials,
                                   int stride, int proj) {
   __shared__ double scratch[16];
   const int lb = xcd_block32(blockIdx.x, gridDim.x);
-  const double a = *alpha;
+  double a;
+  if (alpha.count > 0) {
+    const double pap = fold_sum<kBlock>(alpha.partials, alpha.count, scratch);
+    a = alpha.scalars[alpha.rho] / pap;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      alpha.scalars[S_PAP] = pap;
+      alpha.scalars[S_ALPHA] = a;
+    }
+  } else {
+    a = alpha.scalars[S_ALPHA];
+  }
   const bool with_x = x != nullptr;
   // two groups of four tiles: each group's loads are issued together (eight
   // tiles of five FP64 operands would not fit the register file)
@@ -755,13 +773,12 @@ __global__ void k_prolong_z2(Tiles t, Lv<Tc> Cl, Lv<Tf> F, int mask, int per) {
 // products r.z (and z.q for the flexible beta).
 template <class T>
 __global__ void k_mg_exit(Tiles t, const T* x, const uint8_t* act,
-                          const double* mean, const double* alpha, double* z,
+                          MeanRef mean, const double* alpha, double* z,
                           const double* r, const double* q, double* partials,
                           int stride) {
   __shared__ double scratch[16];
   const int lb = xcd_block32(blockIdx.x, gridDim.x);
   const double a = alpha == nullptr ? 1.0 : *alpha;
-  const double m = mean == nullptr ? 0.0 : *mean;
   T xs[kRedPer];
   double rv[kRedPer], qv[kRedPer];
   bool ok[kRedPer], fluid[kRedPer];
@@ -775,6 +792,7 @@ __global__ void k_mg_exit(Tiles t, const T* x, const uint8_t* act,
     rv[u] = r != nullptr ? r[cc[u]] : 0.0;
     qv[u] = q != nullptr ? q[cc[u]] : 0.0;
   }
+  const double m = mean_value<kBlock>(mean, scratch);
   double rz = 0.0, zq = 0.0;
 #pragma unroll
   for (int u = 0; u < kRedPer; ++u) {
@@ -782,7 +800,7 @@ __global__ void k_mg_exit(Tiles t, const T* x, const uint8_t* act,
     double v = 0.0;
     if (fluid[u]) {
       double xv = static_cast<double>(ld(xs[u]));
-      if (mean != nullptr) xv = static_cast<double>(ld(st<T>(xv - m)));
+      if (mean.at != nullptr) xv = static_cast<double>(ld(st<T>(xv - m)));
       v = xv * a;
     }
     if (z != nullptr) z[cc[u]] = v;
@@ -805,16 +823,26 @@ __global__ void k_mg_exit(Tiles t, const T* x, const uint8_t* act,
 // so the exit need not store z.  With sol: first the iteration's solution
 // update sol += step p (add_scaled, src/solver_krylov.cpp:383-399) with the
 // p it replaces, which k_update_xr_entry left out.  Tiles of the reduction
-// layout.
+// layout.  beta.count > 0: r.z (and z.q for the flexible beta) are still the
+// exit's block sums; every block folds them (F_BETA_FR, F_BETA_PR).
+struct BetaRef {
+  double* scalars;
+  const double* partials;  // r.z; z.q a stride further
+  int count;
+  int stride;
+  int rho;       // slot of r.z of the iteration before; the new one goes to
+  int flexible;  // the other rho slot
+};
+
 template <class T>
 __global__ void k_update_p_exit(Tiles t, const T* x, const uint8_t* act,
                                 const double* mean, const double* alpha,
-                                double* p, const double* beta, double* sol,
+                                double* p, BetaRef beta, double* sol,
                                 const double* step) {
+  __shared__ double scratch[16];
   const int lb = xcd_block32(blockIdx.x, gridDim.x);
   const double a = alpha == nullptr ? 1.0 : *alpha;
   const double m = mean == nullptr ? 0.0 : *mean;
-  const double be = *beta;
   const double sa = sol != nullptr ? *step : 0.0;
   T xs[kRedPer];
   double pv[kRedPer], sv[kRedPer];
@@ -828,6 +856,25 @@ __global__ void k_update_p_exit(Tiles t, const T* x, const uint8_t* act,
     xs[u] = x[cc[u]];
     pv[u] = p[cc[u]];
     sv[u] = sol != nullptr ? sol[cc[u]] : 0.0;
+  }
+  double be;
+  if (beta.count > 0) {
+    const double rz = fold_sum<kBlock>(beta.partials, beta.count, scratch);
+    const double rho = beta.scalars[beta.rho];
+    double zq = 0.0;
+    if (beta.flexible) {
+      zq = fold_sum<kBlock>(beta.partials + beta.stride, beta.count, scratch);
+      be = -beta.scalars[S_ALPHA] * zq / rho;
+    } else {
+      be = rz / rho;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      beta.scalars[other_rho(beta.rho)] = rz;
+      beta.scalars[S_ZQ] = zq;
+      beta.scalars[S_BETA] = be;
+    }
+  } else {
+    be = beta.scalars[S_BETA];
   }
 #pragma unroll
   for (int u = 0; u < kRedPer; ++u) {

@@ -222,4 +222,92 @@ __device__ __forceinline__ double block_sum(double v, double* scratch) {
   return total;
 }
 
+// Device scalars of the solvers.
+enum ScalarSlot : int {
+  S_RHO = 0,
+  S_PAP = 1,
+  S_ALPHA = 2,
+  S_RNORM2 = 3,
+  S_BETA = 4,
+  S_RHONEXT = 5,
+  S_ZQ = 6,
+  S_MEAN0 = 7,  // 7..7+kMaxLevels: projection means per level
+  S_PROJ0 = 48, // three dots of the residual-minimising scaling
+  S_PROJ1 = 49,
+  S_PROJ2 = 50,
+  S_MGALPHA = 51,
+  S_SUM = 52,
+  S_SUM2 = 53,
+  S_LINE_FAIL = 54,  // nonzero after a line relaxation pivot vanished
+  S_NSCALE = 55,     // scaled norm: largest magnitude
+  S_NSUM = 56,       // scaled norm: sum of scaled squares
+  S_COUNT = 64
+};
+
+// r.z lies in one of two slots: a new one is stored beside the one that the
+// same kernel divides by.
+__host__ __device__ constexpr int other_rho(int slot) {
+  return S_RHO + S_RHONEXT - slot;
+}
+
+// Sum of `count` partials (up to a few thousand) in the order of k_finalize's
+// 1024 threads, made by every thread of a block of kThreads; the result is
+// valid in all of them.  `scratch` holds 16 doubles of LDS.
+template <int kThreads>
+__device__ __forceinline__ double fold_sum(const double* partials, int count,
+                                           double* scratch) {
+  constexpr int kWaves = kThreads / kWave;
+  constexpr int kEach = (16 + kWaves - 1) / kWaves;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  double v[kEach];
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) v[e] = 0.0;
+  for (int base = 0; base < count; base += 16 * kWave) {
+    double q[kEach];
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) {
+      const int g = wave + e * kWaves;
+      const int b = base + g * kWave + lane;
+      q[e] = g < 16 && b < count ? partials[b] : 0.0;
+    }
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) v[e] += q[e];
+  }
+#pragma unroll
+  for (int e = 0; e < kEach; ++e) {
+    const int g = wave + e * kWaves;
+    const double s = wave_sum(v[e]);
+    if (lane == 0 && g < 16) scratch[g] = s;
+  }
+  __syncthreads();
+  double total = 0.0;
+#pragma unroll
+  for (int g = 0; g < 16; ++g) total += scratch[g];
+  __syncthreads();
+  return total;
+}
+
+// A mean that a kernel takes: the scalar at `at` (null: none is pending), or,
+// with count > 0, still the block sums of the kernel before it, divided by
+// `over`: then every block folds them and the first one stores the mean at
+// `at` for later kernels.  A launch of one block to fold them costs 3.5 us
+// and a gap; the fold in the consumer about 1 us.
+struct MeanRef {
+  double* at;
+  const double* partials;
+  int count;
+  double over;
+};
+
+template <int kThreads>
+__device__ __forceinline__ double mean_value(const MeanRef& m,
+                                             double* scratch) {
+  if (m.at == nullptr) return 0.0;
+  if (m.count == 0) return *m.at;
+  const double mean = fold_sum<kThreads>(m.partials, m.count, scratch) / m.over;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *m.at = mean;
+  return mean;
+}
+
 }  // namespace hf

@@ -446,36 +446,16 @@ k_refresh_finish(const double* volume, RefreshLevels levels, const int* bad,
 // block finaliser that also performs the scalar Krylov algebra on device so
 // the host only reads back what it must test.
 // ---------------------------------------------------------------------------
-enum ScalarSlot : int {
-  S_RHO = 0,
-  S_PAP = 1,
-  S_ALPHA = 2,
-  S_RNORM2 = 3,
-  S_BETA = 4,
-  S_RHONEXT = 5,
-  S_ZQ = 6,
-  S_MEAN0 = 7,  // 7..7+kMaxLevels: projection means per level
-  S_PROJ0 = 48, // three dots of the residual-minimising scaling
-  S_PROJ1 = 49,
-  S_PROJ2 = 50,
-  S_MGALPHA = 51,
-  S_SUM = 52,
-  S_SUM2 = 53,
-  S_LINE_FAIL = 54,  // nonzero after a line relaxation pivot vanished
-  S_NSCALE = 55,     // scaled norm: largest magnitude
-  S_NSUM = 56,       // scaled norm: sum of scaled squares
-  S_COUNT = 64
-};
-
 enum FinalOp : int {
   F_STORE = 0,     // scalars[a] = sum0
-  F_ALPHA = 1,     // pap = sum0, alpha = rho / pap
+  F_ALPHA = 1,     // pap = sum0, alpha = rho / pap (rho: scalars[slot])
   F_RHO = 2,       // rho = sum0
-  F_BETA_FR = 3,   // beta = sum0/rho, rho = sum0
-  F_BETA_PR = 4,   // rho_next = sum0, zq = sum1, beta = -alpha*zq/rho
+  F_BETA_FR = 3,   // beta = sum0/rho, the other rho = sum0
+  F_BETA_PR = 4,   // zq = sum1, beta = -alpha*zq/rho, the other rho = sum0
   F_MEAN = 5,      // scalars[a] = sum0 / volume
   F_MGALPHA = 6,   // three sums -> residual-minimising alpha
-  F_STORE2 = 7     // scalars[a] = sum0, scalars[a+1] = sum1
+  F_STORE2 = 7,    // scalars[a] = sum0, scalars[a+1] = sum1
+  F_STORE_MEAN = 8 // scalars[a] = sum0, scalars[S_MEAN0] = sum1 / volume
 };
 
 // First fold of many block partials: block (s, a) sums span s of
@@ -516,21 +496,23 @@ k_finalize(const double* partials, int64_t blocks, int64_t stride, int nacc,
       break;
     case F_ALPHA:
       scalars[S_PAP] = sums[0];
-      scalars[S_ALPHA] = scalars[S_RHO] / sums[0];
+      scalars[S_ALPHA] = scalars[slot] / sums[0];
       break;
     case F_RHO:
-      scalars[S_RHO] = sums[0];
+      scalars[slot] = sums[0];
       break;
     case F_BETA_FR:
-      scalars[S_RHONEXT] = sums[0];
-      scalars[S_BETA] = sums[0] / scalars[S_RHO];
-      scalars[S_RHO] = sums[0];
+      scalars[other_rho(slot)] = sums[0];
+      scalars[S_BETA] = sums[0] / scalars[slot];
       break;
     case F_BETA_PR:
-      scalars[S_RHONEXT] = sums[0];
+      scalars[other_rho(slot)] = sums[0];
       scalars[S_ZQ] = sums[1];
-      scalars[S_BETA] = -scalars[S_ALPHA] * sums[1] / scalars[S_RHO];
-      scalars[S_RHO] = sums[0];
+      scalars[S_BETA] = -scalars[S_ALPHA] * sums[1] / scalars[slot];
+      break;
+    case F_STORE_MEAN:
+      scalars[slot] = sums[0];
+      scalars[S_MEAN0] = sums[1] / volume;
       break;
     case F_MEAN:
       scalars[slot] = sums[0] / volume;

@@ -58,7 +58,7 @@ struct LegArgs {
   Lv<Tc> Cl;
   Bc bc;
   T* xout;             // not F.x when F.x is read
-  const double* mean;  // pending constant projection of b, else null
+  MeanRef mean;        // pending constant projection of b (at: null, none)
   int passes;          // colour passes, or Chebyshev stages
   int first;           // colour of the first pass
   int from_zero;       // way down: x starts from zero
@@ -121,7 +121,6 @@ __global__ void __launch_bounds__(kLegThreads) k_leg(LegArgs<T, Tc> a) {
   // cells' parity: periodic extents are even), so that a pass works on one
   // slot; else slot q is cell q.
   const int flip = kMode == kLegRb ? (gi + gj + gk) & 1 : 0;
-  const double mean = a.mean != nullptr ? *a.mean : 0.0;
 
   // Way up: the column's corners in a coarse plane and their x, y weights.
   // The coarse cells that the region interpolates from (at most 8 along an
@@ -173,8 +172,9 @@ __global__ void __launch_bounds__(kLegThreads) k_leg(LegArgs<T, Tc> a) {
 
   // ---- load the pair's coefficients, b and x
   C d[2], b[2], f[2][6];
+  T braw[2];
   int at[2], ozl[2], ozh[2], colour[2];
-  bool valid[2];
+  bool valid[2], fluid_b[2];
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     const int z = q ^ flip;
@@ -198,13 +198,8 @@ __global__ void __launch_bounds__(kLegThreads) k_leg(LegArgs<T, Tc> a) {
     f[q][3] = s.yh;
     f[q][4] = s.zl;
     f[q][5] = s.zh;
-    const T braw = L.b[c];
-    if (a.mean != nullptr) {
-      const T projected = st<T>(static_cast<double>(ld(braw)) - mean);
-      b[q] = L.act[c] ? C(ld(projected)) : C(0);
-    } else {
-      b[q] = C(ld(braw));
-    }
+    braw[q] = L.b[c];
+    fluid_b[q] = a.mean.at != nullptr && L.act[c] != 0;
     C x = C(0);
     if (!kDown || !a.from_zero) x = C(ld(L.x[c]));
     if constexpr (!kDown) {
@@ -243,6 +238,16 @@ __global__ void __launch_bounds__(kLegThreads) k_leg(LegArgs<T, Tc> a) {
       x = fluid ? sw_round<T>(x + value) : C(0);
     }
     xs[at[q]] = in ? x : C(0);
+  }
+  const double mean = mean_value<kLegThreads>(a.mean, scratch);
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    if (a.mean.at != nullptr) {
+      const T projected = st<T>(static_cast<double>(ld(braw[q])) - mean);
+      b[q] = fluid_b[q] ? C(ld(projected)) : C(0);
+    } else {
+      b[q] = C(ld(braw[q]));
+    }
   }
   __syncthreads();
 

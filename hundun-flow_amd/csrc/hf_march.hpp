@@ -66,7 +66,7 @@ struct MarchArgs {
   Bc bc;
   T* xout;
   T* bout;             // projected b (kZero with mean), else null
-  const double* mean;  // pending projection mean (kZero), else null
+  MeanRef mean;        // pending projection mean (kZero; at: null, none)
   int first;           // colour updated first: 0 forward, 1 reverse
   int zc;              // planes per chunk
   int gx, gy;          // tiles along x and y
@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(kMaThreads<T>) k_rb_march(MarchArgs<T> a) {
   const uint32_t ofx = static_cast<uint32_t>(wj * (nx + 1) + wi) * kS;
   const bool mine = ok && m >= 2 && m < 30 && row >= kMaHalo &&
                     row < kRows - kMaHalo && gi < nx && gj < ny;
-  const double mean = a.mean != nullptr ? *a.mean : 0.0;
+  const double mean = kZero ? mean_value<kMaThreads<T>>(a.mean, red) : 0.0;
   const C omega = C(0.72);
 
   // the plane in memory of plane k: wrapped, or (not used then) the nearest
@@ -199,7 +199,7 @@ __global__ void __launch_bounds__(kMaThreads<T>) k_rb_march(MarchArgs<T> a) {
     nyl = sw_load2<T>(rfy, oc, sy);
     nyh = sw_load2<T>(rfy, oc, sy + nx * kS);
     nzh = sw_load2<T>(rfz, oc, sc + nxy * kS);
-    if ((kZero && a.mean != nullptr) || kMean)
+    if ((kZero && a.mean.at != nullptr) || kMean)
       nact = *reinterpret_cast<const uint16_t*>(L.act + (sc + oc) / kS);
     if constexpr (!kZero)
       nx2 = sw_load2<T>(rx, oc, static_cast<uint32_t>(wx) * nxy * kS);
@@ -236,7 +236,7 @@ __global__ void __launch_bounds__(kMaThreads<T>) k_rb_march(MarchArgs<T> a) {
     fx[U][2] = C(ld(nf2));
     if (kZero || kMean) act[U] = nact;
     MaPair<C> bk;
-    if (kZero && a.mean != nullptr) {
+    if (kZero && a.mean.at != nullptr) {
       const T lo = st<T>(static_cast<double>(ld(nb.lo)) - mean);
       const T hi = st<T>(static_cast<double>(ld(nb.hi)) - mean);
       bk.v[0] = (nact & 0xffu) ? C(ld(lo)) : C(0);

@@ -319,6 +319,9 @@ struct hf_plan {
   // reductions
   double* partials = nullptr;
   int64_t partial_stride = 0;
+  // a level mean whose block sums the level's next kernel folds (-1: none)
+  int pending_level = -1;
+  MeanRef pending{};
   double* folded = nullptr;
   double* scalars = nullptr;
   double* host_scalars = nullptr;  // pinned
@@ -801,6 +804,7 @@ void build_exec(hf_plan* p) {
 // ---- reductions -----------------------------------------------------------
 // acc0: index of the first accumulator read (partials of accumulator a sit
 // at p->partials + a * partial_stride).
+// (partials that a later kernel folds by itself: MeanRef)
 void finalize(hf_plan* p, int64_t blocks, int nacc, int op, int slot,
               double volume = 0.0, int unit_linear = 1, int acc0 = 0) {
   HF_PROF(p, P_FINALIZE);
@@ -822,6 +826,58 @@ void finalize(hf_plan* p, int64_t blocks, int nacc, int op, int slot,
   HF_LAUNCH(k_finalize, 1, 1024, 0, p->stream, src, count, stride, nacc,
             p->scalars, op, slot, volume, unit_linear);
   ++p->reductions;
+}
+
+// Block sums that a consumer may fold: with more, a launch of one block for
+// the fold is cheaper than one in every block of the consumer.
+constexpr int64_t kFoldInConsumer = 1024;
+
+// The accumulator of a level's mean on the way down: the kernel that makes
+// level l + 1's sums may fold its own level's in the same launch, so
+// neighbouring levels use two.
+double* mean_partials_of(hf_plan* p, int l) {
+  return p->partials + (l & 1 ? 2 * p->partial_stride : 0);
+}
+
+// The sums of level l's mean (over `volume`) lie in `partials`, made by
+// `blocks` blocks: left to the level's next kernel where that folds them
+// (by_consumer), else folded now.
+void leave_mean(hf_plan* p, int l, double* partials, int64_t blocks,
+                bool by_consumer) {
+  if (by_consumer && blocks <= kFoldInConsumer) {
+    p->pending_level = l;
+    p->pending = {p->scalars + S_MEAN0 + l, partials,
+                  static_cast<int>(blocks), p->levels[l].volume};
+    ++p->reductions;
+    return;
+  }
+  finalize(p, blocks, 1, F_MEAN, S_MEAN0 + l, p->levels[l].volume, 1,
+           static_cast<int>((partials - p->partials) / p->partial_stride));
+}
+
+// The mean of level l for a kernel that folds pending sums (MeanRef).
+MeanRef take_mean(hf_plan* p, int l) {
+  MeanRef m{p->scalars + S_MEAN0 + l, nullptr, 0, 0.0};
+  if (p->pending_level == l) m = p->pending;
+  p->pending_level = -1;
+  return m;
+}
+
+// Folds pending sums by a launch of their own.
+void flush_mean(hf_plan* p) {
+  if (p->pending_level < 0) return;
+  --p->reductions;
+  leave_mean(p, p->pending_level, const_cast<double*>(p->pending.partials),
+             p->pending.count, false);
+  p->pending_level = -1;
+}
+
+// Whether level l's next smoothing from zero folds pending sums: a leg, the
+// tail, a march.
+bool folds_mean(const hf_plan* p, int l) {
+  const Level& L = p->levels[l];
+  if (L.leg || L.tail) return true;
+  return L.march && p->policy.pre_sweeps == 2;
 }
 
 // Copies the scalar block to the host.  A line relaxation failure since the
@@ -945,10 +1001,9 @@ void march_smooth(hf_plan* p, int l, int reverse, int from_zero,
   a.L = view<T>(L);
   a.bc = p->bc;
   a.xout = static_cast<T*>(L.x2);
-  a.mean = from_zero && p->policy.null_space_constant
-               ? p->scalars + S_MEAN0 + l
-               : nullptr;
-  a.bout = a.mean != nullptr ? static_cast<T*>(L.b2) : nullptr;
+  a.mean = from_zero && p->policy.null_space_constant ? take_mean(p, l)
+                                                      : MeanRef{};
+  a.bout = a.mean.at != nullptr ? static_cast<T*>(L.b2) : nullptr;
   a.first = reverse ? 1 : 0;
   a.zc = L.march_zc;
   a.gx = (L.n[0] + kMaOutX - 1) / kMaOutX;
@@ -1245,8 +1300,8 @@ void exec_leg(hf_plan* p, const CycleOp& op, bool down,
         a.bc = p->bc;
         a.xout = static_cast<Tf*>(L.x2);
         a.mean = proj && !(op.level == 0 && entry_projects(p))
-                     ? p->scalars + S_MEAN0 + op.level
-                     : nullptr;
+                     ? take_mean(p, op.level)
+                     : MeanRef{};
         a.passes = smoothing_passes(L, op.sweeps);
         a.first = op.reverse ? 1 : 0;
         a.from_zero = op.from_zero;
@@ -1255,7 +1310,9 @@ void exec_leg(hf_plan* p, const CycleOp& op, bool down,
         a.o = box.o;
         a.gx = box.g[0];
         a.gy = box.g[1];
-        a.partials = down ? (proj ? p->partials : nullptr) : mean_partials;
+        a.partials = !down  ? mean_partials
+                     : proj ? mean_partials_of(p, op.level + 1)
+                            : nullptr;
         ChebStage factors(p->policy.chebyshev_lower_fraction);
         for (int s = 0; L.cheb && s < a.passes; ++s) {
           double rf = 0.0, pf = 0.0;
@@ -1283,7 +1340,8 @@ void exec_leg(hf_plan* p, const CycleOp& op, bool down,
           launch(std::integral_constant<int, kLegSeparated>{});
       }
       if (down && proj) {
-        finalize(p, box.blocks, 1, F_MEAN, S_MEAN0 + op.level + 1, Cd.volume);
+        leave_mean(p, op.level + 1, mean_partials_of(p, op.level + 1),
+                   box.blocks, folds_mean(p, op.level + 1));
         if (wants_stored_start(Cd))
           project_apply<Tc>(p, op.level + 1, static_cast<Tc*>(Cd.b));
       }
@@ -1296,6 +1354,10 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
                   double* mean_partials = nullptr,
                   bool defect_restrict = false) {
   Level& L = p->levels[op.level];
+  // (only a march from zero folds a pending mean here)
+  if (p->pending_level == op.level &&
+      !(op.kind == T_SMOOTH && L.march && op.from_zero && op.sweeps == 2))
+    flush_mean(p);
   if (op.kind == T_SMOOTH) {
     // a one-stage Chebyshev smoothing from zero before the fused defect and
     // restriction: that kernel forms the stage's x from b and D itself.
@@ -1332,7 +1394,7 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
           HF_LAUNCH((k_defect_restrict<Tf, Tc, true>), L.tz.blocks, kBlock, 0,
                     p->stream, L.tz, view<Tf>(L), p->bc, view<Tc>(Cd),
                     stored ? 1 : 0,
-                    proj ? p->partials : static_cast<double*>(nullptr),
+                    proj ? mean_partials_of(p, op.level + 1) : nullptr,
                     static_cast<C>(rf0), static_cast<Tf*>(L.x2));
           std::swap(L.x, L.x2);
         } else {
@@ -1340,11 +1402,11 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
           HF_LAUNCH((k_defect_restrict<Tf, Tc>), L.tz.blocks, kBlock, 0,
                     p->stream, L.tz, view<Tf>(L), p->bc, view<Tc>(Cd),
                     stored ? 1 : 0,
-                    proj ? p->partials : static_cast<double*>(nullptr));
+                    proj ? mean_partials_of(p, op.level + 1) : nullptr);
         }
         if (proj) {
-          finalize(p, L.tz.blocks, 1, F_MEAN, S_MEAN0 + op.level + 1,
-                   Cd.volume);
+          leave_mean(p, op.level + 1, mean_partials_of(p, op.level + 1),
+                     L.tz.blocks, folds_mean(p, op.level + 1));
           if (stored)
             project_apply<Tc>(p, op.level + 1, static_cast<Tc*>(Cd.b));
         }
@@ -1365,11 +1427,11 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
           HF_LAUNCH((k_restrict<Tf, Tc>), Cn.tr.blocks, kBlock, 0, p->stream,
                     Cn.tr, view<Tf>(L), view<Tc>(Cn), L.coarsen_mask,
                     stored ? 1 : 0,
-                    proj ? p->partials : static_cast<double*>(nullptr));
+                    proj ? mean_partials_of(p, op.level + 1) : nullptr);
         }
         if (proj) {
-          finalize(p, Cn.tr.blocks, 1, F_MEAN, S_MEAN0 + op.level + 1,
-                   Cn.volume);
+          leave_mean(p, op.level + 1, mean_partials_of(p, op.level + 1),
+                     Cn.tr.blocks, folds_mean(p, op.level + 1));
           if (stored) project_apply<Tc>(p, op.level + 1, static_cast<Tc*>(Cn.b));
         }
       });
@@ -1432,8 +1494,8 @@ void run_cycle(hf_plan* p, double* mean_partials = nullptr) {
     t.cells0 = static_cast<int>(T.cells);
     t.mean = p->policy.null_space_constant != 0 &&
                      !(p->tail_first == 0 && entry_projects(p))
-                 ? p->scalars + S_MEAN0 + p->tail_first
-                 : nullptr;
+                 ? take_mean(p, p->tail_first)
+                 : MeanRef{};
     t.levels = static_cast<int>(p->tail_geo.size());
     t.work = p->tail_work;
     t.head = p->tail_head;
@@ -1448,9 +1510,9 @@ void run_cycle(hf_plan* p, double* mean_partials = nullptr) {
 }
 
 // z = M r on device arrays; optional fused Krylov dots (r.z, z.q).
-// entered: b of level 0 (and, with the null space, the partial sums of its
-// mean in accumulator 1) were stored by the PCG update (k_update_xr_entry);
-// only when level 0 is a grid level (not the tail, not line relaxed).
+// entered: b of level 0 was stored by the PCG update (k_update_xr_entry), the
+// true residual or the basis combination and, with the null space, its mean
+// formed; only when level 0 is a grid level (not the tail, not line relaxed).
 // The operands from which the exit forms z (level-0 candidate, projection
 // mean, scale), for a consumer that forms z itself (k_update_p_exit).
 struct ExitOperands {
@@ -1463,10 +1525,11 @@ struct ExitOperands {
 // receives the operands z is formed from.
 hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
                    bool dots, bool entered = false,
-                   ExitOperands* exit = nullptr, int64_t entry_blocks = 0) {
+                   ExitOperands* exit = nullptr) {
   Level& L0 = p->levels[0];
   const bool proj = p->policy.null_space_constant != 0;
   const bool tail0 = entry_projects(p);
+  p->pending_level = -1;
   // (a grid Chebyshev level 0 starts with a from-zero stage, which reads
   // b and D only, and the tail and a leg start from zero by themselves: no
   // x = 0 there)
@@ -1485,15 +1548,16 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
                 proj ? p->partials : static_cast<double*>(nullptr));
     }
     if (proj) {
-      // an entry made by the caller leaves its partials in accumulator 1
-      // (entry_blocks of them when not in the reduction layout)
-      finalize(p, entered && entry_blocks > 0 ? entry_blocks : L0.tred.blocks,
-               1, F_MEAN, S_MEAN0, L0.volume, 1, entered ? 1 : 0);
+      if (!entered)
+        leave_mean(p, 0, p->partials, L0.tred.blocks,
+                   !tail0 && folds_mean(p, 0));
       if (tail0) project_apply<T>(p, 0, b);
     }
   });
   // the cycle's last fused sweep also sums the level-0 mean of its output
   const int64_t sweep_mean = proj && !p->shortcut ? mean_blocks(p) : 0;
+  // (the exit may fold these sums while it writes its own)
+  double* const exit_partials = p->partials + 2 * p->partial_stride;
   if (p->shortcut) {
     // z = D^-1 r (src/solver_mg.cpp:4926-4936); the shortcut is only
     // selected without a null space
@@ -1505,25 +1569,26 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
                 view<T>(L0));
     });
   } else {
-    run_cycle(p, sweep_mean > 0 ? p->partials : nullptr);
+    run_cycle(p, sweep_mean > 0 ? exit_partials : nullptr);
   }
   const double* alpha = nullptr;
-  const double* mean = nullptr;
+  MeanRef mean{};
   dispatch(L0.prec, [&](auto t) {
     using T = decltype(t);
     T* x = static_cast<T*>(L0.x);
     if (proj) {
       if (sweep_mean > 0)
-        finalize(p, sweep_mean, 1, F_MEAN, S_MEAN0, L0.volume);
+        leave_mean(p, 0, exit_partials, sweep_mean,
+                   p->policy.unit_linear != 0);
       else
         level_mean<T>(p, 0, x);
-      mean = p->scalars + S_MEAN0;
+      mean = take_mean(p, 0);
     }
     if (!p->policy.unit_linear) {
       // residual-minimising scaling needs the projected candidate stored
       if (proj) {
         project_apply<T>(p, 0, x);
-        mean = nullptr;
+        mean = MeanRef{};
       }
       level_defect<T>(p, view<T>(L0));
       {
@@ -1544,7 +1609,7 @@ hf_status mg_apply(hf_plan* p, const double* r, double* z, const double* q,
               static_cast<int>(p->partial_stride));
     if (exit != nullptr) {
       exit->x = x;
-      exit->mean = mean;
+      exit->mean = mean.at;
       exit->alpha = alpha;
     }
   });
@@ -2907,13 +2972,22 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
     });
     return ok();
   };
+  // the slot of the current r.z
+  int rho_slot = S_RHO;
+  // r.r and, where the pass made the entry, the mean of the projection
+  const bool entry_mean = fuse_entry && p->policy.null_space_constant != 0;
+  auto residual_sums = [&](int64_t blocks) {
+    finalize(p, blocks, entry_mean ? 2 : 1, entry_mean ? F_STORE_MEAN : F_STORE,
+             S_RNORM2, p->levels[0].volume);
+    if (entry_mean) ++p->reductions;
+  };
   // ||b|| and the initial true residual come from one pass and one read; the
   // gates then run in the reference's order (a non-finite ||b||, a zero
   // ||b||, whose residual goes unused, then the residual)
   HF_LAUNCH(k_copy, nbv, kBlock, 0, p->stream, ch, x, solution);
   HF_TRY(true_residual(true));
   finalize(p, tr.blocks, 1, F_STORE, S_SUM, 0.0, 1, 2);
-  finalize(p, tr.blocks, 1, F_STORE, S_RNORM2);
+  residual_sums(tr.blocks);
   HF_TRY(read_scalars(p));
   double bnorm = std::sqrt(p->host_scalars[S_SUM]);
   if (!std::isfinite(bnorm)) {
@@ -2950,15 +3024,15 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
   // p = z = M r: the preconditioner writes z straight into p (nothing else
   // reads this z)
   auto precondition_restart = [&]() -> hf_status {
-    HF_TRY(mg_apply(p, r, pp, nullptr, true, fuse_entry, nullptr, tr.blocks));
+    HF_TRY(mg_apply(p, r, pp, nullptr, true, fuse_entry));
     res->preconditioner_applies++;
-    finalize(p, p->levels[0].tred.blocks, 1, F_RHO, 0);
+    finalize(p, p->levels[0].tred.blocks, 1, F_RHO, rho_slot);
     return ok();
   };
   HF_TRY(precondition_restart());
   HF_TRY(read_scalars(p));
   {
-    const double rho = p->host_scalars[S_RHO];
+    const double rho = p->host_scalars[rho_slot];
     if (!(rho > 0.0) || !std::isfinite(rho))
       return finish(fail(HF_NUMERICAL_FAILURE, kDetailBreakdown), HF_TERM_BREAKDOWN);
   }
@@ -2977,7 +3051,7 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
     auto rho_failed = [&]() -> bool {
       if (!rho_pending) return false;
       rho_pending = false;
-      const double rho = p->host_scalars[S_RHO];
+      const double rho = p->host_scalars[rho_slot];
       if (rho > 0.0 && std::isfinite(rho)) return false;
       res->operator_applies = operator_applies0;
       res->iterations = iterations0;
@@ -2990,16 +3064,24 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
     int64_t op_blocks = 0;
     {
       HF_PROF(p, P_OPERATOR);
-      op_blocks = operator_pass(p, pp, q, p->partials);
+      op_blocks = operator_pass(p, pp, q, p->partials + 2 * stride);
     }
     res->operator_applies++;
-    finalize(p, op_blocks, 1, F_ALPHA, 0);
     // an iteration that verifies on schedule replaces r with the true
     // residual, so its update forms x alone and its step checks wait for the
     // true residual's read
     const bool scheduled =
         (res->iterations + 1) % ctl->true_residual_interval == 0 ||
         res->iterations + 1 == ctl->maximum_iterations;
+    // p.q: folded by the update where that pays
+    AlphaRef step{p->scalars, p->partials + 2 * stride,
+                  static_cast<int>(op_blocks), rho_slot};
+    if (!scheduled && fuse_entry && op_blocks <= kFoldInConsumer) {
+      ++p->reductions;
+    } else {
+      step.count = 0;
+      finalize(p, op_blocks, 1, F_ALPHA, rho_slot, 0.0, 1, 2);
+    }
     if (scheduled) {
       HF_PROF(p, P_UPDATE_XR);
       HF_LAUNCH(k_update_x, nbv, kBlock, 0, p->stream, ch, x,
@@ -3016,7 +3098,7 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
         HF_LAUNCH(k_update_xr_entry<T>, L0.tred.blocks, kBlock, 0, p->stream,
                   L0.tred, static_cast<double*>(nullptr),
                   static_cast<const double*>(nullptr), r,
-                  static_cast<const double*>(q), p->scalars + S_ALPHA,
+                  static_cast<const double*>(q), step,
                   static_cast<const uint8_t*>(L0.act), widths(p),
                   static_cast<T*>(L0.b), p->partials,
                   static_cast<int>(p->partial_stride),
@@ -3028,8 +3110,7 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
                 p->scalars + S_ALPHA, p->partials);
     }
     if (!scheduled)
-      finalize(p, fuse_entry ? p->levels[0].tred.blocks : nbv, 1, F_STORE,
-               S_RNORM2);
+      residual_sums(fuse_entry ? p->levels[0].tred.blocks : nbv);
     res->iterations++;
     // p.Ap and alpha (read with the recursive norm, or with the true one)
     auto step_failure = [&]() -> int {
@@ -3068,7 +3149,7 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
         x_pending = false;
       }
       HF_TRY(true_residual(false));
-      finalize(p, tr.blocks, 1, F_STORE, S_RNORM2);
+      residual_sums(tr.blocks);
       HF_TRY(read_scalars(p));
       if (rho_failed()) return fail_rho();
       // a step that fails these checks stops before the true residual, as
@@ -3103,8 +3184,18 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
                     fuse_entry, &ex));
     res->preconditioner_applies++;
     rho_pending = true;
-    finalize(p, p->levels[0].tred.blocks, ctl->flexible ? 2 : 1,
-             ctl->flexible ? F_BETA_PR : F_BETA_FR, 0);
+    // r.z (and z.q): folded by the direction update where that pays
+    BetaRef beta{p->scalars, p->partials,
+                 static_cast<int>(p->levels[0].tred.blocks), stride, rho_slot,
+                 ctl->flexible ? 1 : 0};
+    if (beta.count <= kFoldInConsumer) {
+      ++p->reductions;
+    } else {
+      beta.count = 0;
+      finalize(p, p->levels[0].tred.blocks, ctl->flexible ? 2 : 1,
+               ctl->flexible ? F_BETA_PR : F_BETA_FR, rho_slot);
+    }
+    rho_slot = other_rho(rho_slot);
     {
       HF_PROF(p, P_UPDATE_P);
       Level& L0 = p->levels[0];
@@ -3113,8 +3204,7 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
         HF_LAUNCH(k_update_p_exit<T>, L0.tred.blocks, kBlock, 0, p->stream,
                   L0.tred, static_cast<const T*>(ex.x),
                   static_cast<const uint8_t*>(L0.act), ex.mean, ex.alpha, pp,
-                  static_cast<const double*>(p->scalars + S_BETA),
-                  x_pending ? x : static_cast<double*>(nullptr),
+                  beta, x_pending ? x : static_cast<double*>(nullptr),
                   static_cast<const double*>(p->scalars + S_ALPHA));
       });
       x_pending = false;

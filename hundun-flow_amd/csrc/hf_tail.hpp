@@ -174,7 +174,7 @@ struct TailRun {
   const double* b0;
   const uint8_t* act0;
   int cells0;
-  const double* mean;  // pending constant projection of b0, else null
+  MeanRef mean;        // pending constant projection of b0 (at: null, none)
   int levels;
   int work;        // LDS doubles of x, b, r (and slots 0 and 1)
   int head;        // doubles of the blob copied to LDS
@@ -489,7 +489,7 @@ __global__ void __launch_bounds__(kTailThreads) k_tail(TailRun a) {
   // ---- the blob's head and the first level's x and b into LDS, every load
   // independent of the others (a.work and a.head are even)
   const int work0 = kTailSlots;
-  const double mean = a.mean != nullptr ? *a.mean : 0.0;
+  const double mean = mean_value<kTailThreads>(a.mean, scratch);
   struct alignas(16) Pair {
     double v[2];
   };
@@ -503,7 +503,7 @@ __global__ void __launch_bounds__(kTailThreads) k_tail(TailRun a) {
   for (int c = tid; c < a.cells0; c += kTailThreads) {
     const double x = a.zero_x ? 0.0 : a.x0[c];
     double b = a.b0[c];
-    if (a.mean != nullptr) b = a.act0[c] ? b - mean : 0.0;
+    if (a.mean.at != nullptr) b = a.act0[c] ? b - mean : 0.0;
     tail_lds[work0 + c] = x;
     tail_lds[work0 + a.cells0 + c] = b;
   }

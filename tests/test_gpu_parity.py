@@ -882,3 +882,31 @@ def test_row_passes_bitwise(torch_cuda, monkeypatch, n, bc):
             if precision == "fp64":
                 assert np.array_equal(z[cells], zo), cells
         assert np.array_equal(z["32768"], z["0"]), precision
+
+
+@pytest.mark.parametrize("n", [(8, 8, 8), (32, 32, 32), (128, 128, 128),
+                               (136, 128, 128)])
+def test_sums_folded_by_their_consumer(torch_cuda, n):
+    """Means, p.q and r.z folded by the kernel that uses them (up to 1024
+    block sums: 128^3 has as many, the next grid more): the projected cycle
+    equals the oracle's to rounding, and PCG converges (with the oracle's
+    iterations where those are quick to compute)."""
+    torch = torch_cuda
+    _say(f"[folded sums] n={n}")
+    case = march_case(n, (1, 1, 1, 1, 2, 2), seed=43)
+    (d, bx, by, bz), mg = O.from_case(case, O.policy())
+    plan = _gpu_plan(torch, case)
+    z = plan.mg_apply(_t(torch, case["rhs"])).cpu().numpy()
+    zo = mg.apply(case["rhs"])
+    assert np.linalg.norm(z - zo) <= 1e-12 * np.linalg.norm(zo)
+    for flexible in (False, True):
+        _, res = plan.solve_pcg(_t(torch, case["rhs"]), rtol=1e-9,
+                                flexible=flexible)
+        assert res.final_true_residual <= 1e-9 * res.rhs_norm
+        if n[0] > 32:
+            continue
+        _, ref = O.pcg(case["n"], case["bc"], d, bx, by, bz,
+                       case["cell_active"], mg, case["rhs"], rtol=1e-9,
+                       flexible=flexible)
+        assert res.iterations == ref.iterations
+    plan.close()
