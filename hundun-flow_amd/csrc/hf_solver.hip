@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "hf_assembly.hpp"
+#include "hf_cheb.hpp"
 #include "hf_kernels.hpp"
 #include "hf_krylov.hpp"
 #include "hf_leg.hpp"
@@ -116,9 +117,11 @@ struct Level : Coeffs {
   void* lcd = nullptr;
   void* lghost = nullptr;
   bool cheb = false;   // Chebyshev-Jacobi smoothing (x2 holds x_next)
+  bool cheb_march = false;  // two stages as one march (k_cheb_march)
   bool sweep = false;  // fused two-colour sweep kernel
   bool leg = false;    // one launch per way down and way up (k_leg)
   bool march = false;  // two sweeps per launch (k_rb_march)
+  int march_gx = 0, march_gy = 0;  // its tiles along x and y
   int march_zc = 0;    // planes per block of it
   int march_blocks = 0;
   int sweep_zc = 0;    // planes per block of the sweep kernel
@@ -563,6 +566,18 @@ int64_t march_min_cells() {
   return int64_t{1} << 18;
 }
 
+// A Chebyshev level runs two stages as one march from this many cells (128^3:
+// as fast in FP32, 31 us against 45 in FP64; 64^3: 11 us against 10).
+// HF_SWEEP_MIN_CELLS overrides it too.
+int64_t cheb_march_min_cells() {
+  const char* env = std::getenv("HF_SWEEP_MIN_CELLS");
+  if (env != nullptr) {
+    const long long v = std::atoll(env);
+    if (v >= 0) return v;
+  }
+  return int64_t{1} << 20;
+}
+
 // Planes per block of the fused sweep on every level that takes it (0: the
 // planner's choice); HF_SWEEP_ZC sets it.
 int sweep_zc_override() {
@@ -574,25 +589,33 @@ int sweep_zc_override() {
   return 0;
 }
 
-// Launch shape of k_rb_march on level L: the z-chunks that take the fewest
+// z-chunks of a march over `tiles` column tiles: those that take the fewest
 // plane steps over the rounds in which 256 CUs, one block each, work them off
-// (a chunk pays six steps to fill).
+// (a chunk pays `fill` steps more than its planes).
+int march_chunk(const Level& L, int64_t tiles, int fill) {
+  if (sweep_zc_override() > 0) return std::min(L.n[2], sweep_zc_override());
+  int64_t best = 0;
+  int planes = L.n[2];
+  for (int chunks = 1; chunks <= L.n[2]; ++chunks) {
+    const int zc = (L.n[2] + chunks - 1) / chunks;
+    const int64_t steps = (tiles * chunks + 255) / 256 * (zc + fill);
+    if (best != 0 && steps >= best) continue;
+    best = steps;
+    planes = zc;
+  }
+  return planes;
+}
+
+// Launch shape of k_rb_march, or of k_cheb_march on a Chebyshev level.
 void plan_march(Level& L) {
   dispatch(L.prec, [&](auto t) {
     using T = decltype(t);
-    const int64_t tiles =
-        static_cast<int64_t>((L.n[0] + kMaOutX - 1) / kMaOutX) *
-        ((L.n[1] + kMaOutY<T> - 1) / kMaOutY<T>);
-    int64_t best = 0;
-    for (int chunks = 1; chunks <= L.n[2]; ++chunks) {
-      const int zc = (L.n[2] + chunks - 1) / chunks;
-      const int64_t steps = (tiles * chunks + 255) / 256 * (zc + 6);
-      if (best != 0 && steps >= best) continue;
-      best = steps;
-      L.march_zc = zc;
-    }
-    if (sweep_zc_override() > 0)
-      L.march_zc = std::min(L.n[2], sweep_zc_override());
+    const int ox = L.cheb ? kChOutX : kMaOutX;
+    const int oy = L.cheb ? kChOutY<T> : kMaOutY<T>;
+    L.march_gx = (L.n[0] + ox - 1) / ox;
+    L.march_gy = (L.n[1] + oy - 1) / oy;
+    const int64_t tiles = static_cast<int64_t>(L.march_gx) * L.march_gy;
+    L.march_zc = march_chunk(L, tiles, L.cheb ? 2 : 6);
     L.march_blocks = static_cast<int>(
         tiles * ((L.n[2] + L.march_zc - 1) / L.march_zc));
   });
@@ -1006,8 +1029,8 @@ void march_smooth(hf_plan* p, int l, int reverse, int from_zero,
   a.bout = a.mean.at != nullptr ? static_cast<T*>(L.b2) : nullptr;
   a.first = reverse ? 1 : 0;
   a.zc = L.march_zc;
-  a.gx = (L.n[0] + kMaOutX - 1) / kMaOutX;
-  a.gy = (L.n[1] + kMaOutY<T> - 1) / kMaOutY<T>;
+  a.gx = L.march_gx;
+  a.gy = L.march_gy;
   a.partials = mean_partials;
   a.wx = p->d_widths[0];
   a.wy = p->d_widths[1];
@@ -1171,6 +1194,25 @@ void cheb_smooth(hf_plan* p, int l, int stages, int retain, int from_zero) {
   Level& L = p->levels[l];
   ChebStage stage_factors(p->policy.chebyshev_lower_fraction);
   const int rb_class = l == 0 ? P_RB_FINEST : P_RB_COARSE;
+  if (L.cheb_march && stages == 2 && !(from_zero && p->cheb_first)) {
+    ChebMarchArgs<T> a;
+    a.L = view<T>(L);
+    a.bc = p->bc;
+    a.xout = static_cast<T*>(L.x2);
+    double rf = 0.0, pf = 0.0;
+    stage_factors.next(&rf, &pf);
+    a.rf1 = static_cast<C>(rf);
+    stage_factors.next(&rf, &pf);
+    a.rf2 = static_cast<C>(rf);
+    a.pf2 = static_cast<C>(pf);
+    a.zc = L.march_zc;
+    a.gx = L.march_gx;
+    a.gy = L.march_gy;
+    HF_PROF(p, rb_class);
+    HF_LAUNCH(k_cheb_march<T>, L.march_blocks, kChThreads<T>, 0, p->stream, a);
+    std::swap(L.x, L.x2);
+    stages = 0;
+  }
   for (int stage = 0; stage < stages; ++stage) {
     double rf = 0.0, pf = 0.0;
     stage_factors.next(&rf, &pf);
@@ -2513,7 +2555,12 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
     }
     L.march = l == 0 ? sweep_shape : sweep_shape && L.cells >= march_min_cells();
     L.march = L.march && L.n[2] >= 8 && march_enabled();
-    if (L.march) plan_march(L);
+    L.cheb_march = L.cheb && !L.tail && !L.leg && L.n[0] >= 32 &&
+                   L.n[0] % 2 == 0 && L.n[1] >= 8 && L.n[2] >= 8 &&
+                   L.cells >= cheb_march_min_cells() && march_enabled() &&
+                   widest * static_cast<int64_t>(elem_size(L.prec)) <
+                       (int64_t{1} << 32);
+    if (L.march || L.cheb_march) plan_march(L);
   }
   p->chunk0 = make_chunk(static_cast<int>(p->cells));
   if (!line_plan && 3 * p->levels.back().cells *

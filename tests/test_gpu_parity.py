@@ -910,3 +910,38 @@ def test_sums_folded_by_their_consumer(torch_cuda, n):
                        flexible=flexible)
         assert res.iterations == ref.iterations
     plan.close()
+
+
+@pytest.mark.parametrize("n,bc", [
+    ((32, 8, 8), (2, 2, 2, 2, 2, 2)),       # regions larger than the level
+    ((60, 28, 12), (0, 1, 1, 0, 1, 1)),     # one whole tile
+    ((62, 57, 9), (2, 2, 0, 1, 0, 0)),      # rims of one pair, of one row
+    ((130, 41, 21), (1, 0, 2, 2, 2, 2)),    # odd periodic y and z
+])
+def test_two_stage_march(torch_cuda, monkeypatch, n, bc):
+    """Two Chebyshev-Jacobi stages as one march (k_cheb_march) on tile edges,
+    wrapped regions, z-chunks and every boundary kind: FP64 equal to the
+    oracle, FP32 and BF16 to the two launches, bit for bit."""
+    torch = torch_cuda
+    _say(f"[cheb march] n={n} bc={bc}")
+    monkeypatch.setenv("HF_TAIL_CELLS", "0")
+    monkeypatch.setenv("HF_LEG_CELLS", "0")
+    monkeypatch.setenv("HF_SWEEP_MIN_CELLS", "0")
+    case = march_case(n, bc, seed=47)
+    pol = dict(null_space_constant=0, anisotropy_threshold=64.0, f_cycle=1,
+               pre_sweeps=1, post_sweeps=2, **_CHEB)
+    _, mg = O.from_case(case, O.policy(**pol))
+    r = np.random.default_rng(53).standard_normal(n[0] * n[1] * n[2])
+    zo = mg.apply(r)
+    for precision in ("fp64", "fp32", "bf16"):
+        z = {}
+        for march, chunk in (("0", "0"), ("1", "0"), ("1", "3")):
+            monkeypatch.setenv("HF_SWEEP_MARCH", march)
+            monkeypatch.setenv("HF_SWEEP_ZC", chunk)
+            plan = _gpu_plan(torch, case, precision=precision, **pol)
+            z[march + chunk] = plan.mg_apply(_t(torch, r)).cpu().numpy()
+            plan.close()
+        assert np.array_equal(z["10"], z["00"]), precision
+        assert np.array_equal(z["13"], z["00"]), precision
+        if precision == "fp64":
+            assert np.array_equal(z["00"], zo)
