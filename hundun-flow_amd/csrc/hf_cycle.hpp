@@ -476,112 +476,6 @@ __device__ __forceinline__ int wrapi(int v, int extent) {
   return v < 0 ? v + extent : (v >= extent ? v - extent : v);
 }
 
-// Retained defect fused with the restriction that consumes it
-// (src/solver_mg.cpp:3633-3720).  The z-marching layout of k_residual_z with
-// full tiles of even width and height and even z-chunks, on a level with
-// even extents coarsened along every axis: each step's defects, stored and
-// reloaded at the fine storage type, go through LDS to the thread owning the
-// coarse cell (even i, even j), which adds its eight children in the order
-// of k_restrict (dz, dy, dx) and stores the coarse b at the end of the odd
-// plane.  The fine r is not stored.  zero_x and partials as in k_restrict.
-//
-// kFirstStage: the level was just smoothed by one Chebyshev-Jacobi stage
-// from x = 0 (the pre-smoothing of a from-zero visit), which is not run:
-// every x this kernel reads is formed from that cell's b and D as the
-// stage stores it, st(0 + rf0 b / D), and the kernel also stores x of its
-// own cells into xs (the stage's direction is dead: the next stage on the
-// level starts a new recurrence).
-template <class Tf, class Tc, bool kFirstStage = false>
-__global__ void k_defect_restrict(Tiles t, Lv<Tf> L, Bc bc, Lv<Tc> Cl,
-                                  int zero_x, double* partials,
-                                  typename Compute<Tf>::type rf0 = 0,
-                                  Tf* xs = nullptr) {
-  using C = typename Compute<Tf>::type;
-  using Cc = typename Compute<Tc>::type;
-  __shared__ double scratch[16];
-  __shared__ Cc defect[kBlock];
-  const int lb = xcd_block32(blockIdx.x, gridDim.x);
-  const int gxy = t.gx * t.gy;
-  const int zb = lb / gxy;
-  int i, j, k_unused;
-  tile_xyz(t, lb - zb * gxy, i, j, k_unused);
-  const int nx = t.nx, ny = t.ny, nz = t.nz;
-  const int k0 = zb * t.per;
-  const int k1 = min(nz, k0 + t.per);
-  const int plane = nx * ny;
-  const int tw = 1 << t.txl;
-  const int tid = threadIdx.x;
-  const bool owner = ((i | j) & 1) == 0;
-  const Tf* x = L.x;
-  // x at cell q: stored, or formed from b and D as the first stage stores it
-  auto xat = [&](int q) -> C {
-    if constexpr (kFirstStage)
-      return C(ld(st<Tf>(C(0) + rf0 * C(ld(L.b[q])) / C(ld(L.D[q])))));
-    else
-      return C(ld(x[q]));
-  };
-  // neighbour_or_boundary through xat
-  auto nob = [&](int mode, C self, int wrapped) -> C {
-    if (mode == 0) return C(0);
-    if (mode == 1) return self;
-    return xat(wrapped);
-  };
-  int c = cell_index(nx, ny, i, j, k0);
-  C xc = xat(c);
-  C zl = k0 > 0 ? xat(c - plane) : nob(bc.m[4], xc, c + (nz - 1) * plane);
-  C fzl = C(ld(L.fz[c]));
-  Cc sum = Cc(0);
-  double pv = 0.0;
-  for (int k = k0; k < k1; ++k) {
-    const C zh = k + 1 < nz ? xat(c + plane)
-                            : nob(bc.m[5], xc, c - (nz - 1) * plane);
-    const C fzh = C(ld(L.fz[c + plane]));
-    const int row = j + ny * k;
-    const C xl = i > 0 ? xat(c - 1) : nob(bc.m[0], xc, c + (nx - 1));
-    const C xh = i + 1 < nx ? xat(c + 1) : nob(bc.m[1], xc, c - (nx - 1));
-    const C yl = j > 0 ? xat(c - nx) : nob(bc.m[2], xc, c + (ny - 1) * nx);
-    const C yh = j + 1 < ny ? xat(c + nx)
-                            : nob(bc.m[3], xc, c - (ny - 1) * nx);
-    if constexpr (kFirstStage) xs[c] = st<Tf>(xc);
-    const int fyo = c + nx * k;
-    C v = C(ld(L.D[c])) * xc;
-    v -= C(ld(L.fx[c + row])) * xl;
-    v -= C(ld(L.fx[c + row + 1])) * xh;
-    v -= C(ld(L.fy[fyo])) * yl;
-    v -= C(ld(L.fy[fyo + nx])) * yh;
-    v -= fzl * zl;
-    v -= fzh * zh;
-    const Tf r = st<Tf>(C(ld(L.b[c])) - v);
-    __syncthreads();  // the previous step's children have been read
-    defect[tid] = Cc(ld(r));
-    __syncthreads();
-    if (owner) {
-      // children (dx, dy) of this plane: dx fastest, as k_restrict adds them
-      sum += defect[tid];
-      sum += defect[tid + 1];
-      sum += defect[tid + tw];
-      sum += defect[tid + tw + 1];
-      if (k & 1) {
-        const int cc = cell_index(Cl.nx, Cl.ny, i >> 1, j >> 1, k >> 1);
-        const Tc stored = st<Tc>(sum);
-        Cl.b[cc] = stored;
-        if (zero_x) Cl.x[cc] = st<Tc>(0.0);
-        if (partials != nullptr)
-          pv += Cl.vol[cc] * static_cast<double>(ld(stored));
-        sum = Cc(0);
-      }
-    }
-    zl = xc;
-    xc = zh;
-    fzl = fzh;
-    c += plane;
-  }
-  if (partials != nullptr) {
-    pv = block_sum(pv, scratch);
-    if (threadIdx.x == 0) partials[lb] = pv;
-  }
-}
-
 // z-marching prolongation (src/solver_mg.cpp:3893-3993: x_f += sum of
 // ((wx*wy)*wz)*x_c over the (az, ay, ax) corners; fine solids := 0): a block
 // owns one 2-D tile of the fine level and t.per consecutive fine planes.

@@ -23,6 +23,7 @@
 #include "hf_leg.hpp"
 #include "hf_line.hpp"
 #include "hf_march.hpp"
+#include "hf_restrict.hpp"
 #include "hf_rows.hpp"
 #include "hf_tail.hpp"
 #include "hundun_flow.h"
@@ -713,20 +714,13 @@ bool op_on_tail(const hf_plan* p, const CycleOp& op) {
 
 // k_defect_restrict applies on level l: a fused-sweep, march or Chebyshev level
 // (its retained defect comes from one stencil pass after the smoothing),
-// coarsened along every axis with even extents, full z-marching tiles of
-// even width and height, even z-chunks.
+// coarsened along every axis with even extents.
 bool defect_restrict_ok(const hf_plan* p, int l) {
   if (!defect_restrict_enabled() || l + 1 >= static_cast<int>(p->levels.size()))
     return false;
   const Level& L = p->levels[l];
-  const Level& Cn = p->levels[l + 1];
-  const Tiles& t = L.tz;
-  const int tw = 1 << t.txl, th = kBlock >> t.txl;
   return (L.sweep || L.march || L.cheb) && L.coarsen_mask == 7 &&
-         L.n[0] % 2 == 0 && L.n[1] % 2 == 0 && L.n[2] % 2 == 0 && Cn.n[0] * 2 == L.n[0] &&
-         Cn.n[1] * 2 == L.n[1] && Cn.n[2] * 2 == L.n[2] && tw % 2 == 0 &&
-         th % 2 == 0 && L.n[0] % tw == 0 && L.n[1] % th == 0 &&
-         t.per % 2 == 0;
+         L.n[0] % 2 == 0 && L.n[1] % 2 == 0 && L.n[2] % 2 == 0;
 }
 
 // Passes over a level of one smoothing: colour passes or Chebyshev stages.
@@ -1402,15 +1396,9 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
     flush_mean(p);
   if (op.kind == T_SMOOTH) {
     // a one-stage Chebyshev smoothing from zero before the fused defect and
-    // restriction: that kernel forms the stage's x from b and D itself.
-    // Each cell then divides five times instead of once: measured, this
-    // pays on FP64 levels and on launch-bound small levels, while a large
-    // FP32 level runs faster as two passes (at 512x256x256: about 350 us
-    // fused against 79 + 210 us).
-    const bool first_stage =
-        defect_restrict && L.cheb && op.from_zero && op.sweeps == 1 &&
-        p->cheb_first &&
-        (L.prec == HF_PRECISION_FP64 || L.cells < (int64_t{1} << 20));
+    // restriction: that kernel forms the stage's x from b and D itself
+    const bool first_stage = defect_restrict && L.cheb && op.from_zero &&
+                             op.sweeps == 1 && p->cheb_first;
     if (!first_stage) {
       dispatch(L.prec, [&](auto t) {
         using T = decltype(t);
@@ -1428,27 +1416,38 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
       using Tf = decltype(tf);
       dispatch(Cd.prec, [&](auto tc) {
         using Tc = decltype(tc);
+        DefectArgs<Tf, Tc> a{};
+        a.L = view<Tf>(L);
+        a.bc = p->bc;
+        a.Cl = view<Tc>(Cd);
+        a.zero_x = stored ? 1 : 0;
+        a.partials = proj ? mean_partials_of(p, op.level + 1) : nullptr;
+        // two coarse planes per block share their rows of x (256^3 FP32 113
+        // us against 117), one fills the chip with more blocks (128^3 10.6
+        // against 12.9); a level with too few cells even so takes blocks of
+        // one wavefront
+        a.per = L.cells >= (int64_t{1} << 24) ? 2 : 1;
+        const int threads = Cd.cells < (int64_t{1} << 16) ? kWave : kBlock;
+        a.per_plane = static_cast<int>(
+            (static_cast<int64_t>(Cd.n[0]) * Cd.n[1] + threads - 1) / threads);
+        const int64_t blocks =
+            static_cast<int64_t>(a.per_plane) * ((Cd.n[2] + a.per - 1) / a.per);
+        HF_PROF(p, P_DEFECT);
         if (first_stage) {
-          using C = typename Compute<Tf>::type;
           double rf0 = 0.0, pf0 = 0.0;
           ChebStage(p->policy.chebyshev_lower_fraction).next(&rf0, &pf0);
-          HF_PROF(p, P_DEFECT);
-          HF_LAUNCH((k_defect_restrict<Tf, Tc, true>), L.tz.blocks, kBlock, 0,
-                    p->stream, L.tz, view<Tf>(L), p->bc, view<Tc>(Cd),
-                    stored ? 1 : 0,
-                    proj ? mean_partials_of(p, op.level + 1) : nullptr,
-                    static_cast<C>(rf0), static_cast<Tf*>(L.x2));
+          a.rf0 = static_cast<typename Compute<Tf>::type>(rf0);
+          a.xs = static_cast<Tf*>(L.x2);
+          HF_LAUNCH((k_defect_restrict<Tf, Tc, true>), blocks, threads, 0,
+                    p->stream, a);
           std::swap(L.x, L.x2);
         } else {
-          HF_PROF(p, P_DEFECT);
-          HF_LAUNCH((k_defect_restrict<Tf, Tc>), L.tz.blocks, kBlock, 0,
-                    p->stream, L.tz, view<Tf>(L), p->bc, view<Tc>(Cd),
-                    stored ? 1 : 0,
-                    proj ? mean_partials_of(p, op.level + 1) : nullptr);
+          HF_LAUNCH((k_defect_restrict<Tf, Tc, false>), blocks, threads, 0,
+                    p->stream, a);
         }
         if (proj) {
-          leave_mean(p, op.level + 1, mean_partials_of(p, op.level + 1),
-                     L.tz.blocks, folds_mean(p, op.level + 1));
+          leave_mean(p, op.level + 1, a.partials, blocks,
+                     folds_mean(p, op.level + 1));
           if (stored)
             project_apply<Tc>(p, op.level + 1, static_cast<Tc*>(Cd.b));
         }
