@@ -137,6 +137,7 @@ struct Level : Coeffs {
 };
 
 constexpr int kFoldSpan = 2048;   // partials per block of the first fold
+constexpr int kFinalizeMost = 16384;  // partials that k_finalize folds alone
 constexpr int kFoldStride = 4096;  // capacity per accumulator of the fold
 
 int ceil_log2(int v) {
@@ -829,7 +830,7 @@ void finalize(hf_plan* p, int64_t blocks, int nacc, int op, int slot,
   const double* src = first;
   int64_t count = blocks;
   int64_t stride = p->partial_stride;
-  if (blocks > kFoldSpan) {
+  if (blocks > kFinalizeMost) {
     // first pass: fixed spans of partials summed in order (deterministic)
     const int64_t spans = (blocks + kFoldSpan - 1) / kFoldSpan;
     hipLaunchKernelGGL(k_fold_partials, dim3(static_cast<uint32_t>(spans),
