@@ -24,7 +24,8 @@ __device__ __forceinline__ double geom_volume(const Widths& w, int i, int j,
 //   d = rf (b - A x) / D            (first stage)
 //   d = pf d + rf (b - A x) / D     (later stages)
 //   x_next = x + d.
-// z-marching as k_residual_z; x and x_next are distinct buffers.
+// z-marching (a thread walks its column through t.per planes, carrying x and
+// the z faces); x and x_next are distinct buffers.
 // ---------------------------------------------------------------------------
 template <class T>
 __global__ void k_cheb_stage(Tiles t, Lv<T> L, Bc bc, const T* x, T* xn,
@@ -263,7 +264,7 @@ enum FgMode : int { kFgArnoldi = 0, kFgResidual = 1, kFgOpDot = 2 };
 
 // Level-0 FP64 action y = A' x, A' = A or A divided by the geometric cell
 // volume (the per-volume rows of the cold system), z-marching as
-// k_residual_z, with the FGMRES epilogues:
+// k_cheb_stage, with the FGMRES epilogues:
 //  kFgArnoldi:  out = A' x - shift * aux (aux = v_col); accumulator a < kNd
 //               holds basis_a . out, accumulator wacc holds out . out;
 //  kFgResidual: out = 1 b + (-1) A' x (b = aux); accumulator 0 = out . out

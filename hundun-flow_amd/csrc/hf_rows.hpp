@@ -7,7 +7,11 @@ namespace hf {
 
 // ---------------------------------------------------------------------------
 // One pass over a level with the operator of every cell, or of every cell of
-// a colour: A x with x . A x (kRowsOperator), b - A x (kRowsDefect), or the
+// a colour: A x with x . A x (kRowsOperator), b - A x (kRowsDefect), the true
+// residual r = b - A x with r . r and, on request, the preconditioner's entry
+// made from it (kRowsResidual; axpby(r, 1, b, -1, Ax),
+// src/solver_krylov.cpp:1082-1091, and k_mg_entry: fluid ? r : 0 at level 0's
+// storage precision, which the restart after an unconverged check reads), or the
 // separated colour update of levels with an odd periodic extent, x_out =
 // x + 0.72 (b - A x) / D on the colour's cells and x elsewhere
 // (kRowsColour; src/solver_mg.cpp:3262-3307: every cell of the pass reads
@@ -31,7 +35,8 @@ namespace hf {
 // 143x101x75 in FP32: 7.1 us against 14.2 for A x of every cell and the
 // update as launches of their own.
 // ---------------------------------------------------------------------------
-constexpr int kRowsOperator = 0, kRowsDefect = 1, kRowsColour = 2;
+constexpr int kRowsOperator = 0, kRowsDefect = 1, kRowsColour = 2,
+              kRowsResidual = 3;
 
 // The pair at p, aligned as one element.
 template <class T>
@@ -59,20 +64,27 @@ __device__ __forceinline__ void rows_store(T* p, T lo, T hi) {
   }
 }
 
-template <class T>
+template <class T, class Te>
 struct RowsArgs {
   Lv<T> L;
   Bc bc;
   const T* x;
   T* out;
-  double* partials;  // kRowsOperator: block sums of x . A x, or null
+  // block sums: of x . A x (kRowsOperator; may be null); of r . r, then, each
+  // `stride` further, vol * entry over the fluid cells (proj) and b . b
+  // (with_bb; kRowsResidual)
+  double* partials;
+  int stride, proj, with_bb;
+  const uint8_t* act;  // with entry
+  Widths w;
+  Te* entry;           // null: not made
   int colour;        // kRowsColour
   int pairs;         // of a row: (nx + 1) / 2
   int per_plane;     // blocks of a plane
 };
 
-template <class T, int kMode, int kPer, bool kLine>
-__global__ void __launch_bounds__(kBlock) k_rows(RowsArgs<T> a) {
+template <class T, int kMode, int kPer, bool kLine, class Te = T>
+__global__ void __launch_bounds__(kBlock) k_rows(RowsArgs<T, Te> a) {
   using C = typename Compute<T>::type;
   __shared__ double scratch[16];
   const Lv<T>& L = a.L;
@@ -80,7 +92,7 @@ __global__ void __launch_bounds__(kBlock) k_rows(RowsArgs<T> a) {
   const int lb = xcd_block32(blockIdx.x, gridDim.x);
   const int zb = lb / a.per_plane;
   const int q = (lb - zb * a.per_plane) * kBlock + static_cast<int>(threadIdx.x);
-  double dot = 0.0;
+  double dot = 0.0, mean = 0.0, bb = 0.0;
   if (q < a.pairs * ny) {
     const int j = q / a.pairs;
     const int i0 = 2 * (q - j * a.pairs);
@@ -117,6 +129,12 @@ __global__ void __launch_bounds__(kBlock) k_rows(RowsArgs<T> a) {
     RowsPair<C> xp[kPer + 2], fz[kPer + 1], yl[kPer], yh[kPer], fyl[kPer],
         fyh[kPer], d[kPer], b[kPer], fx[kPer];
     C fx2[kPer], xl[kPer], xh[kPer];
+    bool fluid[kPer][2];
+    double wxy[2] = {0.0, 0.0};
+    if (kMode == kRowsResidual && a.entry != nullptr) {
+      wxy[0] = a.w.x[i0] * a.w.y[j];
+      wxy[1] = a.w.x[single ? i0 : i0 + 1] * a.w.y[j];
+    }
 #pragma unroll
     for (int u = 0; u < kPer + 2; ++u)
       xp[u] = pair(a.x + (plane_at(k0 - 1 + u) * plane + lo));
@@ -139,6 +157,10 @@ __global__ void __launch_bounds__(kBlock) k_rows(RowsArgs<T> a) {
       yh[u] = pair(a.x + (c + yh_at));
       xl[u] = C(ld(a.x[c + xl_at]));
       xh[u] = C(ld(a.x[c + xh_at]));
+      if (kMode == kRowsResidual && a.entry != nullptr) {
+        fluid[u][0] = a.act[c + at] != 0;
+        fluid[u][1] = a.act[c + at + (single ? 0 : 1)] != 0;
+      }
     }
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
@@ -194,6 +216,26 @@ __global__ void __launch_bounds__(kBlock) k_rows(RowsArgs<T> a) {
           o[0] = st<T>(b[u].v[0] - v0);
           o[1] = st<T>(b[u].v[1] - v1);
         }
+        if constexpr (kMode == kRowsResidual) {
+          Te made[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            if (e == 1 && single) break;
+            dot += o[e] * o[e];
+            bb += b[u].v[e] * b[u].v[e];
+            if (a.entry == nullptr) continue;
+            made[e] = fluid[u][e] ? st<Te>(o[e]) : st<Te>(0.0);
+            if (fluid[u][e])
+              mean += wxy[e] * a.w.z[k] * static_cast<double>(ld(made[e]));
+          }
+          if (a.entry != nullptr) {
+            Te* const entry = a.entry + (k * plane + at);
+            if (single)
+              *entry = made[0];
+            else
+              rows_store(entry, made[0], made[1]);
+          }
+        }
       }
       T* const out = a.out + (k * plane + at);
       if (single)
@@ -202,10 +244,19 @@ __global__ void __launch_bounds__(kBlock) k_rows(RowsArgs<T> a) {
         rows_store(out, o[0], o[1]);
     }
   }
-  if constexpr (kMode == kRowsOperator) {
-    if (a.partials != nullptr) {
-      dot = block_sum(dot, scratch);
-      if (threadIdx.x == 0) a.partials[lb] = dot;
+  if constexpr (kMode == kRowsOperator || kMode == kRowsResidual) {
+    if (a.partials == nullptr) return;
+    dot = block_sum(dot, scratch);
+    if (threadIdx.x == 0) a.partials[lb] = dot;
+  }
+  if constexpr (kMode == kRowsResidual) {
+    if (a.proj) {
+      mean = block_sum(mean, scratch);
+      if (threadIdx.x == 0) a.partials[lb + a.stride] = mean;
+    }
+    if (a.with_bb) {
+      bb = block_sum(bb, scratch);
+      if (threadIdx.x == 0) a.partials[lb + 2 * a.stride] = bb;
     }
   }
 }

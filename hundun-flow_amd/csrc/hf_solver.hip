@@ -953,36 +953,41 @@ Widths widths(const hf_plan* p) {
 // stays in the last-level cache is faster (A x in FP64, 1 and 2 planes:
 // 201x149x97 22.3 and 25.3 us, 192x192x128 33.9 and 37.5, 300x180x140 77 and
 // 74, 511x255x255 376 and 347).
-template <class T, int kMode>
-int64_t rows_pass(hf_plan* p, const Lv<T>& v, const T* x, T* out,
-                  double* partials, int colour) {
-  RowsArgs<T> a;
-  a.L = v;
+template <class T, int kMode, class Te = T>
+int64_t rows_pass(hf_plan* p, RowsArgs<T, Te> a) {
+  const Lv<T>& v = a.L;
   a.bc = p->bc;
-  a.x = x;
-  a.out = out;
-  a.partials = partials;
-  a.colour = colour;
   a.pairs = (v.nx + 1) / 2;
   a.per_plane = static_cast<int>(
       blocks_for(static_cast<int64_t>(a.pairs) * v.ny));
   const bool cached = static_cast<int64_t>(v.cells) * sizeof(T) < (48ll << 20);
-  const int64_t blocks =
-      static_cast<int64_t>(a.per_plane) * (cached || v.nx == 1 ? v.nz : (v.nz + 1) / 2);
+  const int64_t blocks = static_cast<int64_t>(a.per_plane) *
+                         (cached || v.nx == 1 ? v.nz : (v.nz + 1) / 2);
   if (v.nx == 1)
-    HF_LAUNCH((k_rows<T, kMode, 1, true>), blocks, kBlock, 0, p->stream, a);
+    HF_LAUNCH((k_rows<T, kMode, 1, true, Te>), blocks, kBlock, 0, p->stream, a);
   else if (cached)
-    HF_LAUNCH((k_rows<T, kMode, 1, false>), blocks, kBlock, 0, p->stream, a);
+    HF_LAUNCH((k_rows<T, kMode, 1, false, Te>), blocks, kBlock, 0, p->stream,
+              a);
   else
-    HF_LAUNCH((k_rows<T, kMode, 2, false>), blocks, kBlock, 0, p->stream, a);
+    HF_LAUNCH((k_rows<T, kMode, 2, false, Te>), blocks, kBlock, 0, p->stream,
+              a);
   return blocks;
+}
+
+template <class T>
+RowsArgs<T, T> rows_args(const Lv<T>& v, const T* x, T* out) {
+  RowsArgs<T, T> a{};
+  a.L = v;
+  a.x = x;
+  a.out = out;
+  return a;
 }
 
 // The retained defect r = b - A x of a level.
 template <class T>
 void level_defect(hf_plan* p, const Lv<T>& v) {
   HF_PROF(p, P_DEFECT);
-  rows_pass<T, kRowsDefect>(p, v, v.x, v.r, nullptr, 0);
+  rows_pass<T, kRowsDefect>(p, rows_args<T>(v, v.x, v.r));
 }
 
 // Mean of a level field for the constant projection: scalars[S_MEAN0 + l].
@@ -1289,8 +1294,9 @@ void point_smooth(hf_plan* p, int l, int sweeps, int reverse, int retain,
                   p->bc, color);
       } else {
         // (the pass reads x from before it everywhere)
-        rows_pass<T, kRowsColour>(p, v, v.x, static_cast<T*>(L.x2), nullptr,
-                                  color);
+        RowsArgs<T, T> a = rows_args<T>(v, v.x, static_cast<T*>(L.x2));
+        a.colour = color;
+        rows_pass<T, kRowsColour>(p, a);
         std::swap(L.x, L.x2);
       }
     }
@@ -2944,9 +2950,12 @@ hf_status hf_plan_set_coefficients(hf_plan* p, const double* diag,
 static int64_t operator_pass(hf_plan* p, const double* x, double* y,
                              double* partials) {
   const Level& L = p->levels[0];
-  if (!p->krylov_pairs || L.n[0] % 128 != 0 || L.cells < (int64_t{12} << 20))
-    return rows_pass<double, kRowsOperator>(p, krylov_view(p), x, y, partials,
-                                            0);
+  if (!p->krylov_pairs || L.n[0] % 128 != 0 ||
+      L.cells < (int64_t{12} << 20)) {
+    RowsArgs<double, double> a = rows_args<double>(krylov_view(p), x, y);
+    a.partials = partials;
+    return rows_pass<double, kRowsOperator>(p, a);
+  }
   HF_LAUNCH((k_fg_stencil2<kFgOpDot, 0>), L.tzp.blocks, kBlock, 0, p->stream,
             L.tzp, krylov_view(p), p->bc, x,
             static_cast<const double*>(nullptr), y,
@@ -2975,7 +2984,6 @@ hf_status hf_mg_apply(hf_plan* p, const double* r, double* z) {
 static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
                           const hf_solve_control* ctl, hf_solve_result* res) {
   const Lv<double> A = krylov_view(p);
-  const Tiles& tr = p->levels[0].tz;  // z-marching Krylov stencils
   // the PCG update stores the preconditioner's entry when level 0 is a grid
   // level (the tail and line-relaxed entries also zero x; a Chebyshev level 0
   // reads no x in its first stage, and mg_apply projects its b)
@@ -3001,21 +3009,27 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
   // from r (accumulator 1), which the restart that follows an unconverged
   // check then skips.
   const int stride = static_cast<int>(p->partial_stride);
+  int64_t residual_blocks = 0;
   auto true_residual = [&](bool with_bb) -> hf_status {
     HF_PROF(p, P_TRUE_RESIDUAL);
-    if (!fuse_entry) {
-      HF_LAUNCH(k_residual_z, tr.blocks, kBlock, 0, p->stream, tr, A, p->bc, static_cast<const double*>(x), rhs,
-                r, p->partials, with_bb ? 2 * stride : 0);
-      return ok();
-    }
     Level& L0 = p->levels[0];
     dispatch(L0.prec, [&](auto t) {
       using T = decltype(t);
-      HF_LAUNCH(k_residual_entry<T>, tr.blocks, kBlock, 0, p->stream, tr, A,
-                p->bc, static_cast<const double*>(x), rhs, r,
-                static_cast<const uint8_t*>(L0.act), widths(p),
-                static_cast<T*>(L0.b), p->partials, stride,
-                p->policy.null_space_constant != 0 ? 1 : 0, with_bb ? 1 : 0);
+      RowsArgs<double, T> a{};
+      a.L = A;
+      a.L.b = const_cast<double*>(rhs);  // (read only)
+      a.x = x;
+      a.out = r;
+      a.partials = p->partials;
+      a.stride = stride;
+      a.with_bb = with_bb ? 1 : 0;
+      if (fuse_entry) {
+        a.proj = p->policy.null_space_constant != 0 ? 1 : 0;
+        a.act = L0.act;
+        a.w = widths(p);
+        a.entry = static_cast<T*>(L0.b);
+      }
+      residual_blocks = rows_pass<double, kRowsResidual, T>(p, a);
     });
     return ok();
   };
@@ -3033,8 +3047,8 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
   // ||b||, whose residual goes unused, then the residual)
   HF_LAUNCH(k_copy, nbv, kBlock, 0, p->stream, ch, x, solution);
   HF_TRY(true_residual(true));
-  finalize(p, tr.blocks, 1, F_STORE, S_SUM, 0.0, 1, 2);
-  residual_sums(tr.blocks);
+  finalize(p, residual_blocks, 1, F_STORE, S_SUM, 0.0, 1, 2);
+  residual_sums(residual_blocks);
   HF_TRY(read_scalars(p));
   double bnorm = std::sqrt(p->host_scalars[S_SUM]);
   if (!std::isfinite(bnorm)) {
@@ -3196,7 +3210,7 @@ static hf_status pcg_impl(hf_plan* p, const double* rhs, double* solution,
         x_pending = false;
       }
       HF_TRY(true_residual(false));
-      residual_sums(tr.blocks);
+      residual_sums(residual_blocks);
       HF_TRY(read_scalars(p));
       if (rho_failed()) return fail_rho();
       // a step that fails these checks stops before the true residual, as
