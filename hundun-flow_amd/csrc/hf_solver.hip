@@ -260,7 +260,8 @@ Lv<double> op_view(const Level& L) {
 using namespace hf;
 
 namespace {
-// Brackets the enclosed launch with a pair of events when profiling is on.
+// Brackets the enclosed launch with a pair of events when profiling is on (a
+// scope holds no other one).
 struct ProfScope {
   hf_plan* p;
   explicit ProfScope(hf_plan* plan, int cls);
@@ -686,7 +687,7 @@ int64_t tail_threshold() {
     const long long v = std::atoll(env);
     if (v >= 0) return v;
   }
-  return 8192;
+  return kTailMaxCells;
 }
 
 // Build the cycle program exactly as mg_cycle recurses
@@ -1439,16 +1440,17 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
             (static_cast<int64_t>(Cd.n[0]) * Cd.n[1] + threads - 1) / threads);
         const int64_t blocks =
             static_cast<int64_t>(a.per_plane) * ((Cd.n[2] + a.per - 1) / a.per);
-        HF_PROF(p, P_DEFECT);
         if (first_stage) {
           double rf0 = 0.0, pf0 = 0.0;
           ChebStage(p->policy.chebyshev_lower_fraction).next(&rf0, &pf0);
           a.rf0 = static_cast<typename Compute<Tf>::type>(rf0);
           a.xs = static_cast<Tf*>(L.x2);
+          HF_PROF(p, P_DEFECT);
           HF_LAUNCH((k_defect_restrict<Tf, Tc, true>), blocks, threads, 0,
                     p->stream, a);
           std::swap(L.x, L.x2);
         } else {
+          HF_PROF(p, P_DEFECT);
           HF_LAUNCH((k_defect_restrict<Tf, Tc, false>), blocks, threads, 0,
                     p->stream, a);
         }

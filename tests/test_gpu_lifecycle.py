@@ -198,3 +198,29 @@ def test_refresh_reaches_every_entry(torch_cuda, n, masked):
                 plan.set_coefficients(*bad, *masks)
             assert err.value.code == 5  # numerical_failure
     plan.close()
+
+
+@pytest.mark.parametrize("n", [(32, 32, 32), (64, 64, 64), (64, 48, 33)])
+@pytest.mark.parametrize("smoother", ["red_black", "chebyshev"])
+def test_profiled_solve(torch_cuda, n, smoother):
+    """A solve under event profiling (each launch in a scope of its own, with
+    the projection of a closed domain between them) is the plain solve."""
+    import hundun_flow as H
+    torch = torch_cuda
+    _say(f"[profiled] n={n} smoother={smoother}")
+    case = hf_cases.lognormal_sphere(n=n, seed=17)
+    pol = dict(f_cycle=1, pre_sweeps=1, point_smoother=1) \
+        if smoother == "chebyshev" else {}
+    plan = H.plan_from_case(case, H.default_policy(
+        anisotropy_threshold=64.0, **pol))
+    b = _t(torch, case["rhs"])
+    x, plain = plan.solve_pcg(b, rtol=1e-9, flexible=True)
+    plan.set_profiling(True)
+    y, profiled = plan.solve_pcg(b, rtol=1e-9, flexible=True)
+    times = plan.profile()
+    plan.set_profiling(False)
+    assert torch.equal(x, y)
+    assert profiled.iterations == plain.iterations
+    assert all(ms >= 0.0 and launches >= 0 for ms, launches in times.values())
+    assert sum(launches for _, launches in times.values()) > 0
+    plan.close()
