@@ -41,7 +41,9 @@ namespace hf {
 // sweeps, one launch against two k_rb_sweep launches, from x and from zero:
 // 512x256x256 FP32 298 and 267 us against 478 and 445, 256x256x128 FP64 163
 // and 149 against 277 and 254, 192x192x128 BF16 44 and 41 against 83 and 77.
-// HBM traffic at 512x256x256 FP32 is 1.2 GB for 0.94 GB of operands.
+// HBM traffic at 512x256x256 FP32 is 1.2 GB for 0.94 GB of operands.  Within
+// a solve, with the projection's mean: 345 us from zero and 330 with the mean
+// of the output (351 while that read the fluid flags).
 //
 // Boundaries: a position outside the domain holds 0 (Dirichlet; never
 // updated) or is the wrapped cell (periodic); on a Neumann face the neighbour
@@ -70,8 +72,10 @@ struct MarchArgs {
   int first;           // colour updated first: 0 forward, 1 reverse
   int zc;              // planes per chunk
   int gx, gy;          // tiles along x and y
-  // kMean: per-block partial sums of vol * x over fluid cells of the output
-  // (the constant projection's mean), cell widths per axis
+  // kMean: per-block partial sums of w_x w_y w_z x of the output (the
+  // constant projection's mean), cell widths per axis.  Solid cells add 0:
+  // the prolongation before this smoothing left x = 0 there, b is 0, their
+  // faces are masked.
   double* partials;
   const double* wx;
   const double* wy;
@@ -173,12 +177,10 @@ __global__ void __launch_bounds__(kMaThreads<T>) k_rb_march(MarchArgs<T> a) {
   // a periodic axis, whose low faces are an array plane of their own
   MaPair<C> d[4], fyl[4], fyh[4], fzh[4], fz0, fzb;
   C fx[4][3];
-  uint32_t act[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     d[u] = fyl[u] = fyh[u] = fzh[u] = {C(1), C(1)};
     fx[u][0] = fx[u][1] = fx[u][2] = C(0);
-    act[u] = 0;
   }
   // raw operands in flight: coefficients of the next step's plane, x of the
   // plane above it
@@ -199,7 +201,7 @@ __global__ void __launch_bounds__(kMaThreads<T>) k_rb_march(MarchArgs<T> a) {
     nyl = sw_load2<T>(rfy, oc, sy);
     nyh = sw_load2<T>(rfy, oc, sy + nx * kS);
     nzh = sw_load2<T>(rfz, oc, sc + nxy * kS);
-    if ((kZero && a.mean.at != nullptr) || kMean)
+    if (kZero && a.mean.at != nullptr)
       nact = *reinterpret_cast<const uint16_t*>(L.act + (sc + oc) / kS);
     if constexpr (!kZero)
       nx2 = sw_load2<T>(rx, oc, static_cast<uint32_t>(wx) * nxy * kS);
@@ -234,7 +236,6 @@ __global__ void __launch_bounds__(kMaThreads<T>) k_rb_march(MarchArgs<T> a) {
     fx[U][0] = C(ld(nf0));
     fx[U][1] = C(ld(nf1));
     fx[U][2] = C(ld(nf2));
-    if (kZero || kMean) act[U] = nact;
     MaPair<C> bk;
     if (kZero && a.mean.at != nullptr) {
       const T lo = st<T>(static_cast<double>(ld(nb.lo)) - mean);
@@ -318,10 +319,9 @@ __global__ void __launch_bounds__(kMaThreads<T>) k_rb_march(MarchArgs<T> a) {
       const uint32_t sc = static_cast<uint32_t>(kk) * nxy * kS;
       sw_store2(rout, oc, sc, lo, hi);
       if constexpr (kMean) {
-        constexpr int U3 = (U + 1) & 3;
         const double wz = a.wz[kk];
-        if (act[U3] & 0xffu) mlo += wz * static_cast<double>(ld(lo));
-        if (act[U3] & 0xff00u) mhi += wz * static_cast<double>(ld(hi));
+        mlo += wz * static_cast<double>(ld(lo));
+        mhi += wz * static_cast<double>(ld(hi));
       }
     }
     if (kZero && a.bout != nullptr && k >= z0 && k < z1 && mine)
