@@ -44,8 +44,8 @@ def class_bytes_per_cell(cls: str, s: int):
         "rb_finest": 5.5 * s,
         # first half-sweep from x = 0: read b, D; write b (projected), x
         "rb_first": 4 * s,
-        # fused two-colour sweep: read x, b, D, 3 face arrays, write x (the
-        # first sweep from zero reads no x and writes the projected b)
+        # two sweeps in one pass: read x, b, D, 3 face arrays, write x (from
+        # zero no x is read and the projected b written)
         "sweep_finest": 7 * s,
         # the cycle's last fused sweep, which also sums the level-0 mean:
         # the sweep's arrays and the fluid flags
@@ -67,8 +67,8 @@ def class_bytes_per_cell(cls: str, s: int):
 # kernel class -> symbol of its kernel for the rocprof traffic lookup
 CLASS_KERNELS = {
     "rb_finest": "void hf::k_rb<{t}>(hf::Tiles, hf::Lv<{t}>, hf::Bc, int)",
-    "sweep_finest": "void hf::k_rb_sweep<{t}, false, false>(hf::SweepArgs<{t}>)",
-    "operator": "void hf::k_stencil_z<double, 0>(hf::Tiles, hf::Lv<double>, hf::Bc, double const*, double const*, double*, double*, int)",
+    "sweep_finest": "void hf::k_rb_march<{t}, false, true>(hf::MarchArgs<{t}>)",
+    "operator": "void hf::k_fg_stencil2<2, 0>(hf::Tiles, hf::Lv<double>, hf::Bc, double const*, double const*, double*, double const*, long, int, double, int, hf::Widths, double*, long)",
 }
 
 
@@ -84,7 +84,7 @@ def measured_traffic(workload_tag, cls, precision, grid):
         data = json.load(f)
     entry = data["kernels"].get(f"{name}|{grid}")
     if entry is None and cls == "sweep_finest":
-        # the fused sweep also runs on large coarse levels: the finest
+        # the march also runs on large coarse levels: the finest
         # level's launches are the ones moving the most bytes
         hits = [v for k, v in data["kernels"].items()
                 if k.split("|")[0] == name]
