@@ -768,6 +768,69 @@ bool leg_ok(const hf_plan* p, int l) {
          leg_boxes(L, h).blocks <= kLegMaxBlocks;
 }
 
+// Blocks of a k_rows pass.  Two planes per block share the rows of x between
+// them; with one plane per block a level that stays in the last-level cache
+// is faster (A x in FP64, 1 and 2 planes: 201x149x97 22.3 and 25.3 us,
+// 192x192x128 33.9 and 37.5, 300x180x140 77 and 74, 511x255x255 376 and 347).
+struct RowsShape {
+  int pairs, per_plane;
+  int per;  // planes per block
+  int64_t blocks;
+};
+
+RowsShape rows_shape(int nx, int ny, int nz, size_t elem) {
+  RowsShape r{};
+  r.pairs = (nx + 1) / 2;
+  r.per_plane =
+      static_cast<int>(blocks_for(static_cast<int64_t>(r.pairs) * ny));
+  const bool cached = static_cast<int64_t>(nx) * ny * nz *
+                          static_cast<int64_t>(elem) < (48ll << 20);
+  r.per = cached || nx == 1 ? 1 : 2;
+  r.blocks = static_cast<int64_t>(r.per_plane) * ((nz + r.per - 1) / r.per);
+  return r;
+}
+
+// Blocks of k_defect_restrict on level L with the coarse level Cd.  Two
+// coarse planes per block share their rows of x (256^3 FP32 113 us against
+// 117), one fills the chip with more blocks (128^3 10.6 against 12.9); a
+// level with too few cells even so takes blocks of one wavefront.
+struct RestrictShape {
+  int threads, per, per_plane;
+  int64_t blocks;
+};
+
+RestrictShape restrict_shape(const Level& L, const Level& Cd) {
+  RestrictShape r{};
+  r.per = L.cells >= (int64_t{1} << 24) ? 2 : 1;
+  r.threads = Cd.cells < (int64_t{1} << 16) ? kWave : kBlock;
+  r.per_plane = static_cast<int>(
+      (static_cast<int64_t>(Cd.n[0]) * Cd.n[1] + r.threads - 1) / r.threads);
+  r.blocks =
+      static_cast<int64_t>(r.per_plane) * ((Cd.n[2] + r.per - 1) / r.per);
+  return r;
+}
+
+// The most block sums (per accumulator) that any launch on level l makes; a
+// plan's buffers hold the most of its levels.  The tiles of a sweep or a march
+// are other ones than tc's, and on a slim level, a plane per chunk, they can
+// be more (58x17x42 FP64: 252 blocks of a march, 210 tiles).  The launches
+// take their blocks from the same fields and functions.
+int64_t level_sum_blocks(const hf_plan* p, size_t l) {
+  const Level& L = p->levels[l];
+  int64_t most = std::max<int64_t>({L.tc.count, L.tr.blocks, L.tred.blocks,
+                                    blocks_for(L.cells)});
+  if (L.sweep) most = std::max<int64_t>(most, L.sweep_blocks);
+  if (L.march) most = std::max<int64_t>(most, L.march_blocks);
+  if (L.leg) most = std::max(most, leg_boxes(L, kLegHalo).blocks);
+  if (defect_restrict_ok(p, static_cast<int>(l)))
+    most = std::max(most, restrict_shape(L, p->levels[l + 1]).blocks);
+  if (l == 0)
+    most = std::max<int64_t>(
+        {most, rows_shape(L.n[0], L.n[1], L.n[2], sizeof(double)).blocks,
+         L.tz.blocks, L.tzp.blocks});
+  return most;
+}
+
 void build_exec(hf_plan* p) {
   p->program.clear();
   p->exec.clear();
@@ -949,30 +1012,24 @@ Widths widths(const hf_plan* p) {
   return Widths{p->d_widths[0], p->d_widths[1], p->d_widths[2]};
 }
 
-// One k_rows pass over a level; returns its blocks.  Two planes per block
-// share the rows of x between them; with one plane per block a level that
-// stays in the last-level cache is faster (A x in FP64, 1 and 2 planes:
-// 201x149x97 22.3 and 25.3 us, 192x192x128 33.9 and 37.5, 300x180x140 77 and
-// 74, 511x255x255 376 and 347).
+// One k_rows pass over a level; returns its blocks.
 template <class T, int kMode, class Te = T>
 int64_t rows_pass(hf_plan* p, RowsArgs<T, Te> a) {
   const Lv<T>& v = a.L;
+  const RowsShape r = rows_shape(v.nx, v.ny, v.nz, sizeof(T));
   a.bc = p->bc;
-  a.pairs = (v.nx + 1) / 2;
-  a.per_plane = static_cast<int>(
-      blocks_for(static_cast<int64_t>(a.pairs) * v.ny));
-  const bool cached = static_cast<int64_t>(v.cells) * sizeof(T) < (48ll << 20);
-  const int64_t blocks = static_cast<int64_t>(a.per_plane) *
-                         (cached || v.nx == 1 ? v.nz : (v.nz + 1) / 2);
+  a.pairs = r.pairs;
+  a.per_plane = r.per_plane;
   if (v.nx == 1)
-    HF_LAUNCH((k_rows<T, kMode, 1, true, Te>), blocks, kBlock, 0, p->stream, a);
-  else if (cached)
-    HF_LAUNCH((k_rows<T, kMode, 1, false, Te>), blocks, kBlock, 0, p->stream,
+    HF_LAUNCH((k_rows<T, kMode, 1, true, Te>), r.blocks, kBlock, 0, p->stream,
+              a);
+  else if (r.per == 1)
+    HF_LAUNCH((k_rows<T, kMode, 1, false, Te>), r.blocks, kBlock, 0, p->stream,
               a);
   else
-    HF_LAUNCH((k_rows<T, kMode, 2, false, Te>), blocks, kBlock, 0, p->stream,
+    HF_LAUNCH((k_rows<T, kMode, 2, false, Te>), r.blocks, kBlock, 0, p->stream,
               a);
-  return blocks;
+  return r.blocks;
 }
 
 template <class T>
@@ -1430,16 +1487,11 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
         a.Cl = view<Tc>(Cd);
         a.zero_x = stored ? 1 : 0;
         a.partials = proj ? mean_partials_of(p, op.level + 1) : nullptr;
-        // two coarse planes per block share their rows of x (256^3 FP32 113
-        // us against 117), one fills the chip with more blocks (128^3 10.6
-        // against 12.9); a level with too few cells even so takes blocks of
-        // one wavefront
-        a.per = L.cells >= (int64_t{1} << 24) ? 2 : 1;
-        const int threads = Cd.cells < (int64_t{1} << 16) ? kWave : kBlock;
-        a.per_plane = static_cast<int>(
-            (static_cast<int64_t>(Cd.n[0]) * Cd.n[1] + threads - 1) / threads);
-        const int64_t blocks =
-            static_cast<int64_t>(a.per_plane) * ((Cd.n[2] + a.per - 1) / a.per);
+        const RestrictShape shape = restrict_shape(L, Cd);
+        a.per = shape.per;
+        a.per_plane = shape.per_plane;
+        const int threads = shape.threads;
+        const int64_t blocks = shape.blocks;
         if (first_stage) {
           double rf0 = 0.0, pf0 = 0.0;
           ChebStage(p->policy.chebyshev_lower_fraction).next(&rf0, &pf0);
@@ -2396,10 +2448,10 @@ hf_status hf_policy_default(hf_policy* policy) {
   return ok();
 }
 
-hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
-                         void* stream, hf_plan** out) {
-  if (out == nullptr) return fail(HF_INVALID_PLAN, kDetailPlan);
-  *out = nullptr;
+// The host half of plan creation: checks, levels, their launch shapes and the
+// cycle program (no device call).
+static hf_status plan_layout(const hf_grid_desc* grid, const hf_policy* policy,
+                             hf_plan* p) {
   if (grid == nullptr || policy == nullptr || grid->nx <= 0 || grid->ny <= 0 ||
       grid->nz <= 0 || grid->faces_x == nullptr || grid->faces_y == nullptr ||
       grid->faces_z == nullptr)
@@ -2429,15 +2481,8 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
         nx * (ny + 1) * nz > limit || nx * ny * (nz + 1) > limit)
       return fail(HF_INVALID_PLAN, kDetailPlan);
   }
-  hf_plan* p = new (std::nothrow) hf_plan();
-  if (p == nullptr) return fail(HF_ALLOCATION_FAILURE, kDetailAlloc);
   p->grid = *grid;
   p->policy = *policy;
-  p->stream = static_cast<hipStream_t>(stream);
-  if (hipGetDevice(&p->device) != hipSuccess) {
-    delete p;
-    return fail(HF_INVALID_PLAN, kDetailHip);
-  }
   p->n[0] = grid->nx;
   p->n[1] = grid->ny;
   p->n[2] = grid->nz;
@@ -2449,7 +2494,6 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
     for (int i = 0; i < p->n[a]; ++i) {
       const double w = p->faces[a][i + 1] - p->faces[a][i];
       if (!(w > 0.0) || !std::isfinite(w)) {
-        delete p;
         return fail(HF_INVALID_PLAN, kDetailPlan);
       }
       p->widths[a][i] = w;
@@ -2464,12 +2508,10 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
                      (grid->boundary[4] == HF_BC_PERIODIC ? 4 : 0);
   plan_levels(p);
   if (p->levels.size() < 2) {
-    delete p;
     return fail(HF_INVALID_PLAN, kDetailPlan);
   }
   const bool line_plan = p->levels[0].line_mask != 0;
   if (line_plan && !line_relaxation_enabled()) {
-    delete p;
     return fail(HF_INVALID_PLAN, kDetailLineOff);
   }
   // the tail is the longest run of coarsest levels whose x, b, r fit the
@@ -2575,12 +2617,31 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
                             static_cast<int64_t>(sizeof(double)) >
                         kTailWorkBytes) {
     // the coarsest level alone exceeds the tail
-    delete p;
     return fail(HF_INVALID_PLAN, kDetailPlan);
   }
   build_exec(p);
+  int64_t most = 0;
+  for (size_t l = 0; l < p->levels.size(); ++l)
+    most = std::max(most, level_sum_blocks(p, l));
+  p->partial_stride = most + 8;
+  return ok();
+}
 
-  hf_status s = ok();
+hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
+                         void* stream, hf_plan** out) {
+  if (out == nullptr) return fail(HF_INVALID_PLAN, kDetailPlan);
+  *out = nullptr;
+  hf_plan* p = new (std::nothrow) hf_plan();
+  if (p == nullptr) return fail(HF_ALLOCATION_FAILURE, kDetailAlloc);
+  hf_status s = plan_layout(grid, policy, p);
+  p->stream = static_cast<hipStream_t>(stream);
+  if (s.code == HF_OK && hipGetDevice(&p->device) != hipSuccess)
+    s = fail(HF_INVALID_PLAN, kDetailHip);
+  if (s.code != HF_OK) {
+    delete p;
+    return s;
+  }
+
   auto guard = [&](hf_status st) {
     if (st.code != HF_OK && s.code == HF_OK) s = st;
   };
@@ -2614,13 +2675,6 @@ hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
       guard(dalloc_raw(p, &L.lghost, es * ghosts));
     }
   }
-  // one partial per tile (level 0 has the most) or per 256-element block
-  int64_t max_blocks = blocks_for(p->cells);
-  for (const Level& L : p->levels) {
-    max_blocks = std::max<int64_t>(max_blocks, L.tc.count);
-    if (L.leg) max_blocks = std::max(max_blocks, leg_boxes(L, kLegHalo).blocks);
-  }
-  p->partial_stride = max_blocks + 8;
   guard(dalloc(p, &p->partials, 3 * p->partial_stride));
   guard(dalloc(p, &p->folded, 3 * kFoldStride));
   guard(dalloc(p, &p->scalars, S_COUNT));
@@ -3642,6 +3696,35 @@ hf_status hf_plan_level_info(const hf_plan* p, int32_t level,
   info->precision = static_cast<uint8_t>(L.prec);
   info->on_tail = L.tail ? 1 : 0;
   return ok();
+}
+
+hf_status hf_launch_shape_of(const hf_grid_desc* grid, const hf_policy* policy,
+                             int32_t level, hf_launch_shape* shape) {
+  if (shape == nullptr) return fail(HF_INVALID_PLAN, kDetailPlan);
+  std::memset(shape, 0, sizeof *shape);
+  hf_plan* p = new (std::nothrow) hf_plan();
+  if (p == nullptr) return fail(HF_ALLOCATION_FAILURE, kDetailAlloc);
+  hf_status s = plan_layout(grid, policy, p);
+  if (s.code == HF_OK &&
+      (level < 0 || level >= static_cast<int32_t>(p->levels.size())))
+    s = fail(HF_INVALID_PLAN, kDetailPlan);
+  if (s.code == HF_OK) {
+    const Level& L = p->levels[level];
+    shape->route = L.tail             ? HF_ROUTE_TAIL
+                   : L.line_mask != 0 ? HF_ROUTE_LINES
+                   : L.leg            ? HF_ROUTE_LEG
+                   : L.cheb_march     ? HF_ROUTE_STAGE_MARCH
+                   : L.cheb           ? HF_ROUTE_STAGES
+                   : L.march          ? HF_ROUTE_MARCH
+                   : L.sweep          ? HF_ROUTE_SWEEP
+                   : L.fused          ? HF_ROUTE_COLOURS
+                                      : HF_ROUTE_SEPARATED;
+    shape->levels = static_cast<int32_t>(p->levels.size());
+    shape->sum_blocks = level_sum_blocks(p, static_cast<size_t>(level));
+    shape->sum_capacity = p->partial_stride;
+  }
+  delete p;
+  return s;
 }
 
 hf_status hf_plan_level_array(const hf_plan* p, int32_t level, int32_t which,

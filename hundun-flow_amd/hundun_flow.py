@@ -27,6 +27,9 @@ TERMINATIONS = ["converged", "zero_rhs", "maximum_iterations", "breakdown",
                 "non_finite", "operator_failure", "preconditioner_failure",
                 "collective_failure", "invalid_plan"]
 PRECISIONS = {"fp64": 0, "fp32": 1, "bf16": 2}
+# hf_route: the kernels that smooth a level
+ROUTES = ["tail", "leg", "march", "sweep", "colours", "separated",
+          "stage_march", "stages", "lines"]
 # kernel classes of hf_plan_profile, in order
 PROFILE_CLASSES = ["rb_finest", "rb_coarse", "defect", "restrict", "prolong",
                    "tail", "operator", "update_xr", "true_residual",
@@ -44,7 +47,7 @@ ABI_FUNCTIONS = [
     "hf_plan_level_array", "hf_plan_device_bytes", "hf_plan_set_profiling",
     "hf_plan_profile", "hf_status_message", "hf_vector_engine_create",
     "hf_vector_engine_destroy", "hf_vector_engine_slot", "hf_vector_dot",
-    "hf_vector_axpby", "hf_vector_copy",
+    "hf_vector_axpby", "hf_vector_copy", "hf_launch_shape_of",
 ]
 
 
@@ -119,6 +122,12 @@ class hf_level_info(ctypes.Structure):
                 ("on_tail", ctypes.c_uint8)]
 
 
+class hf_launch_shape(ctypes.Structure):
+    _fields_ = [("route", ctypes.c_int32), ("levels", ctypes.c_int32),
+                ("sum_blocks", ctypes.c_int64),
+                ("sum_capacity", ctypes.c_int64)]
+
+
 class HundunFlowError(RuntimeError):
     def __init__(self, what: str, status: hf_status):
         name = STATUS_NAMES[status.code] if 0 <= status.code < 8 else "?"
@@ -186,6 +195,9 @@ def load_library(path: str = LIBRARY_PATH):
         "hf_plan_level_count": [P, ctypes.POINTER(ctypes.c_int32)],
         "hf_plan_level_info": [P, ctypes.c_int32,
                                ctypes.POINTER(hf_level_info)],
+        "hf_launch_shape_of": [ctypes.POINTER(hf_grid_desc),
+                               ctypes.POINTER(hf_policy), ctypes.c_int32,
+                               ctypes.POINTER(hf_launch_shape)],
         "hf_plan_level_array": [P, ctypes.c_int32, ctypes.c_int32, D],
         "hf_plan_device_bytes": [P, ctypes.POINTER(ctypes.c_uint64)],
         "hf_plan_set_profiling": [P, ctypes.c_int32],
@@ -252,6 +264,30 @@ def _ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+def _grid_desc(n, faces, bc) -> hf_grid_desc:
+    """The C description of a grid; `faces` (float64 arrays) must outlive it."""
+    g = hf_grid_desc()
+    g.nx, g.ny, g.nz = n
+    g.faces_x, g.faces_y, g.faces_z = (
+        f.ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for f in faces)
+    for i, v in enumerate(bc):
+        g.boundary[i] = int(v)
+    return g
+
+
+def launch_shape(n, faces, bc, policy: hf_policy, level: int = 0) -> dict:
+    """How one level of such a plan runs (host arithmetic, no GPU)."""
+    lib = load_library()
+    faces = [np.ascontiguousarray(f, dtype=np.float64) for f in faces]
+    g = _grid_desc(tuple(int(v) for v in n), faces, bc)
+    s = hf_launch_shape()
+    _check("hf_launch_shape_of",
+           lib.hf_launch_shape_of(ctypes.byref(g), ctypes.byref(policy),
+                                  level, ctypes.byref(s)))
+    return dict(route=ROUTES[s.route], levels=s.levels,
+                sum_blocks=s.sum_blocks, sum_capacity=s.sum_capacity)
+
+
 class Plan:
     """A compiled hierarchy on one GPU (NativeCartesianMgPlan counterpart)."""
 
@@ -268,13 +304,7 @@ class Plan:
         if stream is None:
             stream = torch.cuda.current_stream()
         self.stream = stream
-        g = hf_grid_desc()
-        g.nx, g.ny, g.nz = self.n
-        g.faces_x = self.faces[0].ctypes.data_as(ctypes.POINTER(ctypes.c_double))
-        g.faces_y = self.faces[1].ctypes.data_as(ctypes.POINTER(ctypes.c_double))
-        g.faces_z = self.faces[2].ctypes.data_as(ctypes.POINTER(ctypes.c_double))
-        for i, v in enumerate(self.bc):
-            g.boundary[i] = int(v)
+        g = _grid_desc(self.n, self.faces, self.bc)
         handle = ctypes.c_void_p()
         _check("hf_plan_create",
                self.lib.hf_plan_create(ctypes.byref(g), ctypes.byref(self.policy),

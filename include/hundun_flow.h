@@ -179,6 +179,28 @@ typedef struct hf_level_info {
   uint8_t on_tail;      /* level handled by the single-workgroup tail */
 } hf_level_info;
 
+/* The kernels that smooth one level.  A march takes the visits of two sweeps
+ * or stages; other counts run by the sweep, the colour or the stage. */
+enum hf_route {
+  HF_ROUTE_TAIL = 0,    /* in the single-workgroup tail */
+  HF_ROUTE_LEG = 1,     /* a launch per way down and way up */
+  HF_ROUTE_MARCH = 2,   /* two red-black sweeps per launch */
+  HF_ROUTE_SWEEP = 3,   /* one red-black sweep per launch */
+  HF_ROUTE_COLOURS = 4, /* one colour per launch */
+  HF_ROUTE_SEPARATED = 5,   /* one colour, from the values before it */
+  HF_ROUTE_STAGE_MARCH = 6, /* two Chebyshev-Jacobi stages per launch */
+  HF_ROUTE_STAGES = 7,      /* one stage per launch */
+  HF_ROUTE_LINES = 8        /* line relaxation */
+};
+
+typedef struct hf_launch_shape {
+  int32_t route;        /* hf_route of the level */
+  int32_t levels;       /* of the plan */
+  int64_t sum_blocks;   /* the most block sums that a launch on the level
+                           makes, per accumulator */
+  int64_t sum_capacity; /* block sums that the plan holds per accumulator */
+} hf_launch_shape;
+
 typedef struct hf_plan hf_plan;
 
 /* Defaults of MgHierarchyPolicy (v04_linear.hpp:115-131), unit_linear,
@@ -350,6 +372,11 @@ hf_status hf_project_mean(hf_plan* plan, double* field);
 hf_status hf_plan_level_count(const hf_plan* plan, int32_t* levels);
 hf_status hf_plan_level_info(const hf_plan* plan, int32_t level,
                              hf_level_info* info);
+/* How level `level` of a plan with this grid and policy runs: host arithmetic
+ * alone, no device is needed or touched. */
+hf_status hf_launch_shape_of(const hf_grid_desc* grid,
+                             const hf_policy* policy, int32_t level,
+                             hf_launch_shape* shape);
 /* Copies one level array of the FP64 hierarchy to a device buffer:
  * which = 0 D, 1 x-faces, 2 y-faces, 3 z-faces, 4 fluid volume. */
 hf_status hf_plan_level_array(const hf_plan* plan, int32_t level,

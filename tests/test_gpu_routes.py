@@ -1,0 +1,71 @@
+"""GPU parity of the multigrid kernels route by route: every case asks the
+library which kernels its levels take and holds the cycle to the CPU oracle or
+to another route (bit for bit, or to 1e-12 where a mean is summed in another
+order)."""
+import sys
+
+import numpy as np
+import pytest
+
+import hf_cases
+import hf_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def _case(n, bc, seed, radius=0.2):
+    """A sphere case on an n grid with six boundary kinds."""
+    case = hf_cases.lognormal_sphere(n=n, seed=seed, radius=radius)
+    act = case["cell_active"].reshape(n[2], n[1], n[0])
+    fx, fy, fz = hf_cases.face_activity(act, bc)
+    case.update(bc=list(bc), x_active=fx, y_active=fy, z_active=fz)
+    return case
+
+
+def _plan(case, **policy):
+    import hundun_flow as H
+    return H.plan_from_case(case, H.default_policy(**policy))
+
+
+def _route(case, level=0, **policy):
+    import hundun_flow as H
+    return H.launch_shape(case["n"], case["faces"], case["bc"],
+                          H.default_policy(**policy), level)["route"]
+
+
+def _t(torch, a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+@pytest.mark.parametrize("n,policy", [
+    ((58, 9, 50), dict(pre_sweeps=3)),
+    ((58, 17, 42), dict(pre_sweeps=3)),
+    ((64, 12, 52), dict(f_cycle=1)),
+    ((64, 12, 64), dict(f_cycle=1)),
+])
+def test_slim_march_means(torch_cuda, n, policy):
+    """Closed domains on slim grids, whose last march sums a mean in more
+    blocks than the grid has plane tiles: the projected cycle equals the
+    oracle's to rounding, and the solve on the static scratch, which packs
+    the block sums, the plain one's bit for bit."""
+    torch = torch_cuda
+    _say(f"[slim march] n={n} policy={policy}")
+    case = _case(n, (1, 1, 1, 1, 2, 2), seed=61)
+    pol = dict(policy, anisotropy_threshold=1e9)
+    assert _route(case, **pol) == "march"
+    plan = _plan(case, **pol)
+    _, mg = O.from_case(case, O.policy(**pol))
+    b = _t(torch, case["rhs"])
+    z, zo = plan.mg_apply(b).cpu().numpy(), mg.apply(case["rhs"])
+    assert np.linalg.norm(z - zo) <= 1e-12 * np.linalg.norm(zo)
+    x, res = plan.solve_pcg(b, rtol=1e-9)
+    y, static = plan.solve_pcg(b, rtol=1e-9, static=True)
+    assert res.final_true_residual <= 1e-9 * res.rhs_norm
+    assert torch.equal(x, y)
+    assert static.iterations == res.iterations
+    plan.close()
