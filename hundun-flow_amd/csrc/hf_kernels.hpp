@@ -462,11 +462,11 @@ enum FinalOp : int {
 // accumulator a in index order.
 __global__ void k_fold_partials(const double* partials, int64_t blocks,
                                 int64_t stride, double* out,
-                                int64_t out_stride) {
+                                int64_t out_stride, int64_t span) {
   __shared__ double scratch[16];
   const int64_t a = blockIdx.y;
-  const int64_t lo = static_cast<int64_t>(blockIdx.x) * 2048;
-  const int64_t hi = lo + 2048 < blocks ? lo + 2048 : blocks;
+  const int64_t lo = static_cast<int64_t>(blockIdx.x) * span;
+  const int64_t hi = lo + span < blocks ? lo + span : blocks;
   double v = 0.0;
   for (int64_t b = lo + threadIdx.x; b < hi; b += blockDim.x)
     v += partials[a * stride + b];

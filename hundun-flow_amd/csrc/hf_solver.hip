@@ -140,6 +140,20 @@ constexpr int kFoldSpan = 2048;   // partials per block of the first fold
 constexpr int kFinalizeMost = 16384;  // partials that k_finalize folds alone
 constexpr int kFoldStride = 4096;  // capacity per accumulator of the fold
 
+// Partials per block of the first fold: more than kFoldSpan where that many
+// spans would pass the fold's capacity (over 8.4M partials: a plane of few
+// cells, a block each).
+int64_t fold_span(int64_t blocks) {
+  return std::max<int64_t>(kFoldSpan, (blocks + kFoldStride - 1) / kFoldStride);
+}
+
+// Blocks of the first fold (0: k_finalize folds alone).
+int64_t fold_blocks(int64_t blocks) {
+  if (blocks <= kFinalizeMost) return 0;
+  const int64_t span = fold_span(blocks);
+  return (blocks + span - 1) / span;
+}
+
 int ceil_log2(int v) {
   int l = 0;
   while ((1 << l) < v) ++l;
@@ -896,11 +910,12 @@ void finalize(hf_plan* p, int64_t blocks, int nacc, int op, int slot,
   int64_t stride = p->partial_stride;
   if (blocks > kFinalizeMost) {
     // first pass: fixed spans of partials summed in order (deterministic)
-    const int64_t spans = (blocks + kFoldSpan - 1) / kFoldSpan;
+    const int64_t spans = fold_blocks(blocks);
     hipLaunchKernelGGL(k_fold_partials, dim3(static_cast<uint32_t>(spans),
                                              static_cast<uint32_t>(nacc)),
                        dim3(kBlock), 0, p->stream, first, blocks,
-                       p->partial_stride, p->folded, kFoldStride);
+                       p->partial_stride, p->folded, kFoldStride,
+                       fold_span(blocks));
     src = p->folded;
     count = spans;
     stride = kFoldStride;
@@ -2087,7 +2102,8 @@ hf_status fgmres_impl(hf_plan* p, const double* rhs, double* solution,
                          dim3(static_cast<uint32_t>(spans),
                               static_cast<uint32_t>(nacc)),
                          dim3(kBlock), 0, p->stream, p->fg_partials, pst, pst,
-                         p->fg_folded, static_cast<int64_t>(kFoldStride));
+                         p->fg_folded, static_cast<int64_t>(kFoldStride),
+                         static_cast<int64_t>(kFoldSpan));
       src = p->fg_folded;
       count = spans;
       stride = kFoldStride;
@@ -3577,7 +3593,8 @@ hf_status hf_vector_dot(hf_vector_engine* e, int64_t n, const double* a,
     const int64_t spans = (blocks + kFoldSpan - 1) / kFoldSpan;
     hipLaunchKernelGGL(k_fold_partials, dim3(static_cast<uint32_t>(spans), 1),
                        dim3(kBlock), 0, e->stream, e->partials, blocks,
-                       blocks, e->folded, static_cast<int64_t>(kFoldStride));
+                       blocks, e->folded, static_cast<int64_t>(kFoldStride),
+                       static_cast<int64_t>(kFoldSpan));
     src = e->folded;
     count = spans;
   }
@@ -3722,6 +3739,8 @@ hf_status hf_launch_shape_of(const hf_grid_desc* grid, const hf_policy* policy,
     shape->levels = static_cast<int32_t>(p->levels.size());
     shape->sum_blocks = level_sum_blocks(p, static_cast<size_t>(level));
     shape->sum_capacity = p->partial_stride;
+    shape->fold_blocks = fold_blocks(shape->sum_blocks);
+    shape->fold_capacity = kFoldStride;
   }
   delete p;
   return s;

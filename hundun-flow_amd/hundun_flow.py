@@ -125,7 +125,9 @@ class hf_level_info(ctypes.Structure):
 class hf_launch_shape(ctypes.Structure):
     _fields_ = [("route", ctypes.c_int32), ("levels", ctypes.c_int32),
                 ("sum_blocks", ctypes.c_int64),
-                ("sum_capacity", ctypes.c_int64)]
+                ("sum_capacity", ctypes.c_int64),
+                ("fold_blocks", ctypes.c_int64),
+                ("fold_capacity", ctypes.c_int64)]
 
 
 class HundunFlowError(RuntimeError):
@@ -285,7 +287,8 @@ def launch_shape(n, faces, bc, policy: hf_policy, level: int = 0) -> dict:
            lib.hf_launch_shape_of(ctypes.byref(g), ctypes.byref(policy),
                                   level, ctypes.byref(s)))
     return dict(route=ROUTES[s.route], levels=s.levels,
-                sum_blocks=s.sum_blocks, sum_capacity=s.sum_capacity)
+                sum_blocks=s.sum_blocks, sum_capacity=s.sum_capacity,
+                fold_blocks=s.fold_blocks, fold_capacity=s.fold_capacity)
 
 
 class Plan:

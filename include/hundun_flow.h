@@ -199,6 +199,8 @@ typedef struct hf_launch_shape {
   int64_t sum_blocks;   /* the most block sums that a launch on the level
                            makes, per accumulator */
   int64_t sum_capacity; /* block sums that the plan holds per accumulator */
+  int64_t fold_blocks;  /* folded sums of these (0: folded in one launch) */
+  int64_t fold_capacity; /* folded sums that the plan holds */
 } hf_launch_shape;
 
 typedef struct hf_plan hf_plan;

@@ -69,3 +69,27 @@ def test_slim_march_means(torch_cuda, n, policy):
     assert torch.equal(x, y)
     assert static.iterations == res.iterations
     plan.close()
+
+
+def test_sums_of_single_cell_planes(torch_cuda):
+    """A grid of nine million planes of one cell: the residual's norm and the
+    entry's mean, two accumulators of a block sum per plane, are folded apart
+    (the norm to 1e-12 of torch's)."""
+    import hundun_flow as H
+    torch = torch_cuda
+    n = (1, 1, 9_000_000)
+    _say(f"[single-cell planes] n={n}")
+    faces = [np.linspace(0.0, 1.0, v + 1) for v in n[:2]]
+    faces.append(np.linspace(0.0, float(n[2]), n[2] + 1))
+    plan = H.Plan(n, faces, (1,) * 6, H.default_policy(
+        anisotropy_threshold=1e9))
+    plan.set_coefficients(*plan.assemble(
+        torch.ones(n[2], dtype=torch.float64, device="cuda")))
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    b = torch.randn(n[2], dtype=torch.float64, device="cuda", generator=gen)
+    b -= b.mean()
+    _, res = plan.solve_pcg(b, rtol=1e-10, maximum_iterations=1, check=False)
+    norm = torch.linalg.vector_norm(b).item()
+    assert abs(res.rhs_norm - norm) <= 1e-12 * norm
+    assert abs(res.initial_true_residual - norm) <= 1e-12 * norm
+    plan.close()

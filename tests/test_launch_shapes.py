@@ -66,6 +66,15 @@ def test_block_sums_fit_everywhere(monkeypatch, precision, env):
     assert {"march", "tail"} <= routes
 
 
+@pytest.mark.parametrize("n", [(1, 1, 9_000_000), (1, 2, 8_388_609),
+                               (512, 512, 512)])
+def test_folded_sums_fit(n):
+    """The first fold's spans grow where spans of the usual length would be
+    more than its buffer holds: a plane of few cells takes a block each."""
+    s = _shape(n)
+    assert 0 < s["fold_blocks"] <= s["fold_capacity"]
+
+
 @pytest.mark.parametrize("n", [(0, 4, 4), (2147483647, 1, 1)])
 def test_shape_of_a_refused_grid(n):
     """A grid that no plan takes has no shape either."""
