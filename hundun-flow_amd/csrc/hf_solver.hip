@@ -3018,11 +3018,15 @@ hf_status hf_plan_set_coefficients(hf_plan* p, const double* diag,
 // taken); returns their number.  Rows of whole 64-pair tiles on a level that
 // streams from memory run as pairs in tiles (k_fg_stencil2; 166 us against
 // 176 at 256^3, 318 against 338 at 512x256x256), the others as k_rows
-// (256x256x128 81 us against 83, 400x160x240 158 against 168).
+// (256x256x128 81 us against 83, 400x160x240 158 against 168), and so do a
+// caller's arrays that are not aligned as a pair (the tiles' pairs are
+// 16-byte accesses, k_rows asks for one element's alignment).
 static int64_t operator_pass(hf_plan* p, const double* x, double* y,
                              double* partials) {
   const Level& L = p->levels[0];
-  if (!p->krylov_pairs || L.n[0] % 128 != 0 ||
+  const bool aligned = ((reinterpret_cast<uintptr_t>(x) |
+                         reinterpret_cast<uintptr_t>(y)) & 15) == 0;
+  if (!p->krylov_pairs || !aligned || L.n[0] % 128 != 0 ||
       L.cells < (int64_t{12} << 20)) {
     RowsArgs<double, double> a = rows_args<double>(krylov_view(p), x, y);
     a.partials = partials;

@@ -93,3 +93,30 @@ def test_sums_of_single_cell_planes(torch_cuda):
     assert abs(res.rhs_norm - norm) <= 1e-12 * norm
     assert abs(res.initial_true_residual - norm) <= 1e-12 * norm
     plan.close()
+
+
+def test_operator_on_unaligned_arrays(torch_cuda):
+    """A x of the smallest grid whose operator runs over aligned pairs in
+    tiles, on arrays that begin in the middle of a pair: bit for bit that of
+    aligned ones."""
+    import hundun_flow as H
+    torch = torch_cuda
+    n = (256, 256, 192)
+    _say(f"[unaligned operator] n={n}")
+    cells = n[0] * n[1] * n[2]
+    faces = [np.linspace(0.0, 1.0, v + 1) for v in n]
+    plan = H.Plan(n, faces, (1, 1, 0, 1, 2, 2))
+    gen = torch.Generator(device="cuda").manual_seed(5)
+
+    def normal(count):
+        return torch.randn(count, dtype=torch.float64, device="cuda",
+                           generator=gen)
+    plan.set_coefficients(*plan.assemble(normal(cells).exp()))
+    x = normal(cells + 1)[1:]
+    y = torch.empty(cells + 1, dtype=torch.float64, device="cuda")[1:]
+    assert x.data_ptr() % 16 == 8 and y.data_ptr() % 16 == 8
+    aligned = plan.operator_apply(x.clone())
+    plan.operator_apply(x, out=y)
+    assert torch.equal(y, aligned)
+    assert torch.equal(plan.operator_apply(x), aligned)
+    plan.close()
