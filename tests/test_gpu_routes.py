@@ -120,3 +120,147 @@ def test_operator_on_unaligned_arrays(torch_cuda):
     assert torch.equal(y, aligned)
     assert torch.equal(plan.operator_apply(x), aligned)
     plan.close()
+
+
+_GRID_LEVELS = {"HF_TAIL_CELLS": "0", "HF_LEG_CELLS": "0",
+                "HF_SWEEP_MIN_CELLS": "0"}
+# smoothing of the finest level by two sweeps, by one and by one colour a
+# launch
+_RED_BLACK = {"march": {},
+              "sweep": {"HF_SWEEP_MARCH": "0"},
+              "colours": {"HF_SWEEP_MARCH": "0", "HF_FUSED_SWEEP": "0"}}
+
+
+def _cycle_on(torch, monkeypatch, env, case, r, **policy):
+    """The cycle of a plan made under `env`, and the finest level's route."""
+    with monkeypatch.context() as m:
+        for k, v in {**_GRID_LEVELS, **env}.items():
+            m.setenv(k, v)
+        route = _route(case, **policy)
+        plan = _plan(case, **policy)
+        z = plan.mg_apply(_t(torch, r)).cpu().numpy()
+        plan.close()
+    return z, route
+
+
+MARCH_GRIDS = [
+    ((32, 8, 8), (0, 0, 1, 1, 2, 2)),      # the smallest grid it takes
+    ((56, 24, 9), (1, 1, 0, 1, 1, 0)),     # one FP32 tile, three FP64 ones
+    ((58, 25, 10), (2, 2, 1, 0, 2, 2)),    # a partial tile of two columns
+    ((114, 18, 12), (0, 1, 2, 2, 1, 1)),   # wrapped rows, walls in z
+    ((64, 40, 36), (1, 1, 1, 1, 1, 1)),    # a coarse level that marches too
+]
+
+
+@pytest.mark.parametrize("zc", ["", "1", "5"])
+@pytest.mark.parametrize("n,bc", MARCH_GRIDS)
+def test_red_black_routes(torch_cuda, monkeypatch, n, bc, zc):
+    """V(2,2) cycles by marches, sweeps and colours, with the tail and the
+    legs out of the way, on tile and chunk edges and every boundary kind: one
+    result in every storage type, in FP64 the oracle's."""
+    torch = torch_cuda
+    _say(f"[red-black] n={n} bc={bc} zc={zc or 'planned'}")
+    case = _case(n, bc, seed=23)
+    pol = dict(null_space_constant=0, anisotropy_threshold=64.0)
+    _, mg = O.from_case(case, O.policy(**pol))
+    r = np.random.default_rng(17).standard_normal(n[0] * n[1] * n[2])
+    zo = mg.apply(r)
+    for precision in ("fp64", "fp32", "bf16"):
+        first = None
+        for name, env in _RED_BLACK.items():
+            z, route = _cycle_on(torch, monkeypatch, {
+                **env, **({"HF_SWEEP_ZC": zc} if zc else {})}, case, r,
+                precision=precision, **pol)
+            assert route == name
+            first = z if first is None else first
+            assert np.array_equal(z, first), (precision, name)
+        if precision == "fp64":
+            assert np.array_equal(first, zo)
+
+
+@pytest.mark.parametrize("unit_linear", [1, 0])
+@pytest.mark.parametrize("f_cycle", [0, 1])
+@pytest.mark.parametrize("n,bc", MARCH_GRIDS)
+def test_red_black_routes_projected(torch_cuda, monkeypatch, n, bc, f_cycle,
+                                    unit_linear):
+    """The same cycles with the constant null space, whose means the marches
+    and sweeps take from and leave to other launches: 1e-12 of the oracle."""
+    torch = torch_cuda
+    _say(f"[red-black means] n={n} bc={bc} f={f_cycle} unit={unit_linear}")
+    case = _case(n, bc, seed=23)
+    pol = dict(anisotropy_threshold=64.0, f_cycle=f_cycle,
+               unit_linear=unit_linear)
+    _, mg = O.from_case(case, O.policy(**pol))
+    zo = mg.apply(case["rhs"])
+    for name, env in _RED_BLACK.items():
+        z, route = _cycle_on(torch, monkeypatch, env, case, case["rhs"], **pol)
+        assert route == name
+        assert np.linalg.norm(z - zo) <= 1e-12 * np.linalg.norm(zo), name
+
+
+@pytest.mark.parametrize("sweeps", [(1, 1), (1, 2), (2, 1), (3, 2), (2, 3),
+                                    (4, 4)])
+@pytest.mark.parametrize("n,route", [((66, 20, 10), "march"),
+                                     ((66, 20, 6), "sweep")])
+def test_sweep_counts(torch_cuda, monkeypatch, n, route, sweeps):
+    """Smoothings that march and smoothings that cannot (other counts than
+    two, too few planes) in one cycle: bit for bit the colour passes and, in
+    FP64, the oracle; projected to 1e-12 of it."""
+    torch = torch_cuda
+    _say(f"[sweep counts] n={n} sweeps={sweeps}")
+    case = _case(n, (1, 1, 1, 1, 2, 2), seed=29)
+    pol = dict(null_space_constant=0, anisotropy_threshold=64.0,
+               pre_sweeps=sweeps[0], post_sweeps=sweeps[1])
+    _, mg = O.from_case(case, O.policy(**pol))
+    r = np.random.default_rng(31).standard_normal(n[0] * n[1] * n[2])
+    zo = mg.apply(r)
+    for precision in ("fp64", "fp32", "bf16"):
+        z, got = _cycle_on(torch, monkeypatch, {}, case, r,
+                           precision=precision, **pol)
+        assert got == route
+        c, got = _cycle_on(torch, monkeypatch, _RED_BLACK["colours"], case, r,
+                           precision=precision, **pol)
+        assert got == "colours"
+        assert np.array_equal(z, c), precision
+        if precision == "fp64":
+            assert np.array_equal(z, zo)
+    pol["null_space_constant"] = 1
+    _, mg = O.from_case(case, O.policy(**pol))
+    zo = mg.apply(case["rhs"])
+    z, _ = _cycle_on(torch, monkeypatch, {}, case, case["rhs"], **pol)
+    assert np.linalg.norm(z - zo) <= 1e-12 * np.linalg.norm(zo)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16"])
+@pytest.mark.parametrize("smoother", ["red_black", "chebyshev"])
+@pytest.mark.parametrize("n,bc", [
+    ((32, 32, 32), (1, 1, 1, 1, 2, 2)),
+    ((128, 16, 8), (1, 1, 0, 1, 2, 2)),
+    ((34, 10, 14), (2, 2, 2, 2, 0, 1)),    # a wavefront's rows partly full
+])
+def test_defect_restriction_routes(torch_cuda, monkeypatch, n, bc, smoother,
+                                   precision):
+    """The retained defect and its restriction in one launch and in two, on
+    levels that neither the tail nor a leg takes: one result, and the single
+    launch seen to be taken."""
+    torch = torch_cuda
+    _say(f"[defect, restriction] n={n} {smoother} {precision}")
+    case = _case(n, bc, seed=37)
+    pol = dict(null_space_constant=0, anisotropy_threshold=64.0,
+               precision=precision)
+    if smoother == "chebyshev":
+        pol.update(point_smoother=1, f_cycle=1, pre_sweeps=1, post_sweeps=2)
+    z, launches = {}, {}
+    for fused in ("1", "0"):
+        with monkeypatch.context() as m:
+            for k, v in {**_GRID_LEVELS, "HF_DEFECT_RESTRICT": fused}.items():
+                m.setenv(k, v)
+            plan = _plan(case, **pol)
+        r = _t(torch, case["rhs"])
+        z[fused] = plan.mg_apply(r).cpu().numpy()
+        plan.set_profiling(True)
+        plan.solve_pcg(r, maximum_iterations=1, check=False)
+        launches[fused] = plan.profile()["restrict"][1]
+        plan.close()
+    assert launches["1"] < launches["0"]
+    assert np.array_equal(z["1"], z["0"])
