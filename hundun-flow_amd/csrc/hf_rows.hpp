@@ -26,7 +26,8 @@ namespace hf {
 // the high element (kLine, nx = 1: there is none, the elements are read one
 // by one), so every access stays inside the row, and no access needs more
 // than the alignment of one element.  All loads of the planes are issued
-// before the first use.
+// before the first use.  Planes of at most half a block of pairs lie several
+// to a block (kRowsPacked), one to a lane.
 //
 // What bounds it: the streams themselves.  A x, FP64, against one cell per
 // lane in 64-wide tiles: 201x149x97 22.3 us against 29.5, 143x101x75 10.6
@@ -82,17 +83,34 @@ struct RowsArgs {
   int colour;        // kRowsColour
   int pairs;         // of a row: (nx + 1) / 2
   int per_plane;     // blocks of a plane
+  int packed;        // planes side by side in a block (then per_plane = 1)
 };
 
-template <class T, int kMode, int kPer, bool kLine, class Te = T>
+// Planes of many pairs; planes of few, side by side in a block; rows of one
+// cell (either).
+constexpr int kRowsWide = 0, kRowsPacked = 1, kRowsLine = 2;
+
+template <class T, int kMode, int kPer, int kPlane, class Te = T>
 __global__ void __launch_bounds__(kBlock) k_rows(RowsArgs<T, Te> a) {
   using C = typename Compute<T>::type;
+  constexpr bool kLine = kPlane == kRowsLine;
   __shared__ double scratch[16];
   const Lv<T>& L = a.L;
   const int nx = L.nx, ny = L.ny, nz = L.nz;
   const int lb = xcd_block32(blockIdx.x, gridDim.x);
-  const int zb = lb / a.per_plane;
-  const int q = (lb - zb * a.per_plane) * kBlock + static_cast<int>(threadIdx.x);
+  int zb, q;
+  if (kPlane != kRowsWide && a.packed > 1) {
+    const int lanes = a.pairs * ny;
+    const int side = static_cast<int>(threadIdx.x) / lanes;
+    zb = lb * a.packed + side;
+    q = side < a.packed && static_cast<uint32_t>(zb) <=
+                                static_cast<uint32_t>((nz - 1) / kPer)
+            ? static_cast<int>(threadIdx.x) - side * lanes
+            : lanes;  // (no pair)
+  } else {
+    zb = lb / a.per_plane;
+    q = (lb - zb * a.per_plane) * kBlock + static_cast<int>(threadIdx.x);
+  }
   double dot = 0.0, mean = 0.0, bb = 0.0;
   if (q < a.pairs * ny) {
     const int j = q / a.pairs;

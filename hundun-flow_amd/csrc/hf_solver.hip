@@ -786,21 +786,26 @@ bool leg_ok(const hf_plan* p, int l) {
 // them; with one plane per block a level that stays in the last-level cache
 // is faster (A x in FP64, 1 and 2 planes: 201x149x97 22.3 and 25.3 us,
 // 192x192x128 33.9 and 37.5, 300x180x140 77 and 74, 511x255x255 376 and 347).
+// Planes that fit into half a block or less are dealt several to one (a block
+// per plane: 1x1x10^6 478 us, 3x3x50000 29; packed 10.9 and 5.4).
 struct RowsShape {
   int pairs, per_plane;
-  int per;  // planes per block
+  int per;     // planes of a lane
+  int packed;  // planes side by side in a block
   int64_t blocks;
 };
 
 RowsShape rows_shape(int nx, int ny, int nz, size_t elem) {
   RowsShape r{};
   r.pairs = (nx + 1) / 2;
-  r.per_plane =
-      static_cast<int>(blocks_for(static_cast<int64_t>(r.pairs) * ny));
+  const int64_t lanes = static_cast<int64_t>(r.pairs) * ny;
+  r.per_plane = static_cast<int>(blocks_for(lanes));
+  r.packed = static_cast<int>(std::max<int64_t>(1, kBlock / lanes));
   const bool cached = static_cast<int64_t>(nx) * ny * nz *
                           static_cast<int64_t>(elem) < (48ll << 20);
-  r.per = cached || nx == 1 ? 1 : 2;
-  r.blocks = static_cast<int64_t>(r.per_plane) * ((nz + r.per - 1) / r.per);
+  r.per = cached || nx == 1 || r.packed > 1 ? 1 : 2;
+  const int64_t deep = (nz + r.per - 1) / r.per;
+  r.blocks = r.per_plane * ((deep + r.packed - 1) / r.packed);
   return r;
 }
 
@@ -1035,15 +1040,22 @@ int64_t rows_pass(hf_plan* p, RowsArgs<T, Te> a) {
   a.bc = p->bc;
   a.pairs = r.pairs;
   a.per_plane = r.per_plane;
+  a.packed = r.packed;
+  auto launch = [&](auto per, auto plane) {
+    HF_LAUNCH((k_rows<T, kMode, decltype(per)::value, decltype(plane)::value,
+                      Te>),
+              r.blocks, kBlock, 0, p->stream, a);
+  };
+  using One = std::integral_constant<int, 1>;
   if (v.nx == 1)
-    HF_LAUNCH((k_rows<T, kMode, 1, true, Te>), r.blocks, kBlock, 0, p->stream,
-              a);
+    launch(One{}, std::integral_constant<int, kRowsLine>{});
+  else if (r.packed > 1)
+    launch(One{}, std::integral_constant<int, kRowsPacked>{});
   else if (r.per == 1)
-    HF_LAUNCH((k_rows<T, kMode, 1, false, Te>), r.blocks, kBlock, 0, p->stream,
-              a);
+    launch(One{}, std::integral_constant<int, kRowsWide>{});
   else
-    HF_LAUNCH((k_rows<T, kMode, 2, false, Te>), r.blocks, kBlock, 0, p->stream,
-              a);
+    launch(std::integral_constant<int, 2>{},
+           std::integral_constant<int, kRowsWide>{});
   return r.blocks;
 }
 

@@ -72,9 +72,9 @@ def test_slim_march_means(torch_cuda, n, policy):
 
 
 def test_sums_of_single_cell_planes(torch_cuda):
-    """A grid of nine million planes of one cell: the residual's norm and the
-    entry's mean, two accumulators of a block sum per plane, are folded apart
-    (the norm to 1e-12 of torch's)."""
+    """A grid of nine million planes of one cell: the norms of the right-hand
+    side and the residual, folded with the entry's mean (to 1e-12 of
+    torch's)."""
     import hundun_flow as H
     torch = torch_cuda
     n = (1, 1, 9_000_000)
@@ -91,6 +91,47 @@ def test_sums_of_single_cell_planes(torch_cuda):
     _, res = plan.solve_pcg(b, rtol=1e-10, maximum_iterations=1, check=False)
     norm = torch.linalg.vector_norm(b).item()
     assert abs(res.rhs_norm - norm) <= 1e-12 * norm
+    assert abs(res.initial_true_residual - norm) <= 1e-12 * norm
+    plan.close()
+
+
+@pytest.mark.parametrize("n", [(3, 4, 600_001),   # two planes to a lane
+                               (1, 7, 100_003),   # rows of one cell
+                               (16, 15, 501),     # two planes to a block
+                               (16, 17, 500)])    # one, half a block
+def test_operator_on_planes_of_few_cells(torch_cuda, n):
+    """A x where a block holds several planes: bit for bit the same sums of
+    products by torch, whose elementwise operations round one by one."""
+    import hundun_flow as H
+    torch = torch_cuda
+    _say(f"[planes of few cells] n={n}")
+    nx, ny, nz = n
+    faces = [np.linspace(0.0, v / 8.0, v + 1) for v in n]
+    plan = H.Plan(n, faces, (1,) * 6, H.default_policy(
+        anisotropy_threshold=1e9))
+    gen = torch.Generator(device="cuda").manual_seed(7)
+
+    def normal():
+        return torch.randn(nx * ny * nz, dtype=torch.float64, device="cuda",
+                           generator=gen)
+    d, bx, by, bz = plan.assemble(normal().exp())
+    plan.set_coefficients(d, bx, by, bz)
+    x = normal()
+    y = plan.operator_apply(x)
+    v = x.view(nz, ny, nx)
+    ref = d.view(nz, ny, nx) * v
+    for dim, f in ((2, bx.view(nz, ny, nx + 1)), (1, by.view(nz, ny + 1, nx)),
+                   (0, bz.view(nz + 1, ny, nx))):
+        m = v.shape[dim]  # a wall's neighbour is the cell itself
+        first, last = v.narrow(dim, 0, 1), v.narrow(dim, m - 1, 1)
+        low = torch.cat([first, v.narrow(dim, 0, m - 1)], dim)
+        high = torch.cat([v.narrow(dim, 1, m - 1), last], dim)
+        ref = ref - f.narrow(dim, 0, m) * low
+        ref = ref - f.narrow(dim, 1, m) * high
+    assert torch.equal(y.view(nz, ny, nx), ref)
+    b = x - x.mean()
+    _, res = plan.solve_pcg(b, maximum_iterations=1, check=False)
+    norm = torch.linalg.vector_norm(b).item()
     assert abs(res.initial_true_residual - norm) <= 1e-12 * norm
     plan.close()
 
