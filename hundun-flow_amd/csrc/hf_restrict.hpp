@@ -11,8 +11,8 @@ namespace hf {
 // every axis.  A lane owns a coarse cell: the pairs of two rows on two
 // planes, whose defects, rounded to the fine storage type, it adds in the
 // order of k_restrict (dz, dy, dx); the fine r is not stored.  Lanes take the
-// cells of a coarse plane row after row and march through a.per coarse
-// planes, carrying x and the z faces.  zero_x and partials as in k_restrict.
+// cells of a coarse plane row after row and go through its two fine planes,
+// carrying x and the z faces.  zero_x and partials as in k_restrict.
 //
 // kFirstStage: the level was to be smoothed by one Chebyshev-Jacobi stage
 // from x = 0 (the pre-smoothing of a from-zero visit), which is not run:
@@ -23,11 +23,12 @@ namespace hf {
 // of a plane.
 //
 // What bounds it: the streams.  Against one fine cell per lane with the
-// children's defects passed through LDS: 256^3 FP32 92 us against 107, 128^3
-// 10.6 against 13.0, 512x256x256 184 against 204; with the first stage, which
-// paid on FP32 levels only below 2^20 cells (five divisions a cell), 256^3
-// FP32 113 against 139 for stage and defect apart, 512x256x256 210 against
-// 265, FP64 399 against 430; 64^3 FP64 5.7 against 7.5.
+// children's defects passed through LDS: 256^3 FP32 95 us against 107, 128^3
+// 10.4 against 13.0, 512x256x256 186 against 204, 128^3 FP64 18.8 against
+// 19.5, 64^3 FP64 4.9 against 5.4; with the first stage, which paid on FP32
+// levels only below 2^20 cells (five divisions a cell), 256^3 FP32 112 against
+// 139 for stage and defect apart, 512x256x256 216 against 265, FP64 403
+// against 430; 64^3 FP64 6.2 against 7.5.
 // ---------------------------------------------------------------------------
 template <class Tf, class Tc>
 struct DefectArgs {
@@ -38,12 +39,21 @@ struct DefectArgs {
   double* partials;
   typename Compute<Tf>::type rf0;
   Tf* xs;
-  int per;        // coarse planes per block
   int per_plane;  // blocks of a coarse plane
 };
 
+// Wavefronts per SIMD that the registers are to leave room for.  Left to
+// itself the compiler fits six FP64 ones, with few loads of each in flight;
+// four with more are faster (64^3 4.9 us against 6.6, 128^3 18.8 against 22.3,
+// 512x256x256 333 against 352).  In FP32 its own seven are as good.
+template <class Tf>
+constexpr int kDefectWavesLow = sizeof(Tf) == 8 ? 4 : 1;
+template <class Tf>
+constexpr int kDefectWavesHigh = sizeof(Tf) == 8 ? 4 : 8;
+
 template <class Tf, class Tc, bool kFirstStage>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kBlock) __attribute__((
+    amdgpu_waves_per_eu(kDefectWavesLow<Tf>, kDefectWavesHigh<Tf>)))
 k_defect_restrict(DefectArgs<Tf, Tc> a) {
   using C = typename Compute<Tf>::type;
   using Cc = typename Compute<Tc>::type;
@@ -101,8 +111,7 @@ k_defect_restrict(DefectArgs<Tf, Tc> a) {
       else
         return C(ld(L.x[c]));
     };
-    const int k0 = 2 * zb * a.per;
-    const int k1 = min(nz, k0 + 2 * a.per);
+    const int k0 = 2 * zb;
     int c = k0 * plane + at;
     const int low_z = k0 > 0 ? c - plane : c + (nz - 1) * plane;
     Two xc[2], zl[2], fzl[2];
@@ -116,75 +125,73 @@ k_defect_restrict(DefectArgs<Tf, Tc> a) {
         zl[r].v[1] = nb(a.bc.m[4], xc[r].v[1], zl[r].v[1]);
       }
     }
-    for (int k = k0; k < k1; k += 2) {
-      Cc sum = Cc(0);
+    Cc sum = Cc(0);
 #pragma unroll
-      for (int dz = 0; dz < 2; ++dz) {
-        const int kk = k + dz;
-        const bool top = kk + 1 == nz;
-        const int up = top ? at : c + plane;
-        const Two below = x2(yl_at + kk * plane), beyond = x2(yh_at + kk * plane);
-        Two zh[2], fzh[2], d[2], b[2], fy[3], fx[2];
-        C fx2[2], xl[2], xh[2];
+    for (int dz = 0; dz < 2; ++dz) {
+      const int kk = k0 + dz;
+      const bool top = kk + 1 == nz;
+      const int up = top ? at : c + plane;
+      const Two below = x2(yl_at + kk * plane), beyond = x2(yh_at + kk * plane);
+      Two zh[2], fzh[2], d[2], b[2], fy[3], fx[2];
+      C fx2[2], xl[2], xh[2];
 #pragma unroll
-        for (int r = 0; r < 3; ++r)
-          fy[r] = load(L.fy + (c + kk * nx + r * nx));
+      for (int r = 0; r < 3; ++r)
+        fy[r] = load(L.fy + (c + kk * nx + r * nx));
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
-          zh[r] = x2(up + r * nx);
-          fzh[r] = load(L.fz + (c + plane + r * nx));
-          d[r] = load(L.D + (c + r * nx));
-          b[r] = load(L.b + (c + r * nx));
-          const Tf* const face = L.fx + (c + kk * ny + j0 + r * (nx + 1));
-          const RowsPair<Tf> f = rows_load(face);
-          fx[r] = {{C(ld(f.v[0])), C(ld(f.v[1]))}};
-          fx2[r] = C(ld(face[2]));
-          xl[r] = x1(xl_at + kk * plane + r * nx);
-          xh[r] = x1(xh_at + kk * plane + r * nx);
-        }
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-          if constexpr (kFirstStage)
-            *reinterpret_cast<Stored*>(a.xs + (c + r * nx)) = {
-                {st<Tf>(xc[r].v[0]), st<Tf>(xc[r].v[1])}};
-          if (top) {
-            zh[r].v[0] = nb(a.bc.m[5], xc[r].v[0], zh[r].v[0]);
-            zh[r].v[1] = nb(a.bc.m[5], xc[r].v[1], zh[r].v[1]);
-          }
-          const C nl[2] = {nb(mxl, xc[r].v[0], xl[r]), xc[r].v[0]};
-          const C nh[2] = {xc[r].v[1], nb(mxh, xc[r].v[1], xh[r])};
-          const C fl[2] = {fx[r].v[0], fx[r].v[1]};
-          const C fh[2] = {fx[r].v[1], fx2[r]};
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const C self = xc[r].v[e];
-            const C yl = r == 0 ? nb(myl, self, below.v[e]) : xc[0].v[e];
-            const C yh = r == 0 ? xc[1].v[e] : nb(myh, self, beyond.v[e]);
-            C v = d[r].v[e] * self;
-            v -= fl[e] * nl[e];
-            v -= fh[e] * nh[e];
-            v -= fy[r].v[e] * yl;
-            v -= fy[r + 1].v[e] * yh;
-            v -= fzl[r].v[e] * zl[r].v[e];
-            v -= fzh[r].v[e] * zh[r].v[e];
-            sum += Cc(ld(st<Tf>(b[r].v[e] - v)));
-          }
-        }
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-          zl[r] = xc[r];
-          xc[r] = zh[r];
-          fzl[r] = fzh[r];
-        }
-        c += plane;
+      for (int r = 0; r < 2; ++r) {
+        zh[r] = x2(up + r * nx);
+        fzh[r] = load(L.fz + (c + plane + r * nx));
+        d[r] = load(L.D + (c + r * nx));
+        b[r] = load(L.b + (c + r * nx));
+        const Tf* const face = L.fx + (c + kk * ny + j0 + r * (nx + 1));
+        const RowsPair<Tf> f = rows_load(face);
+        fx[r] = {{C(ld(f.v[0])), C(ld(f.v[1]))}};
+        fx2[r] = C(ld(face[2]));
+        xl[r] = x1(xl_at + kk * plane + r * nx);
+        xh[r] = x1(xh_at + kk * plane + r * nx);
       }
-      const int cc = (k >> 1) * Cl.nx * Cl.ny + q;
-      const Tc stored = st<Tc>(sum);
-      Cl.b[cc] = stored;
-      if (a.zero_x) Cl.x[cc] = st<Tc>(0.0);
-      if (a.partials != nullptr)
-        pv += Cl.vol[cc] * static_cast<double>(ld(stored));
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        if constexpr (kFirstStage)
+          *reinterpret_cast<Stored*>(a.xs + (c + r * nx)) = {
+              {st<Tf>(xc[r].v[0]), st<Tf>(xc[r].v[1])}};
+        if (top) {
+          zh[r].v[0] = nb(a.bc.m[5], xc[r].v[0], zh[r].v[0]);
+          zh[r].v[1] = nb(a.bc.m[5], xc[r].v[1], zh[r].v[1]);
+        }
+        const C nl[2] = {nb(mxl, xc[r].v[0], xl[r]), xc[r].v[0]};
+        const C nh[2] = {xc[r].v[1], nb(mxh, xc[r].v[1], xh[r])};
+        const C fl[2] = {fx[r].v[0], fx[r].v[1]};
+        const C fh[2] = {fx[r].v[1], fx2[r]};
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const C self = xc[r].v[e];
+          const C yl = r == 0 ? nb(myl, self, below.v[e]) : xc[0].v[e];
+          const C yh = r == 0 ? xc[1].v[e] : nb(myh, self, beyond.v[e]);
+          C v = d[r].v[e] * self;
+          v -= fl[e] * nl[e];
+          v -= fh[e] * nh[e];
+          v -= fy[r].v[e] * yl;
+          v -= fy[r + 1].v[e] * yh;
+          v -= fzl[r].v[e] * zl[r].v[e];
+          v -= fzh[r].v[e] * zh[r].v[e];
+          sum += Cc(ld(st<Tf>(b[r].v[e] - v)));
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        zl[r] = xc[r];
+        xc[r] = zh[r];
+        fzl[r] = fzh[r];
+      }
+      c += plane;
     }
+    const int cc = zb * Cl.nx * Cl.ny + q;
+    const Tc stored = st<Tc>(sum);
+    Cl.b[cc] = stored;
+    if (a.zero_x) Cl.x[cc] = st<Tc>(0.0);
+    if (a.partials != nullptr)
+      pv = Cl.vol[cc] * static_cast<double>(ld(stored));
   }
   if (a.partials != nullptr) {
     pv = block_sum(pv, scratch);

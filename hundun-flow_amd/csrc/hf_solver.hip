@@ -809,23 +809,23 @@ RowsShape rows_shape(int nx, int ny, int nz, size_t elem) {
   return r;
 }
 
-// Blocks of k_defect_restrict on level L with the coarse level Cd.  Two
-// coarse planes per block share their rows of x (256^3 FP32 113 us against
-// 117), one fills the chip with more blocks (128^3 10.6 against 12.9); a
-// level with too few cells even so takes blocks of one wavefront.
+// Blocks of k_defect_restrict onto the coarse level Cd.  A coarse plane per
+// block: two, sharing a row of x, measured the same from 320^3 on (cycles 0.3%
+// faster to 1.3% slower) and slower below (128^3 FP32 240 us against 234,
+// 256x256x128 518 against 507).  A level with too few cells to fill the chip
+// takes blocks of one wavefront (cycles in FP32, 64 and 256 threads: 48^3
+// 114.9 and 116.7 us, 80^3 161.8 and 163.4, 96^3 180.7 and 181.0).
 struct RestrictShape {
-  int threads, per, per_plane;
+  int threads, per_plane;
   int64_t blocks;
 };
 
-RestrictShape restrict_shape(const Level& L, const Level& Cd) {
+RestrictShape restrict_shape(const Level& Cd) {
   RestrictShape r{};
-  r.per = L.cells >= (int64_t{1} << 24) ? 2 : 1;
   r.threads = Cd.cells < (int64_t{1} << 16) ? kWave : kBlock;
   r.per_plane = static_cast<int>(
       (static_cast<int64_t>(Cd.n[0]) * Cd.n[1] + r.threads - 1) / r.threads);
-  r.blocks =
-      static_cast<int64_t>(r.per_plane) * ((Cd.n[2] + r.per - 1) / r.per);
+  r.blocks = static_cast<int64_t>(r.per_plane) * Cd.n[2];
   return r;
 }
 
@@ -842,7 +842,7 @@ int64_t level_sum_blocks(const hf_plan* p, size_t l) {
   if (L.march) most = std::max<int64_t>(most, L.march_blocks);
   if (L.leg) most = std::max(most, leg_boxes(L, kLegHalo).blocks);
   if (defect_restrict_ok(p, static_cast<int>(l)))
-    most = std::max(most, restrict_shape(L, p->levels[l + 1]).blocks);
+    most = std::max(most, restrict_shape(p->levels[l + 1]).blocks);
   if (l == 0)
     most = std::max<int64_t>(
         {most, rows_shape(L.n[0], L.n[1], L.n[2], sizeof(double)).blocks,
@@ -1514,8 +1514,7 @@ void exec_grid_op(hf_plan* p, const CycleOp& op,
         a.Cl = view<Tc>(Cd);
         a.zero_x = stored ? 1 : 0;
         a.partials = proj ? mean_partials_of(p, op.level + 1) : nullptr;
-        const RestrictShape shape = restrict_shape(L, Cd);
-        a.per = shape.per;
+        const RestrictShape shape = restrict_shape(Cd);
         a.per_plane = shape.per_plane;
         const int threads = shape.threads;
         const int64_t blocks = shape.blocks;
