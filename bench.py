@@ -44,23 +44,25 @@ def class_bytes_per_cell(cls: str, s: int):
         "rb_finest": 5.5 * s,
         # first half-sweep from x = 0: read b, D; write b (projected), x
         "rb_first": 4 * s,
-        # two sweeps in one pass: read x, b, D, 3 face arrays, write x (from
-        # zero no x is read and the projected b written)
+        # two sweeps in one pass, also the one that sums the level-0 mean:
+        # read x, b, D, 3 face arrays, write x (from zero no x is read and the
+        # projected b written)
         "sweep_finest": 7 * s,
-        # the cycle's last fused sweep, which also sums the level-0 mean:
-        # the sweep's arrays and the fluid flags
+        # a cycle's last sweep where sweeps run one by one, which also sums
+        # the level-0 mean: the sweep's arrays and the fluid flags
         "sweep_mean": 7 * s + 1,
         # retained defect r = b - A x: x, b, D, 3 faces, r
         "defect": 7 * s,
         # Krylov q = A p + dot: p, D, 3 faces, q (FP64)
         "operator": 6 * 8,
-        # x += a p, r -= a q: read x p r q, write x r
-        "update_xr": 6 * 8,
+        # r -= a q and the entry made from it: read r, q and the fluid flags,
+        # write r and b (s)
+        "update_xr": 3 * 8 + s + 1,
         # r = b - A x: x, b, D, 3 faces, r
         "true_residual": 7 * 8,
-        # p = z + beta p, z formed from the level-0 candidate: read x (s),
-        # the fluid flags and p, write p
-        "update_p": s + 1 + 2 * 8,
+        # sol += a p and p = z + beta p, z formed from the level-0 candidate:
+        # read x (s), the fluid flags, sol and p, write sol and p
+        "update_p": s + 1 + 4 * 8,
     }.get(cls)
 
 

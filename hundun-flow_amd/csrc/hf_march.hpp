@@ -34,10 +34,13 @@ namespace hf {
 // The loads of a step are issued a step ahead (coefficients of plane k + 1,
 // x of plane k + 2), and a barrier does not wait for them.
 //
-// What bounds it: instruction issue and the chain of the four passes, about
-// 1.4 us a step from L2 and 2 us with HBM behind it (one block of 16
-// wavefronts per CU; the coefficients of four planes take the registers of
-// more, and without b in LDS they spill: 384 us in place of 298 below).  Two
+// What bounds it: the chain of the four passes and the barrier at one block
+// per CU, about 1.4 us a step from L2 and 2 us with HBM behind it (the
+// coefficients of four planes take the registers of more wavefronts than
+// sixteen, and without b in LDS they spill: 384 us in place of 298 below).
+// Counters at 512x256x256 FP32: wavefronts issue for 21% of their time, wait
+// for memory, LDS or the barrier for 45 and for a turn to issue for the rest;
+// the vector units work for 44% of the time (256x256x128 FP64: 34%).  Two
 // sweeps, one launch against two k_rb_sweep launches, from x and from zero:
 // 512x256x256 FP32 298 and 267 us against 478 and 445, 256x256x128 FP64 163
 // and 149 against 277 and 254, 192x192x128 BF16 44 and 41 against 83 and 77.
@@ -74,8 +77,8 @@ struct MarchArgs {
   int gx, gy;          // tiles along x and y
   // kMean: per-block partial sums of w_x w_y w_z x of the output (the
   // constant projection's mean), cell widths per axis.  Solid cells add 0:
-  // the prolongation before this smoothing left x = 0 there, b is 0, their
-  // faces are masked.
+  // the prolongation before this smoothing left x = 0 there, b is 0, and a
+  // refresh refuses a solid row with an open face (row_invalid).
   double* partials;
   const double* wx;
   const double* wy;

@@ -40,8 +40,9 @@ struct alignas(8) TailOp {
 // then colour 1, so that a colour pass keeps whole wavefronts busy; x, b and
 // r in LDS stay in natural order.
 //
-// Blob: a TailGeo per level, then per level, coarsest first, its coefficients by slot (kTailCoefs arrays of `cells` doubles) and its tables
-// by slot (kTailTables arrays of `cells` 16-bit values).
+// Blob: a TailGeo per level, then per level, coarsest first, its coefficients
+// by slot (kTailCoefs arrays of `cells` doubles) and its tables by slot
+// (kTailTables arrays of `cells` 16-bit values).
 enum TailCoef : int {
   kTailD = 0,
   kTailXl,
@@ -78,10 +79,10 @@ struct TailGeo {
   double volume;     // sum of fluid volumes
 };
 constexpr int kTailGeoDoubles = sizeof(TailGeo) / sizeof(double);
-static_assert(kTailGeoDoubles == 6, "kTailOverhead and tail_geo");
+static_assert(kTailGeoDoubles == 6, "kTailOverhead below and tail_geo()");
 
 constexpr int kTailThreads = 1024;
-constexpr int kTailMaxCells = 3072;  // three cells per thread
+constexpr int kTailMaxCells = 3072;  // three cells per thread, at most
 // (a level of at most 3072 cells has at most twelve levels below it, and an
 // F-cycle through those takes fewer ops than this)
 constexpr int kTailMaxLevels = 16;
@@ -92,8 +93,11 @@ constexpr int64_t kTailLdsBytes = 156 * 1024;
 constexpr int kTailSlots = 2;
 constexpr int64_t kTailOverhead =
     kTailSlots + kTailMaxLevels * 6 + kTailMaxOps;
-// what x, b and r of the tail levels may take (the coarsest alone must fit)
+// what x, b and r of the tail levels may take together, 2730 cells (the
+// coarsest alone must fit)
 constexpr int64_t kTailWorkBytes = 64 * 1024;
+static_assert(kTailWorkBytes + 8 * kTailOverhead <= kTailLdsBytes,
+              "the geometry and the ops fit beside the largest work space");
 
 // Doubles of one level's image.
 __host__ __device__ constexpr int64_t tail_image_doubles(int64_t cells) {
@@ -175,7 +179,6 @@ struct TailRun {
   const uint8_t* act0;
   int cells0;
   MeanRef mean;        // pending constant projection of b0 (at: null, none)
-  int levels;
   int work;        // LDS doubles of x, b, r (and slots 0 and 1)
   int head;        // doubles of the blob copied to LDS
   int resident;    // first level whose image is in that head
