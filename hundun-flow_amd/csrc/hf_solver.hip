@@ -2657,13 +2657,23 @@ static hf_status plan_layout(const hf_grid_desc* grid, const hf_policy* policy,
   return ok();
 }
 
+// plan_layout, whose host allocations grow with the grid's extents.
+static hf_status plan_layout_no_throw(const hf_grid_desc* grid,
+                                      const hf_policy* policy, hf_plan* p) {
+  try {
+    return plan_layout(grid, policy, p);
+  } catch (const std::bad_alloc&) {
+    return fail(HF_ALLOCATION_FAILURE, kDetailAlloc);
+  }
+}
+
 hf_status hf_plan_create(const hf_grid_desc* grid, const hf_policy* policy,
                          void* stream, hf_plan** out) {
   if (out == nullptr) return fail(HF_INVALID_PLAN, kDetailPlan);
   *out = nullptr;
   hf_plan* p = new (std::nothrow) hf_plan();
   if (p == nullptr) return fail(HF_ALLOCATION_FAILURE, kDetailAlloc);
-  hf_status s = plan_layout(grid, policy, p);
+  hf_status s = plan_layout_no_throw(grid, policy, p);
   p->stream = static_cast<hipStream_t>(stream);
   if (s.code == HF_OK && hipGetDevice(&p->device) != hipSuccess)
     s = fail(HF_INVALID_PLAN, kDetailHip);
@@ -3739,7 +3749,7 @@ hf_status hf_launch_shape_of(const hf_grid_desc* grid, const hf_policy* policy,
   std::memset(shape, 0, sizeof *shape);
   hf_plan* p = new (std::nothrow) hf_plan();
   if (p == nullptr) return fail(HF_ALLOCATION_FAILURE, kDetailAlloc);
-  hf_status s = plan_layout(grid, policy, p);
+  hf_status s = plan_layout_no_throw(grid, policy, p);
   if (s.code == HF_OK &&
       (level < 0 || level >= static_cast<int32_t>(p->levels.size())))
     s = fail(HF_INVALID_PLAN, kDetailPlan);

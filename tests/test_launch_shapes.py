@@ -1,6 +1,9 @@
 """CPU checks of the launch shapes that a plan's host code works out: the
 routes of its levels and the room for the block sums of their launches."""
 import itertools
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -83,3 +86,34 @@ def test_shape_of_a_refused_grid(n):
     with pytest.raises(H.HundunFlowError) as err:
         H.launch_shape(n, faces, (1,) * 6, H.default_policy())
     assert err.value.code == 2
+
+
+_STARVED = """
+import ctypes, resource, sys
+import numpy as np
+sys.path.insert(0, sys.argv[1])
+import hundun_flow as H
+lib = H.load_library()
+n = (1, 1, 500_000_000)
+faces = [np.linspace(0.0, 1.0, 2)] * 2 + [np.zeros(n[2] + 1)]
+grid = H._grid_desc(n, faces, (1,) * 6)
+policy = H.default_policy()
+size = int(open("/proc/self/statm").read().split()[0]) * 4096
+resource.setrlimit(resource.RLIMIT_AS, (size + (1 << 30),) * 2)
+shape, plan = H.hf_launch_shape(), ctypes.c_void_p()
+for st in (lib.hf_launch_shape_of(ctypes.byref(grid), ctypes.byref(policy), 0,
+                                  ctypes.byref(shape)),
+           lib.hf_plan_create(ctypes.byref(grid), ctypes.byref(policy), None,
+                              ctypes.byref(plan))):
+    assert (st.code, st.detail) == (3, 9102), (st.code, st.detail)
+"""
+
+
+def test_out_of_host_memory_is_a_status():
+    """A grid whose face coordinates no longer fit into host memory is an
+    allocation failure, not an exception through the C interface."""
+    import hundun_flow as H
+    run = subprocess.run([sys.executable, "-c", _STARVED,
+                          os.path.dirname(H.__file__)], timeout=120,
+                         capture_output=True, text=True)
+    assert run.returncode == 0, run.stderr[-2000:]
